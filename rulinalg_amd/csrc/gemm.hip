@@ -4,21 +4,28 @@
 // SYRK update and the mixed-precision updates:
 //   C = alpha * A * op(B) + beta * C, all row-major with row strides.
 //
-// Tiling (FP64/FP32): a 256-thread workgroup owns a 128 x 128 tile of C and
-// walks K in steps of 16 (FP64) or 32 (FP32), double-buffered through LDS.  The four wave64s
-// are arranged 2 x 2; each owns a 64 x 64 sub-tile held as 4 x 4 MFMA
-// accumulators of 16 x 16 (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32).
+// Tiling (FP64/FP32): a 256-thread workgroup owns a 128 x 128, 64 x 64 or
+// 32 x 32 tile of C (tile_edge) and walks K in steps of 16 (FP64) or 32
+// (FP32), double-buffered through LDS.  The four wave64s are arranged 2 x 2;
+// each owns a quarter of the tile as 16 x 16 MFMA accumulators
+// (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32; 4 x 4 of them at 128).
 // A is staged k-major (As[k][i]) so that an MFMA A-fragment (lane l holds
 // A[l%16][l/16]) is four contiguous 128-byte row segments; B is staged
 // As-is (Bs[k][j]).  The +1 padding of transposed stages spreads the
-// transposing LDS writes over all banks.
+// transposing LDS writes over all banks (rows 16 elements apart modulo the
+// banks, which make the fragment reads conflict-free, measured slower: FP64
+// 8192^3 16.3 against 15.1 ms).  The k order is the same for every tile edge
+// and load width, so the results do not depend on them.
 //
 // Low precision (FP16/BF16): operands stay FP32 in memory and are rounded on
 // their way into LDS; v_mfma_f32_16x16x32_{f16,bf16} accumulate in FP32.
 // Fragments hold 8 consecutive k per lane, so both stages are k-contiguous
 // ([i][k] and [j][k]).
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "mfma.hpp"
+#include "wave.hpp"
 
 namespace rlg {
 
@@ -54,208 +61,222 @@ __device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int &tm, i
     tn = r / gm;
 }
 
-// k per LDS stage: 16 in FP64 (2 x 33 KB of stages, two workgroups per CU),
-// 32 in FP32 (the same bytes): twice the matrix-core work between barriers.
+// k per LDS stage: 16 in FP64 (2 x 33 KB of stages at 128 x 128, two
+// workgroups per CU), 32 in FP32 (the same bytes): twice the matrix-core work
+// between barriers.
 template <class T> struct StageK { static constexpr int value = GBK; };
 template <> struct StageK<float> { static constexpr int value = 2 * GBK; };
 
+// Issue order of one stage: NM MFMAs per k-step, with the next k-step's four
+// fragment reads among its last ones; the first k-step's also carry the LDS
+// stores (NW) and, as their registers come free, the global loads (NL).
+template <int NM, int KS, int NW, int NL>
+__device__ __forceinline__ void stage_schedule() {
+    constexpr int MFMA = 0x8, VMEM = 0x20, DSR = 0x100, DSW = 0x200;
+    constexpr int H = NM - 8;  // MFMAs before the next k-step's reads
+    __builtin_amdgcn_sched_group_barrier(DSR, 4, 0);
+    static_for<KS>([&](auto ksc) __attribute__((always_inline)) {
+        constexpr int ks = decltype(ksc)::value;
+        if constexpr (ks == 0) {
+            static_for<H>([&](auto) __attribute__((always_inline)) {
+                __builtin_amdgcn_sched_group_barrier(MFMA, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(DSW, (NW + H - 1) / H, 0);
+                __builtin_amdgcn_sched_group_barrier(VMEM, (NL + H - 1) / H, 0);
+            });
+        } else {
+            __builtin_amdgcn_sched_group_barrier(MFMA, H, 0);
+        }
+        static_for<4>([&](auto) __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_group_barrier(MFMA, 2, 0);
+            if constexpr (ks + 1 < KS) __builtin_amdgcn_sched_group_barrier(DSR, 1, 0);
+        });
+    });
+}
+
+// C = alpha A op(B) + beta C for one BM x BN tile of C per 256-thread
+// workgroup, four waves 2 x 2, each (BM / 2) x (BN / 2) as 16 x 16 MFMA
+// accumulators.
+//
+// Bound by the matrix cores: an FP64 16x16x4 MFMA keeps its SIMD busy for 64
+// cycles (FP32: 32), so everything else has to issue between MFMAs.  The loop
+// therefore runs two stages ahead: stage t writes stage t + 1 (already in
+// registers) to the other LDS buffer and issues the loads of stage t + 2
+// while its own MFMAs run, and no load is behind a branch: row and column
+// indices past the matrix are clamped (they feed only entries of C that are
+// not stored) and only a partial last stage masks k.
+//
 // VEC: operands 16-byte aligned with row strides, K (and N for the
 // untransposed B) multiples of 16 bytes' worth of elements: the tiles are
-// loaded with 16-byte loads (a quarter (FP32) or half (FP64) of the load
-// instructions), which measured 18 % faster on the LU's depth-256 FP32
-// update.  The untransposed B stage is padded by 16 bytes per row.
-// CP: the C tile is read during the last stage (FP32 with VEC only; chosen
-// for shallow products, where the epilogue is a large share of a tile's time).
-template <class T, bool TRANSB, bool LOWER, bool VEC, bool CP>
+// loaded with 16-byte loads.  The untransposed B stage is padded by 16 bytes
+// per row.
+template <class T, int BM, int BN, bool TRANSB, bool LOWER, bool VEC>
 __global__ __launch_bounds__(GTHREADS, 2) void k_gemm(
     int M, int N, int K, T alpha, const T *__restrict__ A, long lda,
     const T *__restrict__ B, long ldb, T beta, T *__restrict__ C, long ldc,
     int tiles_m, int tiles_n) {
     using Acc = typename Mfma<T>::acc;
     constexpr int BK = StageK<T>::value;
-    constexpr int PER = BK * GBM / GTHREADS;  // staged elements per thread per operand
-    constexpr int VL = 16 / sizeof(T);        // elements per 16-byte load
-    constexpr int VPER = PER / VL;            // 16-byte loads per thread per operand
-    static_assert(GBM == GBN && PER * GTHREADS == BK * GBM && VPER * VL == PER, "whole stages");
+    constexpr int VL = VEC ? 16 / (int)sizeof(T) : 1;  // elements per load
+    constexpr int QA = BK * BM / GTHREADS / VL;        // loads per thread, A
+    constexpr int QB = BK * BN / GTHREADS / VL;        // and B
+    constexpr int MI = BM / 32, NJ = BN / 32;          // 16 x 16 tiles per wave
+    static_assert(QA * VL * GTHREADS == BK * BM && QB * VL * GTHREADS == BK * BN, "whole stages");
     typedef T vT __attribute__((ext_vector_type(VL)));
-    __shared__ T As[2][BK][GBM + 1];
-    __shared__ __attribute__((aligned(16))) T Bs[2][BK][GBN + (TRANSB ? 1 : VL)];
+    constexpr int BPAD = TRANSB ? 1 : 16 / (int)sizeof(T);
+    __shared__ T As[2][BK][BM + 1];
+    __shared__ __attribute__((aligned(16))) T Bs[2][BK][BN + BPAD];
 
     int tm, tn;
     tile_coords<LOWER>(tiles_m, tiles_n, tm, tn);
-    if (LOWER && tn > tm) return;  // strictly above the diagonal
-    const int m0 = tm * GBM, n0 = tn * GBN;
+    const int m0 = tm * BM, n0 = tn * BN;
+    if (LOWER && n0 >= m0 + BM) return;  // strictly above the diagonal
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
     const int lr = lane & 15, lk = lane >> 4;
 
-    Acc acc[4][4];
+    Acc acc[MI][NJ];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = Acc{0, 0, 0, 0};
+        for (int j = 0; j < NJ; ++j) acc[i][j] = Acc{0, 0, 0, 0};
 
-    T ra[VEC ? 1 : PER], rb[VEC ? 1 : PER];
-    vT rav[VEC ? VPER : 1], rbv[VEC ? VPER : 1];
-    auto load = [&](int k0) {
-        if constexpr (VEC) {
+    // this thread's loads: A rows (k-vectors), B rows along n (k-vectors of
+    // B^T when transposed)
+    constexpr int AV = BK / VL, BV = TRANSB ? BK / VL : BN / VL;  // vectors per staged row
+    const T *pa[QA], *pb[QB];
 #pragma unroll
-            for (int q = 0; q < VPER; ++q) {
-                const int e = q * GTHREADS + tid;
-                {   // A tile, 128 x BK in BK / VL vectors per row
-                    const int i = e / (BK / VL), gk = k0 + (e % (BK / VL)) * VL, gi = m0 + i;
-                    rav[q] = (gi < M && gk < K) ? *reinterpret_cast<const vT *>(A + (long)gi * lda + gk)
-                                                : vT{};
-                }
-                if (!TRANSB) {  // B tile, BK x 128 in 128 / VL vectors per row
-                    const int gk = k0 + e / (GBN / VL), gj = n0 + (e % (GBN / VL)) * VL;
-                    rbv[q] = (gk < K && gj < N) ? *reinterpret_cast<const vT *>(B + (long)gk * ldb + gj)
-                                                : vT{};
-                } else {        // B^T given as N x K, vectors along k
-                    const int gj = n0 + e / (BK / VL), gk = k0 + (e % (BK / VL)) * VL;
-                    rbv[q] = (gj < N && gk < K) ? *reinterpret_cast<const vT *>(B + (long)gj * ldb + gk)
-                                                : vT{};
-                }
-            }
-        } else {
+    for (int q = 0; q < QA; ++q) {
+        const int e = q * GTHREADS + tid;
+        pa[q] = A + (long)min(m0 + e / AV, M - 1) * lda + (e % AV) * VL;
+    }
 #pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                const int e = q * GTHREADS + tid;
-                {   // A tile, 128 x BK: e -> (i = e / BK, kk = e % BK)
-                    const int i = e / BK, kk = e % BK;
-                    const int gi = m0 + i, gk = k0 + kk;
-                    ra[q] = (gi < M && gk < K) ? A[(long)gi * lda + gk] : T(0);
-                }
-                if (!TRANSB) {  // B tile, BK x 128: e -> (kk = e / 128, j = e % 128)
-                    const int kk = e / GBN, j = e % GBN;
-                    const int gk = k0 + kk, gj = n0 + j;
-                    rb[q] = (gk < K && gj < N) ? B[(long)gk * ldb + gj] : T(0);
-                } else {        // B^T given as N x K: e -> (j = e / BK, kk = e % BK)
-                    const int j = e / BK, kk = e % BK;
-                    const int gj = n0 + j, gk = k0 + kk;
-                    rb[q] = (gj < N && gk < K) ? B[(long)gj * ldb + gk] : T(0);
-                }
+    for (int q = 0; q < QB; ++q) {
+        const int e = q * GTHREADS + tid;
+        pb[q] = TRANSB ? B + (long)min(n0 + e / BV, N - 1) * ldb + (e % BV) * VL
+                       : B + (long)(e / BV) * ldb + min(n0 + (e % BV) * VL, N - VL);
+    }
+    const long bstep = TRANSB ? (long)BK : (long)BK * ldb;
+    vT ra[QA], rb[QB];
+    auto load_full = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < QA; ++q) { ra[q] = *reinterpret_cast<const vT *>(pa[q]); pa[q] += BK; }
+#pragma unroll
+        for (int q = 0; q < QB; ++q) { rb[q] = *reinterpret_cast<const vT *>(pb[q]); pb[q] += bstep; }
+    };
+    auto load = [&](int k0) __attribute__((always_inline)) {
+        if (k0 + BK <= K) { load_full(); return; }
+        // the partial last stage: zeros from k = K on
+#pragma unroll
+        for (int q = 0; q < QA; ++q)
+            ra[q] = k0 + ((q * GTHREADS + tid) % AV) * VL < K ? *reinterpret_cast<const vT *>(pa[q]) : vT(T(0));
+#pragma unroll
+        for (int q = 0; q < QB; ++q) {
+            const int e = q * GTHREADS + tid;
+            const int gk = k0 + (TRANSB ? (e % BV) * VL : e / BV);
+            rb[q] = gk < K ? *reinterpret_cast<const vT *>(pb[q]) : vT(T(0));
+        }
+    };
+    auto store = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < QA; ++q) {
+            const int e = q * GTHREADS + tid, i = e / AV, kb = (e % AV) * VL;
+#pragma unroll
+            for (int v = 0; v < VL; ++v) As[buf][kb + v][i] = ra[q][v];
+        }
+#pragma unroll
+        for (int q = 0; q < QB; ++q) {
+            const int e = q * GTHREADS + tid;
+            if (!TRANSB) {
+                *reinterpret_cast<vT *>(&Bs[buf][e / BV][(e % BV) * VL]) = rb[q];
+            } else {
+#pragma unroll
+                for (int v = 0; v < VL; ++v) Bs[buf][(e % BV) * VL + v][e / BV] = rb[q][v];
             }
         }
     };
-    auto store = [&](int buf) {
-        if constexpr (VEC) {
+    auto mfmas = [&](int buf, int ks) __attribute__((always_inline)) {
+        T af[MI], bf[NJ];
 #pragma unroll
-            for (int q = 0; q < VPER; ++q) {
-                const int e = q * GTHREADS + tid;
-                const int i = e / (BK / VL), kb = (e % (BK / VL)) * VL;
+        for (int i = 0; i < MI; ++i) af[i] = As[buf][ks * 4 + lk][wm + i * 16 + lr];
 #pragma unroll
-                for (int v = 0; v < VL; ++v) As[buf][kb + v][i] = rav[q][v];
-                if (!TRANSB) {
-                    *reinterpret_cast<vT *>(&Bs[buf][e / (GBN / VL)][(e % (GBN / VL)) * VL]) = rbv[q];
-                } else {
+        for (int j = 0; j < NJ; ++j) bf[j] = Bs[buf][ks * 4 + lk][wn + j * 16 + lr];
 #pragma unroll
-                    for (int v = 0; v < VL; ++v) Bs[buf][kb + v][i] = rbv[q][v];
-                }
-            }
-        } else {
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int q = 0; q < PER; ++q) {
-                const int e = q * GTHREADS + tid;
-                As[buf][e % BK][e / BK] = ra[q];
-                if (!TRANSB)
-                    Bs[buf][e / GBN][e % GBN] = rb[q];
-                else
-                    Bs[buf][e % BK][e / BK] = rb[q];
-            }
-        }
-    };
-
-    // FP32 with 16-byte tile loads: the first two row groups of the C tile
-    // are read during the last stage's MFMAs (32 more registers, within the
-    // two-workgroups-per-CU budget; all four, or the scalar-load form, would
-    // spill), the other two before the first store.  Measured: depth-256
-    // updates 83 -> 89 TF/s; at depth 8192 it costs 6 %, hence CP.
-    constexpr bool CPRE = sizeof(T) == 4 && VEC && CP;
-    constexpr int CG = CPRE ? 2 : 1;
-    T cpre[CG][4][4];
-    auto load_c = [&]() {
-#pragma unroll
-        for (int i = 0; i < CG; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int gi = m0 + wm + i * 16 + Mfma<T>::row(lk, r);
-                    const int gj = n0 + wn + j * 16 + lr;
-                    cpre[i][j][r] = (beta != T(0) && gi < M && gj < N) ? C[(long)gi * ldc + gj] : T(0);
-                }
+            for (int j = 0; j < NJ; ++j) acc[i][j] = Mfma<T>::op(af[i], bf[j], acc[i][j]);
     };
 
     const int KT = (K + BK - 1) / BK;
-    load(0);
-    store(0);
-    __syncthreads();
-    for (int kt = 0; kt < KT; ++kt) {
-        const int buf = kt & 1;
-        if (kt + 1 < KT) load((kt + 1) * BK);
-        else if constexpr (CPRE) load_c();
-#pragma unroll
-        for (int ks = 0; ks < BK / 4; ++ks) {
-            T af[4], bf[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) af[i] = As[buf][ks * 4 + lk][wm + i * 16 + lr];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) bf[j] = Bs[buf][ks * 4 + lk][wn + j * 16 + lr];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<T>::op(af[i], bf[j], acc[i][j]);
-        }
-        if (kt + 1 < KT) store(buf ^ 1);
+    if (KT > 0) {
+        load(0);
+        store(0);
+        if (KT > 1) load(BK);
         __syncthreads();
     }
-    if constexpr (CPRE) {
-        if (KT == 0) load_c();  // K = 0: no stage read it
+    int kt = 0;
+    // one basic block per stage while stage kt + 2 is whole
+    for (const int kf = K / BK - 2; kt < kf; ++kt) {
+        const int buf = kt & 1;
+        mfmas(buf, 0);
+        store(buf ^ 1);
+        load_full();
+#pragma unroll
+        for (int ks = 1; ks < BK / 4; ++ks) mfmas(buf, ks);
+        if constexpr (BM == 128) stage_schedule<MI * NJ, BK / 4, QA * VL / 2 + QB, QA + QB>();
+        __syncthreads();
+    }
+    for (; kt < KT; ++kt) {
+        const int buf = kt & 1;
+        if (kt + 1 < KT) store(buf ^ 1);
+        if (kt + 2 < KT) load((kt + 2) * BK);
+#pragma unroll
+        for (int ks = 0; ks < BK / 4; ++ks) mfmas(buf, ks);
+        __syncthreads();
     }
 
-    // epilogue in four row groups: the 16 loads of C of a group are issued
-    // before its stores (a load behind a store to C would wait for it); in
-    // FP32 groups 0-1 are in cpre and groups 2-3 are loaded before any store
-    T clate[CPRE ? 2 : 1][4][4];
-    if constexpr (CPRE) {
+    // epilogue, one row group of 16 at a time: the group's loads of C are
+    // issued before its stores (a load behind a store to C would wait for it)
+    const int row0 = m0 + wm, col0 = n0 + wn + lr;
+    auto epilogue = [&](auto full_c) __attribute__((always_inline)) {
+        constexpr bool FULL = decltype(full_c)::value;  // no row or column past C
+        if (beta == T(0)) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int gi = row0 + i * 16 + Mfma<T>::row(lk, r), gj = col0 + j * 16;
+                        if (FULL || (gi < M && gj < N)) C[(long)gi * ldc + gj] = alpha * acc[i][j][r];
+                    }
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            T cin[NJ][4];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int gi = m0 + wm + (i + 2) * 16 + Mfma<T>::row(lk, r);
-                    const int gj = n0 + wn + j * 16 + lr;
-                    clate[i][j][r] = (beta != T(0) && gi < M && gj < N) ? C[(long)gi * ldc + gj] : T(0);
+                    const int gi = row0 + i * 16 + Mfma<T>::row(lk, r), gj = col0 + j * 16;
+                    cin[j][r] = (FULL || (gi < M && gj < N)) ? C[(long)gi * ldc + gj] : T(0);
                 }
-    }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        T cin[4][4];
+            for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int gi = m0 + wm + i * 16 + Mfma<T>::row(lk, r);
-                const int gj = n0 + wn + j * 16 + lr;
-                if constexpr (CPRE) cin[j][r] = i < 2 ? cpre[i < 2 ? i : 0][j][r] : clate[i >= 2 ? i - 2 : 0][j][r];
-                else cin[j][r] = (beta != T(0) && gi < M && gj < N) ? C[(long)gi * ldc + gj] : T(0);
-            }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int gi = m0 + wm + i * 16 + Mfma<T>::row(lk, r);
-                const int gj = n0 + wn + j * 16 + lr;
-                if (gi < M && gj < N) {
-                    T v = alpha * acc[i][j][r];
-                    if (beta != T(0)) v += beta * cin[j][r];
-                    C[(long)gi * ldc + gj] = v;
+                for (int r = 0; r < 4; ++r) {
+                    const int gi = row0 + i * 16 + Mfma<T>::row(lk, r), gj = col0 + j * 16;
+                    if (FULL || (gi < M && gj < N)) {
+                        T v = alpha * acc[i][j][r];
+                        v += beta * cin[j][r];
+                        C[(long)gi * ldc + gj] = v;
+                    }
                 }
-            }
-    }
+        }
+    };
+    if (m0 + BM <= M && n0 + BN <= N) epilogue(std::true_type{});
+    else epilogue(std::false_type{});
 }
 
 // Depth K <= 64 (the LU and Cholesky updates inside an outer block, which
@@ -263,50 +284,55 @@ __global__ __launch_bounds__(GTHREADS, 2) void k_gemm(
 // every load of A, B and C is issued before the first wait and a workgroup
 // pays one memory latency, where k_gemm pays one per stage plus the
 // epilogue's.  Same fragments, k order and epilogue as k_gemm, so the
-// results are identical.  Needs 16-byte vectors (the VEC conditions).
+// results are identical.  VEC as in k_gemm.
 constexpr int SHK = 64;
-template <class T, bool TRANSB>
+template <class T, int BM, int BN, bool TRANSB, bool VEC>
 __global__ __launch_bounds__(GTHREADS) void k_gemm_shallow(int M, int N, int K, T alpha,
                                                            const T *__restrict__ A, long lda,
                                                            const T *__restrict__ B, long ldb, T beta,
                                                            T *__restrict__ C, long ldc, int tiles_m,
                                                            int tiles_n) {
     using Acc = typename Mfma<T>::acc;
-    constexpr int VL = 16 / sizeof(T);
-    constexpr int VPER = SHK * GBM / GTHREADS / VL;  // 16-byte loads per thread per operand
+    constexpr int VL = VEC ? 16 / (int)sizeof(T) : 1;
+    constexpr int QA = SHK * BM / GTHREADS / VL, QB = SHK * BN / GTHREADS / VL;
+    constexpr int MI = BM / 32, NJ = BN / 32;
     typedef T vT __attribute__((ext_vector_type(VL)));
-    __shared__ T As[SHK][GBM + 1];
-    __shared__ __attribute__((aligned(16))) T Bs[SHK][GBN + (TRANSB ? 1 : VL)];
+    __shared__ T As[SHK][BM + 1];
+    __shared__ __attribute__((aligned(16))) T Bs[SHK][BN + (TRANSB ? 1 : 16 / (int)sizeof(T))];
 
     int tm, tn;
     tile_coords<false>(tiles_m, tiles_n, tm, tn);
-    const int m0 = tm * GBM, n0 = tn * GBN;
+    const int m0 = tm * BM, n0 = tn * BN;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
     const int lr = lane & 15, lk = lane >> 4;
+    constexpr int AV = SHK / VL, BV = TRANSB ? SHK / VL : BN / VL;
 
-    vT rav[VPER], rbv[VPER];
+    // indices past M and N are clamped (they feed only entries that are not
+    // stored); k past K reads as zero
+    vT ra[QA], rb[QB];
 #pragma unroll
-    for (int q = 0; q < VPER; ++q) {
+    for (int q = 0; q < QA; ++q) {
+        const int e = q * GTHREADS + tid, gk = (e % AV) * VL;
+        ra[q] = gk < K ? *reinterpret_cast<const vT *>(A + (long)min(m0 + e / AV, M - 1) * lda + gk) : vT(T(0));
+    }
+#pragma unroll
+    for (int q = 0; q < QB; ++q) {
         const int e = q * GTHREADS + tid;
-        {   // A tile, 128 x SHK in SHK / VL vectors per row
-            const int i = e / (SHK / VL), gk = (e % (SHK / VL)) * VL, gi = m0 + i;
-            rav[q] = (gi < M && gk < K) ? *reinterpret_cast<const vT *>(A + (long)gi * lda + gk) : vT{};
-        }
-        if (!TRANSB) {  // B tile, SHK x 128 in 128 / VL vectors per row
-            const int gk = e / (GBN / VL), gj = n0 + (e % (GBN / VL)) * VL;
-            rbv[q] = (gk < K && gj < N) ? *reinterpret_cast<const vT *>(B + (long)gk * ldb + gj) : vT{};
-        } else {        // B^T given as N x K, vectors along k
-            const int gj = n0 + e / (SHK / VL), gk = (e % (SHK / VL)) * VL;
-            rbv[q] = (gj < N && gk < K) ? *reinterpret_cast<const vT *>(B + (long)gj * ldb + gk) : vT{};
+        if (!TRANSB) {
+            const int gk = e / BV, gj = min(n0 + (e % BV) * VL, N - VL);
+            rb[q] = gk < K ? *reinterpret_cast<const vT *>(B + (long)gk * ldb + gj) : vT(T(0));
+        } else {
+            const int gj = min(n0 + e / BV, N - 1), gk = (e % BV) * VL;
+            rb[q] = gk < K ? *reinterpret_cast<const vT *>(B + (long)gj * ldb + gk) : vT(T(0));
         }
     }
-    T cin[4][4][4];
+    T cin[MI][NJ][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int gi = m0 + wm + i * 16 + Mfma<T>::row(lk, r);
@@ -314,44 +340,47 @@ __global__ __launch_bounds__(GTHREADS) void k_gemm_shallow(int M, int N, int K, 
                 cin[i][j][r] = (beta != T(0) && gi < M && gj < N) ? C[(long)gi * ldc + gj] : T(0);
             }
 #pragma unroll
-    for (int q = 0; q < VPER; ++q) {
-        const int e = q * GTHREADS + tid;
-        const int i = e / (SHK / VL), kb = (e % (SHK / VL)) * VL;
+    for (int q = 0; q < QA; ++q) {
+        const int e = q * GTHREADS + tid, i = e / AV, kb = (e % AV) * VL;
 #pragma unroll
-        for (int v = 0; v < VL; ++v) As[kb + v][i] = rav[q][v];
+        for (int v = 0; v < VL; ++v) As[kb + v][i] = ra[q][v];
+    }
+#pragma unroll
+    for (int q = 0; q < QB; ++q) {
+        const int e = q * GTHREADS + tid;
         if (!TRANSB) {
-            *reinterpret_cast<vT *>(&Bs[e / (GBN / VL)][(e % (GBN / VL)) * VL]) = rbv[q];
+            *reinterpret_cast<vT *>(&Bs[e / BV][(e % BV) * VL]) = rb[q];
         } else {
 #pragma unroll
-            for (int v = 0; v < VL; ++v) Bs[kb + v][i] = rbv[q][v];
+            for (int v = 0; v < VL; ++v) Bs[(e % BV) * VL + v][e / BV] = rb[q][v];
         }
     }
     __syncthreads();
 
-    Acc acc[4][4];
+    Acc acc[MI][NJ];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = Acc{0, 0, 0, 0};
+        for (int j = 0; j < NJ; ++j) acc[i][j] = Acc{0, 0, 0, 0};
     // as many k-steps as k_gemm's whole stages take (rows from K on are
     // zero), so that even the signs of zero results agree with it
     constexpr int BK = StageK<T>::value;
     const int ksteps = (K + BK - 1) / BK * (BK / 4);
     for (int ks = 0; ks < ksteps; ++ks) {
-        T af[4], bf[4];
+        T af[MI], bf[NJ];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) af[i] = As[ks * 4 + lk][wm + i * 16 + lr];
+        for (int i = 0; i < MI; ++i) af[i] = As[ks * 4 + lk][wm + i * 16 + lr];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bf[j] = Bs[ks * 4 + lk][wn + j * 16 + lr];
+        for (int j = 0; j < NJ; ++j) bf[j] = Bs[ks * 4 + lk][wn + j * 16 + lr];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<T>::op(af[i], bf[j], acc[i][j]);
+            for (int j = 0; j < NJ; ++j) acc[i][j] = Mfma<T>::op(af[i], bf[j], acc[i][j]);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int gi = m0 + wm + i * 16 + Mfma<T>::row(lk, r);
@@ -941,14 +970,56 @@ static int check_dims(size_t m, size_t n, size_t k) {
     return RLG_OK;
 }
 
+// Tile edge of a product: 128, 64 or 32.  The time of a launch is what the
+// fullest CU takes for its r tiles, per unit of k (nanoseconds, fitted to
+// launches of one round up to 64 on 256 CUs):
+//   a full chip runs 128-wide tiles best (FP64 8192^3: 14.9 ms against 16.8 at
+//   64 and 19.7 at 32), but a product with few tiles leaves CUs idle or one
+//   wave per SIMD (FP64 1000 x 777 x 1283: 106 us at 128, 62 at 64, 54 at 32;
+//   256^3: 34, 13 and 5.9; 1024^3: 124, 45.5 and 47.4).
+// Scalar loads (odd strides) cost the wide tile most.
+static int tile_edge(size_t m, size_t n, size_t cus, bool f32, bool vec, bool lower) {
+    struct Cost { double per, once; };
+    static const Cost table[2][2][3] = {
+        {{{128, 0}, {35, 12}, {11.4, 2}}, {{118, 0}, {32.5, 12}, {10.7, 2}}},   // FP64: scalar, vector loads
+        {{{74, 0}, {21.5, 8}, {7.1, 3}}, {{63, 0}, {17, 8}, {5.4, 3}}}};        // FP32
+    int best = 128;
+    double least = 0;
+    for (int i = 0; i < 3; ++i) {
+        const int e = 128 >> i;
+        size_t tiles = (size_t)ceil_div(m, e) * ceil_div(n, e);
+        if (lower) tiles = (tiles + ceil_div(m, e)) / 2;
+        const Cost &c = table[f32][vec][i];
+        const double t = c.per * (double)((tiles + cus - 1) / cus) + c.once;
+        if (i == 0 || t < least) { best = e; least = t; }
+    }
+    return best;
+}
+
+template <class T, int E, bool TB, bool LO, bool V>
+static void gemm_launch(hipStream_t s, size_t m, size_t n, size_t k, T alpha, const T *a, size_t lda,
+                        const T *b, size_t ldb, T beta, T *c, size_t ldc, size_t lds_pad, bool shallow) {
+    const int tiles_m = (int)ceil_div(m, E), tiles_n = (int)ceil_div(n, E);
+    const dim3 grid(tiles_m * tiles_n), block(GTHREADS);
+    if constexpr (!LO && E <= 64) {
+        if (shallow) {
+            hipLaunchKernelGGL((k_gemm_shallow<T, E, E, TB, V>), grid, block, 0, s, (int)m, (int)n, (int)k,
+                               alpha, a, (long)lda, b, (long)ldb, beta, c, (long)ldc, tiles_m, tiles_n);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_gemm<T, E, E, TB, LO, V>), grid, block, (unsigned)lds_pad, s, (int)m, (int)n, (int)k,
+                       alpha, a, (long)lda, b, (long)ldb, beta, c, (long)ldc, tiles_m, tiles_n);
+}
+
 template <class T>
 static int gemm_impl(hipStream_t s, const char *cls, size_t m, size_t n, size_t k, T alpha,
                      const T *a, size_t lda, const T *b, size_t ldb, T beta, T *c,
                      size_t ldc, bool trans_b, bool lower_only, size_t lds_pad = 0) {
     if (m == 0 || n == 0) return RLG_OK;
     RLG_TRY(check_dims(m, n, k));
-    const int tiles_m = (int)ceil_div(m, GBM), tiles_n = (int)ceil_div(n, GBN);
-    dim3 grid(tiles_m * tiles_n), block(GTHREADS);
+    Device *d = nullptr;
+    RLG_TRY(current_device(&d));
     const double flops = (lower_only ? 1.0 : 2.0) * (double)m * (double)n * (double)k;
     static const int cls_id = prof_class(cls);
     ProfScope prof_scope(cls_id, s, flops);
@@ -957,33 +1028,23 @@ static int gemm_impl(hipStream_t s, const char *cls, size_t m, size_t n, size_t 
     auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool vec = k % VL == 0 && lda % VL == 0 && ldb % VL == 0 && al16(a) && al16(b) &&
                      (trans_b || n % VL == 0);
-    const bool cp = vec && sizeof(T) == 4 && k <= 1024;
-    if (vec && !lower_only && k > 0 && k <= (size_t)SHK && lds_pad == 0) {
-        if (trans_b)
-            hipLaunchKernelGGL((k_gemm_shallow<T, true>), grid, block, 0, s, (int)m, (int)n, (int)k, alpha,
-                               a, (long)lda, b, (long)ldb, beta, c, (long)ldc, tiles_m, tiles_n);
-        else
-            hipLaunchKernelGGL((k_gemm_shallow<T, false>), grid, block, 0, s, (int)m, (int)n, (int)k, alpha,
-                               a, (long)lda, b, (long)ldb, beta, c, (long)ldc, tiles_m, tiles_n);
-        RLG_LAUNCHED();
-        return RLG_OK;
-    }
-#define RLG_GEMM_LAUNCH(TB, LO, V, CPF)                                                                \
-    hipLaunchKernelGGL((k_gemm<T, TB, LO, V, CPF>), grid, block, (unsigned)lds_pad, s, (int)m, (int)n, \
-                       (int)k, alpha, a, (long)lda, b, (long)ldb, beta, c, (long)ldc, tiles_m, tiles_n)
-#define RLG_GEMM_LAUNCH_V(TB, LO)                                                   \
-    do {                                                                            \
-        if (cp) RLG_GEMM_LAUNCH(TB, LO, true, true);                                \
-        else if (vec) RLG_GEMM_LAUNCH(TB, LO, true, false);                         \
-        else RLG_GEMM_LAUNCH(TB, LO, false, false);                                 \
-    } while (0)
-    if (trans_b) {
-        if (lower_only) RLG_GEMM_LAUNCH_V(true, true); else RLG_GEMM_LAUNCH_V(true, false);
-    } else {
-        if (lower_only) RLG_GEMM_LAUNCH_V(false, true); else RLG_GEMM_LAUNCH_V(false, false);
-    }
-#undef RLG_GEMM_LAUNCH_V
-#undef RLG_GEMM_LAUNCH
+    const bool shallow = !lower_only && k > 0 && k <= (size_t)SHK && lds_pad == 0;
+    int edge = lds_pad ? GBM : tile_edge(m, n, (size_t)d->num_cus, sizeof(T) == 4, vec, lower_only);
+    // a shallow product is bound by its C traffic, and at 128 by one workgroup
+    // per CU (133 KB of LDS): FP64 16000 x 64 x 448 takes 37 us there, 29 at 64
+    if (shallow && edge > 64) edge = 64;
+    auto go = [&](auto e, auto tb, auto lo, auto v) {
+        gemm_launch<T, decltype(e)::value, decltype(tb)::value, decltype(lo)::value, decltype(v)::value>(
+            s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, lds_pad, shallow);
+    };
+    using std::false_type;
+    using std::true_type;
+    auto pick_v = [&](auto e, auto tb, auto lo) { if (vec) go(e, tb, lo, true_type{}); else go(e, tb, lo, false_type{}); };
+    auto pick_lo = [&](auto e, auto tb) { if (lower_only) pick_v(e, tb, true_type{}); else pick_v(e, tb, false_type{}); };
+    auto pick_tb = [&](auto e) { if (trans_b) pick_lo(e, true_type{}); else pick_lo(e, false_type{}); };
+    if (edge == 128) pick_tb(std::integral_constant<int, 128>{});
+    else if (edge == 64) pick_tb(std::integral_constant<int, 64>{});
+    else pick_tb(std::integral_constant<int, 32>{});
     RLG_LAUNCHED();
     return RLG_OK;
 }
