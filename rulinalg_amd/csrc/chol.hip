@@ -5,8 +5,9 @@
 // depth 512 on the lower tiles of the trailing matrix (512 measured faster
 // than 128 or 256 at order 16384, and wider blocks no faster).  Inside an outer
 // block, 64-column blocks are processed left to right:
-//   1. one launch (k_chol_block) factors the diagonal block with the
-//      reference's left-looking "gaxpy" recurrence: a[k][j] -= dot(row k,
+//   1. one launch factors the diagonal block and solves the rows below against
+//      it: k_chol_col (see there) above order 64, and at most that order
+//      k_chol_block with the reference's left-looking "gaxpy" recurrence: a[k][j] -= dot(row k,
 //      row j) over the block's previous columns in utils::dot's eight-lane
 //      order, the |d| < eps and d < 0 checks, and division by sqrt(d);
 //      in the same launch the rows below are solved against it with the
@@ -20,6 +21,7 @@
 #include <utility>
 
 #include "kernels.hpp"
+#include "mfma.hpp"
 #include "wave.hpp"
 
 namespace rlg {
@@ -67,7 +69,7 @@ __device__ __forceinline__ T dot8_reg(const T (&x)[CNB], const T *l) {
 // (the same arithmetic, so the same values).  The block is written back in
 // place, so it may be written only once every workgroup has read it: the
 // workgroups count themselves in `arrive` once their loads are done, and the
-// last to arrive writes the block and the divisors (a workgroup may start
+// last to arrive writes the block (a workgroup may start
 // long after the others when other streams' kernels hold the CUs, and then
 // must still read the unfactored block).  Workgroup 0 writes the failure
 // index, which no workgroup reads.  Wave 1 solves the workgroup's 64
@@ -80,8 +82,7 @@ __device__ __forceinline__ T dot8_reg(const T (&x)[CNB], const T *l) {
 // are read and written whole (coalesced) and transposed through LDS.
 template <class T>
 __global__ __launch_bounds__(128) void k_chol_block(T *__restrict__ A, long lda, int j0, int jb,
-                                                    int r0, int n, T *__restrict__ divisor,
-                                                    int64_t *__restrict__ info,
+                                                    int r0, int n, int64_t *__restrict__ info,
                                                     unsigned *__restrict__ arrive) {
 #pragma clang fp contract(off)
     __shared__ T a[CNB][CNB + 1];
@@ -156,7 +157,6 @@ __global__ __launch_bounds__(128) void k_chol_block(T *__restrict__ A, long lda,
         for (int c = 0; c < CNB; ++c)
             if (c == t && c < jend) a[t][t] = x[c];
         if (last) {  // set before the loop's first barrier (jb >= 1)
-            if (t < jend) divisor[j0 + t] = sdiv[t];
 #pragma unroll 8
             for (int r = 0; r < jb; ++r)
                 if (t <= r) A[(long)(j0 + r) * lda + j0 + t] = a[r][t];
@@ -172,10 +172,175 @@ __global__ __launch_bounds__(128) void k_chol_block(T *__restrict__ A, long lda,
     }
 }
 
-// Workspace: the divisors, then one arrival counter per 64-column block.
-static size_t chol_div_bytes(size_t n, size_t elem) { return ((n + 1) * elem + 255) & ~(size_t)255; }
+// ---------------------------------------------------------------- block columns beyond the first order
+
+// k_chol_block keeps the reference's operation order, which only an order of
+// at most 64 can show bit for bit: 64 columns of two barriers, a 63-term dot
+// product, a square root and a division each, 66 us in FP64 whatever the
+// height.  Larger orders take k_chol_col, which does the same work in 16-column
+// panels: one wave factors a panel with the rows of the diagonal block in its
+// lanes (no barrier per column, the square root and its reciprocal from one
+// Goldschmidt iteration, fused multiply-adds), the matrix cores apply it to
+// the rest of the diagonal block, and the rows below are solved panel by panel
+// beside the next panel's factorization.  Like the reference's dot products,
+// every panel's products are summed before they are subtracted (subtracted one
+// by one, the factor's residual at order 128 was 19 % larger).  It is bound by the serial chain of
+// the 64 columns (about 180 cycles each).  Order 4096: 6.27 -> 2.58 ms for the
+// factorization, order 16384: 49.6 -> 33.2 ms (44 TF).
+
+// s = sqrt(d) and r = 1 / s for d >= epsilon (Goldschmidt's iteration from the
+// hardware's reciprocal square root estimate, then one residual step for s).
+__device__ __forceinline__ void sqrt_recip(double d, double &s, double &r) {
+    const double y = __builtin_amdgcn_rsq(d);
+    double g = d * y, h = 0.5 * y;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const double e = fma(-h, g, 0.5);
+        g = fma(g, e, g);
+        h = fma(h, e, h);
+    }
+    s = fma(fma(-g, g, d), h, g);
+    s = d == __builtin_inf() ? d : s;
+    r = h + h;
+}
+__device__ __forceinline__ void sqrt_recip(float d, float &s, float &r) {
+    s = sqrtf(d);
+    r = 1.0f / s;
+}
+// x / s from r = 1 / s: the quotient and one residual correction (Markstein),
+// left out where the residual is not finite.
+template <class T> __device__ __forceinline__ T div_recip(T x, T s, T r) {
+    const T q = x * r, e = fma(-q, s, x);
+    return fabs(e) < T(__builtin_inf()) ? fma(e, r, q) : q;
+}
+
+constexpr int PW = 16;           // panel width inside a block column
+constexpr int CLD = CNB + 2;     // LDS row of 64 (16-byte aligned)
+
+// One 64-column block column j0 .. j0 + jb of an order above 64: the diagonal
+// block (factored redundantly by every workgroup, written back by the last to
+// have read it, see k_chol_block) and 64 rows below it per workgroup.  S and X
+// hold columns (S[c][r]: entry (r, c)), so a wave's lanes run along rows
+// without bank conflicts.  Between barriers, panel p:
+//   wave 0      factors panel p of the diagonal block in registers;
+//   waves 1, 2  solve panel p - 1 of their 32 rows below and subtract the
+//               solved panels' part from panel p (matrix cores);
+//   wave 3      applies panel p - 1 to the diagonal block right of panel p;
+// then waves 0-2 apply panel p to panel p + 1.
+template <class T>
+__global__ __launch_bounds__(256) void k_chol_col(T *__restrict__ A, long lda, int j0, int jb, int r0,
+                                                  int n, int64_t *__restrict__ info,
+                                                  unsigned *__restrict__ arrive) {
+    using Acc = typename Mfma<T>::acc;
+    __shared__ __attribute__((aligned(16))) T S[CNB][CLD], X[CNB][CLD];
+    __shared__ T sd[CNB], rd[CNB];  // sqrt of the pivots, and 1 / it
+    __shared__ int last;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int rb = r0 + (int)blockIdx.x * 64;
+    const int nr = n - rb >= 64 ? 64 : (n - rb > 0 ? n - rb : 0);
+    {   // all loads in flight before their LDS stores; past jb the identity
+        T v[16], w[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int r = q * 4 + wave;
+            v[q] = (r < jb && lane <= r) ? A[(long)(j0 + r) * lda + j0 + lane] : (r == lane ? T(1) : T(0));
+            w[q] = (r < nr && lane < jb) ? A[(long)(rb + r) * lda + j0 + lane] : T(0);
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            S[lane][q * 4 + wave] = v[q];
+            X[lane][q * 4 + wave] = w[q];
+        }
+    }
+    __syncthreads();
+    // every load of this workgroup has returned (its values are in LDS)
+    if (tid == 0)
+        last = __hip_atomic_fetch_add(arrive, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+               gridDim.x - 1;
+
+    // D[jc][ir] -= sum over the PW columns of panel q of L[jc][k] R[ir][k], a
+    // 16 x 16 tile: L from S, R and D from S (the block itself) or X
+    auto tile = [&](T(*R)[CLD], int q0, int q1, int cj, int ri) __attribute__((always_inline)) {
+        Acc acc = Acc{0, 0, 0, 0};
+        T d[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d[r] = R[cj + Mfma<T>::row(lk, r)][ri + lr];
+        for (int k = q0 * PW; k < q1 * PW; k += 4)
+            acc = Mfma<T>::op(S[k + lk][cj + lr], R[k + lk][ri + lr], acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) R[cj + Mfma<T>::row(lk, r)][ri + lr] = d[r] - acc[r];
+    };
+    // rows [32 h, 32 h + 32) of X, panel q: x L11^T = b, one row per lane
+    auto solve = [&](int h, int q) __attribute__((always_inline)) {
+        const int c0 = q * PW, row = 32 * h + (lane & 31);
+        T y[PW], sum[PW];
+#pragma unroll
+        for (int c = 0; c < PW; ++c) { y[c] = X[c0 + c][row]; sum[c] = T(0); }
+        static_for<PW>([&](auto cc) __attribute__((always_inline)) {
+            constexpr int c = decltype(cc)::value;
+            y[c] = div_recip(y[c] - sum[c], sd[c0 + c], rd[c0 + c]);
+#pragma unroll
+            for (int e = c + 1; e < PW; ++e) sum[e] = fma(y[c], S[c0 + c][c0 + e], sum[e]);
+        });
+#pragma unroll
+        for (int c = 0; c < PW; ++c)
+            if (lane < 32) X[c0 + c][row] = y[c];
+    };
+
+    int fail = jb;  // wave 0: the first pivot below epsilon or negative
+    for (int p = 0; p < CNB / PW; ++p) {
+        if (wave == 0) {
+            T x[PW], sum[PW];
+#pragma unroll
+            for (int c = 0; c < PW; ++c) { x[c] = S[p * PW + c][lane]; sum[c] = T(0); }
+            T sv = T(0), rv = T(0);  // lane c keeps column c's square root
+            static_for<PW>([&](auto cc) __attribute__((always_inline)) {
+                constexpr int c = decltype(cc)::value;
+                x[c] -= sum[c];
+                const T d = lane_get(x[c], p * PW + c);
+                const bool bad = fabs(d) < ceps<T>() || d < T(0);
+                fail = (bad && fail > p * PW + c) ? p * PW + c : fail;
+                T s, r;
+                sqrt_recip(d, s, r);
+                x[c] = div_recip(x[c], s, r);
+                sv = lane == c ? s : sv;
+                rv = lane == c ? r : rv;
+#pragma unroll
+                for (int e = c + 1; e < PW; ++e) sum[e] = fma(x[c], lane_get(x[c], p * PW + e), sum[e]);
+            });
+#pragma unroll
+            for (int c = 0; c < PW; ++c) S[p * PW + c][lane] = x[c];
+            if (lane < PW) { sd[p * PW + lane] = sv; rd[p * PW + lane] = rv; }
+        } else if (p > 0) {
+            if (wave < 3) {
+                solve(wave - 1, p - 1);
+                tile(X, 0, p, p * PW, 32 * (wave - 1));
+                tile(X, 0, p, p * PW, 32 * (wave - 1) + 16);
+            } else {
+                for (int cj = p + 1; cj < CNB / PW; ++cj)
+                    for (int ri = cj; ri < CNB / PW; ++ri) tile(S, p - 1, p, cj * PW, ri * PW);
+            }
+        }
+        __syncthreads();
+        if (p + 1 + wave < CNB / PW) tile(S, p, p + 1, (p + 1) * PW, (p + 1 + wave) * PW);
+        __syncthreads();
+    }
+    if (wave == 1 || wave == 2) solve(wave - 1, CNB / PW - 1);
+    if (wave == 0 && lane == 0 && blockIdx.x == 0 && fail < jb && *info == (int64_t)n) *info = j0 + fail;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const int r = q * 4 + wave;
+        if (last && r < jb && lane <= r) A[(long)(j0 + r) * lda + j0 + lane] = S[lane][r];
+        if (r < nr && lane < jb) A[(long)(rb + r) * lda + j0 + lane] = X[lane][r];
+    }
+}
+
+// Workspace: one arrival counter per 64-column block.
 size_t chol_work_bytes(size_t n, size_t elem) {
-    return chol_div_bytes(n, elem) + ((ceil_div(n, CNB) * sizeof(unsigned) + 255) & ~(size_t)255);
+    (void)elem;
+    return (ceil_div(n, CNB) * sizeof(unsigned) + 255) & ~(size_t)255;
 }
 
 // LDS the look-ahead's update workgroups reserve beyond their own 66 KB
@@ -204,8 +369,7 @@ struct CholEvents {
 template <class T>
 static int chol_impl(hipStream_t s, size_t n, T *a, size_t lda, int64_t *info, void *work,
                      int lowp_prec) {
-    T *divisor = static_cast<T *>(work);
-    unsigned *arrive = reinterpret_cast<unsigned *>(static_cast<char *>(work) + chol_div_bytes(n, sizeof(T)));
+    unsigned *arrive = static_cast<unsigned *>(work);
     RLG_TRY(fill_i64(info, 1, (int64_t)n, s));
     RLG_TRY(fill_u32(arrive, ceil_div(n, CNB), 0u, s));
     const bool native = lowp_prec != RLG_PREC_F16 && lowp_prec != RLG_PREC_BF16;
@@ -229,9 +393,13 @@ static int chol_impl(hipStream_t s, size_t n, T *a, size_t lda, int64_t *info, v
             {
                 RLG_PROF("chol_block", s);
                 const size_t below = n - r0;  // rows under the diagonal block
-                hipLaunchKernelGGL(k_chol_block<T>, dim3(below ? ceil_div(below, 64) : 1), dim3(128), 0,
-                                   s, a, (long)lda, (int)j0, (int)jb, (int)r0, (int)n, divisor, info,
-                                   arrive + j0 / CNB);
+                const dim3 grid(below ? ceil_div(below, 64) : 1);
+                if (n <= (size_t)CNB)  // the reference's bits
+                    hipLaunchKernelGGL(k_chol_block<T>, grid, dim3(128), 0, s, a, (long)lda, (int)j0, (int)jb,
+                                       (int)r0, (int)n, info, arrive + j0 / CNB);
+                else
+                    hipLaunchKernelGGL(k_chol_col<T>, grid, dim3(256), 0, s, a, (long)lda, (int)j0, (int)jb,
+                                       (int)r0, (int)n, info, arrive + j0 / CNB);
                 RLG_LAUNCHED();
             }
             if (r0 < k0 + kb) {
