@@ -174,13 +174,14 @@ int lu_solve_host(const rlg_lu *h, size_t b_len, size_t nrhs, const T *b, size_t
     Device *d;
     RLG_TRY(current_device(&d));
     hipStream_t s = d->stream;
-    PoolBuf db, tmp;
+    PoolBuf db, dx, tmp;
     RLG_TRY(db.alloc(nrhs * n * sizeof(T), s));
+    RLG_TRY(dx.alloc(nrhs * n * sizeof(T), s));
     RLG_TRY(tmp.alloc(nrhs * n * sizeof(T), s));
     RLG_TRY(upload_matrix<T>(s, db.as<T>(), n, b, ldb, nrhs, n));
     RLG_TRY(lu_solve<T>(s, n, static_cast<const T *>(h->a), h->lda, h->raw_d.as<int64_t>(), nrhs,
-                        db.as<T>(), n, db.as<T>(), n, tmp.as<T>()));
-    RLG_TRY(download_matrix<T>(s, x, ldx, db.as<T>(), n, nrhs, n));
+                        db.as<T>(), n, dx.as<T>(), n, tmp.as<T>()));
+    RLG_TRY(download_matrix<T>(s, x, ldx, dx.as<T>(), n, nrhs, n));
     RLG_HIP(hipStreamSynchronize(s));
     return RLG_OK;
 }

@@ -457,18 +457,25 @@ int chol_factor_lowp(hipStream_t s, int prec, size_t n, float *a, size_t lda, in
 }
 
 // Cholesky::solve (cholesky.rs:194-202): forward substitution with L, then
-// transpose_back_substitution with L^T.  b is copied to tmp first, so x may
-// alias b; the first solve writes x, the second reads x and writes tmp.
+// transpose_back_substitution with L^T.  The first solve works from b in x
+// (x may be b itself) into tmp, the second from tmp into x; only a b that
+// overlaps x otherwise goes to tmp first.
 template <class T>
 int chol_solve(hipStream_t s, size_t n, const T *l, size_t lda, size_t nrhs, const T *b, size_t ldb,
                T *x, size_t ldx, T *tmp) {
     if (n == 0 || nrhs == 0) return RLG_OK;
-    RLG_HIP(hipMemcpy2DAsync(tmp, n * sizeof(T), b, ldb * sizeof(T), n * sizeof(T), nrhs,
-                             hipMemcpyDeviceToDevice, s));
-    RLG_TRY(trsv_lower<T>(s, n, l, lda, false, nrhs, tmp, n, x, ldx));
-    RLG_TRY(trsv_lower_t<T>(s, n, l, lda, nrhs, x, ldx, tmp, n));
-    RLG_HIP(hipMemcpy2DAsync(x, ldx * sizeof(T), tmp, n * sizeof(T), n * sizeof(T), nrhs,
-                             hipMemcpyDeviceToDevice, s));
+    const bool same = b == x && (ldb == ldx || nrhs == 1);
+    const bool apart = same || !vectors_overlap(n, nrhs, b, ldb, x, ldx);
+    T *y = apart ? x : tmp, *z = apart ? tmp : x;
+    const size_t ldy = apart ? ldx : n, ldz = apart ? n : ldx;
+    if (!same)
+        RLG_HIP(hipMemcpy2DAsync(y, ldy * sizeof(T), b, ldb * sizeof(T), n * sizeof(T), nrhs,
+                                 hipMemcpyDeviceToDevice, s));
+    RLG_TRY(trsv_lower<T>(s, n, l, lda, false, nrhs, y, ldy, z, ldz));
+    RLG_TRY(trsv_lower_t<T>(s, n, l, lda, nrhs, z, ldz, y, ldy));
+    if (!apart)
+        RLG_HIP(hipMemcpy2DAsync(x, ldx * sizeof(T), tmp, n * sizeof(T), n * sizeof(T), nrhs,
+                                 hipMemcpyDeviceToDevice, s));
     return RLG_OK;
 }
 template int chol_solve<double>(hipStream_t, size_t, const double *, size_t, size_t, const double *,

@@ -117,6 +117,14 @@ int *lu_timeout_flag(void *work, size_t n, size_t elem);
 // reference's final inverse (lu.rs:186-193).
 void perm_from_ipiv(size_t n, const int64_t *ipiv, int64_t *raw);
 
+// Whether the address ranges of two blocks of nrhs vectors of length n meet.
+template <class T>
+inline bool vectors_overlap(size_t n, size_t nrhs, const T *a, size_t lda, const T *b, size_t ldb) {
+    const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), a1 = a0 + ((nrhs - 1) * lda + n) * sizeof(T);
+    const uintptr_t b0 = reinterpret_cast<uintptr_t>(b), b1 = b0 + ((nrhs - 1) * ldb + n) * sizeof(T);
+    return a0 < b1 && b0 < a1;
+}
+
 // X = U^-1 L^-1 P B for nrhs vectors (vector r at b + r*ldb); x may alias b.
 // `tmp` holds n * nrhs elements.
 template <class T>

@@ -1091,17 +1091,22 @@ template <class T>
 int lu_solve(hipStream_t s, size_t n, const T *lu, size_t lda, const int64_t *raw, size_t nrhs,
              const T *b, size_t ldb, T *x, size_t ldx, T *tmp) {
     if (n == 0 || nrhs == 0) return RLG_OK;
+    // y = P b, then L^-1 y, then U^-1 of that, each into the buffer the one
+    // before does not use; with x and b apart the last lands in x by itself
+    const bool apart = !vectors_overlap(n, nrhs, b, ldb, x, ldx);
+    T *y = apart ? x : tmp, *z = apart ? tmp : x;
+    const size_t ldy = apart ? ldx : n, ldz = apart ? n : ldx;
     {
         RLG_PROF("gather", s);
         hipLaunchKernelGGL(k_gather_rows<T>, dim3(ceil_div(n, 256), (unsigned)nrhs), dim3(256), 0, s, n,
-                           nrhs, raw, b, ldb, tmp, n);
+                           nrhs, raw, b, ldb, y, ldy);
         RLG_LAUNCHED();
     }
-    // y = L^-1 (P b) lands in x (b is no longer read), then U^-1 y in tmp
-    RLG_TRY(trsv_lower<T>(s, n, lu, lda, true, nrhs, tmp, n, x, ldx));
-    RLG_TRY(trsv_upper<T>(s, n, lu, lda, nrhs, x, ldx, tmp, n));
-    RLG_HIP(hipMemcpy2DAsync(x, ldx * sizeof(T), tmp, n * sizeof(T), n * sizeof(T), nrhs,
-                             hipMemcpyDeviceToDevice, s));
+    RLG_TRY(trsv_lower<T>(s, n, lu, lda, true, nrhs, y, ldy, z, ldz));
+    RLG_TRY(trsv_upper<T>(s, n, lu, lda, nrhs, z, ldz, y, ldy));
+    if (!apart)
+        RLG_HIP(hipMemcpy2DAsync(x, ldx * sizeof(T), tmp, n * sizeof(T), n * sizeof(T), nrhs,
+                                 hipMemcpyDeviceToDevice, s));
     return RLG_OK;
 }
 template int lu_solve<double>(hipStream_t, size_t, const double *, size_t, const int64_t *, size_t,

@@ -17,14 +17,26 @@
 // and updates only rows outside it, so reads and writes of one launch never
 // touch the same element.  The solution goes to `out`, a different buffer.
 //
-// Within a sub-block the order of operations is the column sweep of the
+// Within a sub-block the entries are found by a column sweep, as in the
 // reference's transpose_back_substitution (src/matrix/decomposition/
-// cholesky.rs:329-361): divide x[c] by the diagonal, then subtract
-// m[i][c] * x[c] (separately rounded) from the remaining rows.
-// forward_substitution, lu_forward_substitution and back_substitution
-// (src/matrix/mod.rs:318-398, lu.rs:624-642) form row dot products instead;
-// the results agree to rounding.
+// cholesky.rs:329-361); forward_substitution, lu_forward_substitution and
+// back_substitution (src/matrix/mod.rs:318-398, lu.rs:624-642) form row dot
+// products instead; the results agree to rounding.
+//
+// A launch is bound by its serial chain, 64 columns per sub-block, on top of
+// one launch and one memory latency.  So a lane divides its row of the triangle
+// and its right-hand side by the row's diagonal up front, which leaves a
+// broadcast and one fused multiply-add per column on the chain, and a wave
+// sweeps up to four right-hand sides together.  Scaled and swept that way, a
+// value that is not finite could reach entries it must not; a sub-block whose
+// result holds one is swept again with a division and a test per column.
+// FP64 at order 4096, per launch of 128 rows: 14.6 -> 9.1 us (upper, one
+// right-hand side), 10.3 -> 8.6 (unit lower); at order 16384 with 16
+// right-hand sides 56 -> 17.9 and 39.5 -> 17.2 us.
+#include <limits>
+
 #include "kernels.hpp"
+#include "mfma.hpp"
 #include "wave.hpp"
 
 namespace rlg {
@@ -37,11 +49,11 @@ constexpr int CPW = 64;     // entries updated per workgroup (transposed form)
 
 enum TriMode { LOWER_UNIT = 0, LOWER = 1, UPPER = 2, LOWER_T = 3 };
 
-// x / d on the solve's serial chain: FP64 divides (the reference divides);
-// FP32 (the refinement's correction solves) multiplies by a reciprocal that
-// every lane computed up front.
-__device__ __forceinline__ double diag_div(double x, double d, double) { return x / d; }
-__device__ __forceinline__ float diag_div(float x, float, float rd) { return x * rd; }
+// a / d from r = 1 / d, with one residual correction (Markstein).
+template <class T> __device__ __forceinline__ T div_recip(T a, T d, T r) {
+    const T q = a * r;
+    return fma(fma(-q, d, a), r, q);
+}
 
 template <int MODE> __device__ __forceinline__ constexpr bool forward() {
     return MODE == LOWER_UNIT || MODE == LOWER;
@@ -50,8 +62,8 @@ template <int MODE> __device__ __forceinline__ constexpr bool stored_upper() { r
 
 // One 64 x 64 tile of M (rows rb.., cols cb.., rs x cs valid), 16 values per
 // thread: tile_load issues the loads, tile_store puts them in LDS.  `diag`
-// keeps only the stored triangle and zeroes the rest, so entries of the
-// other triangle are never read as numbers.  With `vec` (M and lda allow
+// keeps only the strict part of the stored triangle and zeroes the rest, so
+// entries of the other triangle are never read as numbers.  With `vec` (M and lda allow
 // 16-byte loads) a full tile is read with 16-byte loads, a quarter (FP32)
 // or half (FP64) of the load instructions: with the update slice also in
 // flight, scalar loads would exceed what a wave can have outstanding.
@@ -74,7 +86,7 @@ __device__ __forceinline__ void tile_load(T (&v)[TPER], const T *__restrict__ M,
 #pragma unroll
             for (int t = 0; t < VL; ++t) {
                 const int j = j0 + t;
-                const bool ok = !diag || (stored_upper<MODE>() ? j >= i : j <= i);
+                const bool ok = !diag || (stored_upper<MODE>() ? j > i : j < i);
                 v[u * VL + t] = ok ? x[t] : T(0);
             }
         }
@@ -84,7 +96,7 @@ __device__ __forceinline__ void tile_load(T (&v)[TPER], const T *__restrict__ M,
             const int e = q * 256 + threadIdx.x;
             const int i = e >> 6, j = e & 63;
             bool ok = i < rs && j < cs;
-            if (diag) ok = ok && (stored_upper<MODE>() ? j >= i : j <= i);
+            if (diag) ok = ok && (stored_upper<MODE>() ? j > i : j < i);
             v[q] = ok ? M[(long)(rb + i) * lda + cb + j] : T(0);
         }
     }
@@ -129,10 +141,27 @@ __device__ __forceinline__ void tile_row(const T (*t)[SB + TP<T>], int lane, T (
     }
 }
 
-// Right-hand sides whose update-phase rows of W are loaded up front.
-constexpr int RPRE = 2;
+// With more right-hand sides than waves the update is a product of a workgroup's
+// 64 rows of M, the step's 128 columns and up to 16 vectors: matrix cores, one
+// 16 x 16 tile per wave.  With fewer it is a dot product per row and vector.
+constexpr int RDOT = 4;
 
+// One right-hand side of a sub-block, a column at a time: each entry divided by
+// its diagonal and subtracted only from the entries after it.
 template <class T, int MODE>
+__device__ __forceinline__ T sweep_plain(const T (*t)[SB + TP<T>], T x, T dl, int lane) {
+#pragma unroll 1
+    for (int cc = 0; cc < SB; ++cc) {
+        const int c = forward<MODE>() ? cc : SB - 1 - cc;
+        if (MODE != LOWER_UNIT && lane == c) x = x / dl;
+        const T xc = lane_get(x, c), m = MODE == LOWER_T ? t[c][lane] : t[lane][c];
+        if (forward<MODE>() ? lane > c : lane < c) x = x - m * xc;
+    }
+    return x;
+}
+
+// NR: right-hand sides per wave (wave w sweeps w, w + 4, ...).
+template <class T, int MODE, int NR>
 __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long lda, int n, int q0,
                                                    int nq, int nrhs, T *__restrict__ W, long ldw,
                                                    T *__restrict__ X, long ldx, int u0, int u1,
@@ -140,7 +169,7 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
     // tiles: [0] diagonal of sub-block 0, [1] diagonal of sub-block 1,
     // [2] the off-diagonal tile inside the stored triangle
     __shared__ __attribute__((aligned(16))) T tl[3][SB][SB + TP<T>];
-    __shared__ T xs[TMAXR][TSB * SB];
+    __shared__ __attribute__((aligned(16))) T xs[TMAXR][TSB * SB + TP<T>];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int s0 = q0 * SB, s1 = min(n, (q0 + nq) * SB), S = s1 - s0;
     const int bs0 = min(SB, S), bs1 = S - bs0;  // rows of sub-blocks 0 and 1
@@ -152,12 +181,40 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
     // the three tiles; this wave's first right-hand side on the super-block.
     constexpr int NIT = RPW / 16, NC = TSB * SB / 16;  // row forms
     constexpr int CW = TSB * SB / 4;                   // transposed form
+    constexpr bool PRODUCT = NR > 1;
+    constexpr int VL = TVL<T>;
     const int ls = lane & 15, grp = lane >> 4;
     const int rbase = u0 + (int)blockIdx.x * RPW + wave * (RPW / 4) + grp;
     const int jt = u0 + (int)blockIdx.x * CPW + lane;
-    T mv[MODE == LOWER_T ? CW : NIT * NC];
-    T wpre[RPRE][MODE == LOWER_T ? 1 : NIT];
-    if constexpr (MODE == LOWER_T) {
+    // product form: the wave's 16 rows (row ls of them per lane), the lane's
+    // columns 4 VL u + VL grp + e, and the W entries of its accumulator
+    const int jp = u0 + (int)blockIdx.x * RPW + wave * 16;
+    T mv[PRODUCT ? CW : MODE == LOWER_T ? CW : NIT * NC];
+    T wpre[PRODUCT ? 1 : RDOT][PRODUCT ? 4 : MODE == LOWER_T ? 1 : NIT];
+    if constexpr (PRODUCT) {
+        typedef T vT __attribute__((ext_vector_type(VL)));
+        const int j = jp + ls;
+#pragma unroll
+        for (int u = 0; u < CW / VL; ++u) {
+            const int c = (4 * u + grp) * VL;
+            if (MODE != LOWER_T && vec && c + VL <= S) {
+                const vT x = j < u1 ? *reinterpret_cast<const vT *>(M + (long)j * lda + s0 + c) : vT(T(0));
+#pragma unroll
+                for (int e = 0; e < VL; ++e) mv[u * VL + e] = x[e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < VL; ++e)
+                    mv[u * VL + e] = j < u1 && c + e < S
+                                         ? M[MODE == LOWER_T ? (long)(s0 + c + e) * lda + j : (long)j * lda + s0 + c + e]
+                                         : T(0);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int jw = jp + Mfma<T>::row(grp, q);
+            wpre[0][q] = jw < u1 && ls < nrhs ? W[(long)ls * ldw + jw] : T(0);
+        }
+    } else if constexpr (MODE == LOWER_T) {
         const bool act = jt < u1;
 #pragma unroll
         for (int q = 0; q < CW; ++q) {
@@ -165,7 +222,7 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
             mv[q] = (act && c < S) ? M[(long)(s0 + c) * lda + jt] : T(0);
         }
 #pragma unroll
-        for (int r = 0; r < RPRE; ++r)
+        for (int r = 0; r < RDOT; ++r)
             wpre[r][0] = (wave == 0 && act && r < nrhs) ? W[(long)r * ldw + jt] : T(0);
     } else {
 #pragma unroll
@@ -179,7 +236,7 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
             }
         }
 #pragma unroll
-        for (int r = 0; r < RPRE; ++r)
+        for (int r = 0; r < RDOT; ++r)
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
                 const int j = rbase + it * 4;
@@ -197,10 +254,17 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
             else
                 tile_load<T, MODE>(v2, M, lda, s0 + SB, s0, bs1, bs0, false, vec);
         }
-        // this wave's first right-hand side on the two sub-blocks
-        const bool r0ok = wave < nrhs;
-        const T xw0 = (r0ok && lane < bs0) ? W[(long)wave * ldw + s0 + lane] : T(0);
-        const T xw1 = (r0ok && nq > 1 && lane < bs1) ? W[(long)wave * ldw + s0 + SB + lane] : T(0);
+        // this wave's right-hand sides on the two sub-blocks, and the diagonal
+        T xw[2][NR], dg[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const bool in = lane < (q == 0 ? bs0 : bs1);
+            const long row = s0 + q * SB + lane;
+#pragma unroll
+            for (int k = 0; k < NR; ++k)
+                xw[q][k] = in && wave + 4 * k < nrhs ? W[(long)(wave + 4 * k) * ldw + row] : T(0);
+            dg[q] = MODE != LOWER_UNIT && in && wave < nrhs ? M[row * lda + row] : T(1);
+        }
         tile_store(tl[0], v0, vf0);
         if (nq > 1) {
             tile_store(tl[1], v1, vf1);
@@ -208,56 +272,70 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
         }
         __syncthreads();
 
-        // ---- 1. the super-block, redundantly in every workgroup
-        for (int r = wave; r < nrhs; r += 4) {
-#pragma clang fp contract(off)
-            T xq0 = T(0), xq1 = T(0);
-            for (int qi = 0; qi < nq; ++qi) {
-                const int q = fwd ? qi : nq - 1 - qi;
-                const int bs = q == 0 ? bs0 : bs1;
-                T x = r == wave ? (q == 0 ? xw0 : xw1)
-                                : (lane < bs ? W[(long)r * ldw + s0 + q * SB + lane] : T(0));
-                // The loops below run all 64 steps, unrolled, so the LDS reads of
-                // the tile are issued ahead of the serial chain.  Steps beyond the
-                // block size change nothing: the staged tiles are zero outside the
-                // block and x is zero on lanes beyond it, so they subtract exact
-                // zeros.
+        // ---- 1. the super-block, redundantly in every workgroup.  The loops run
+        // all 64 columns: the staged tiles are zero outside the block and x is
+        // zero on lanes beyond it, so the columns past it subtract exact zeros.
+        if (wave < nrhs) {
+            T sol[2][NR];
+#pragma unroll
+            for (int k = 0; k < NR; ++k) sol[0][k] = sol[1][k] = T(0);
+#pragma unroll
+            for (int qi = 0; qi < 2; ++qi) {
+                if (qi >= nq) break;
+                // the sub-block solved now; with one sub-block it is block 0
+                const bool second = fwd ? qi == 1 : qi == 0 && nq > 1;
+                T x[NR];
+#pragma unroll
+                for (int k = 0; k < NR; ++k) x[k] = second ? xw[1][k] : xw[0][k];
+                const T dl = second ? dg[1] : dg[0];
                 if (qi == 1) {  // contribution of the sub-block solved first
-                    const T xp = fwd ? xq0 : xq1;
-                    T m[SB];
+                    T m[SB], sum[NR];
                     tile_row<T, MODE>(tl[2], lane, m);
 #pragma unroll
-                    for (int c = 0; c < SB; ++c) {
-                        const T xc = lane_get(xp, c);
-                        x = x - m[c] * xc;
-                    }
-                }
-                const T(*d)[SB + TP<T>] = tl[q];
-                T dr[SB];  // this lane's row (column for the transposed form) of d
-                tile_row<T, MODE>(d, lane, dr);
-                const T dl = lane < bs ? d[lane][lane] : T(1);
-                const T rd = T(1) / dl;  // used by the FP32 form only
-                if (fwd) {
+                    for (int k = 0; k < NR; ++k) sum[k] = T(0);
 #pragma unroll
-                    for (int c = 0; c < SB; ++c) {
-                        if (MODE == LOWER && lane == c) x = diag_div(x, dl, rd);
-                        const T xc = lane_get(x, c);
-                        if (lane > c) x = x - dr[c] * xc;
-                    }
+                    for (int c = 0; c < SB; ++c)
+#pragma unroll
+                        for (int k = 0; k < NR; ++k) sum[k] = fma(m[c], lane_get(sol[0][k], c), sum[k]);
+#pragma unroll
+                    for (int k = 0; k < NR; ++k) x[k] -= sum[k];
+                }
+                const T(*t)[SB + TP<T>] = second ? tl[1] : tl[0];
+                T m[SB], y[NR];
+                tile_row<T, MODE>(t, lane, m);
+                if constexpr (MODE != LOWER_UNIT) {
+                    const T rd = T(1) / dl;
+#pragma unroll
+                    for (int c = 0; c < SB; ++c) m[c] = div_recip(m[c], dl, rd);
+#pragma unroll
+                    for (int k = 0; k < NR; ++k) y[k] = div_recip(x[k], dl, rd);
                 } else {
 #pragma unroll
-                    for (int cc = 0; cc < SB; ++cc) {
-                        const int c = SB - 1 - cc;
-                        if (lane == c) x = diag_div(x, dl, rd);
-                        const T xc = lane_get(x, c);
-                        if (lane < c) x = x - dr[c] * xc;
-                    }
+                    for (int k = 0; k < NR; ++k) y[k] = x[k];
                 }
-                if (lane >= bs) x = T(0);
-                if (q == 0) xq0 = x; else xq1 = x;
+#pragma unroll
+                for (int cc = 0; cc < SB; ++cc) {
+                    const int c = fwd ? cc : SB - 1 - cc;
+#pragma unroll
+                    for (int k = 0; k < NR; ++k) y[k] = fma(-m[c], lane_get(y[k], c), y[k]);
+                }
+#pragma unroll
+                for (int k = 0; k < NR; ++k) {
+                    if (__any(!(fabs(y[k]) < std::numeric_limits<T>::infinity())))
+                        y[k] = sweep_plain<T, MODE>(t, x[k], dl, lane);
+                    if (lane >= (second ? bs1 : bs0)) y[k] = T(0);
+                    sol[qi][k] = y[k];
+                }
             }
-            xs[r][lane] = xq0;
-            xs[r][SB + lane] = xq1;
+#pragma unroll
+            for (int k = 0; k < NR; ++k) {
+                const int r = wave + 4 * k;
+                const bool swap = !fwd && nq > 1;  // block 1 was solved first
+                if (r < nrhs) {
+                    xs[r][lane] = swap ? sol[1][k] : sol[0][k];
+                    xs[r][SB + lane] = swap ? sol[0][k] : sol[1][k];
+                }
+            }
         }
     }
     __syncthreads();
@@ -268,13 +346,32 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
         }
 
     // ---- 2. remove the solved rows from this workgroup's share of [u0, u1)
-    if constexpr (MODE == LOWER_T) {
+    if constexpr (PRODUCT) {
+        // four sums of 32 products each: one of 128 gave a solution of order 4096
+        // 1.5 times the backward error
+        typename Mfma<T>::acc part[4] = {};
+#pragma unroll
+        for (int u = 0; u < CW / VL; ++u)
+#pragma unroll
+            for (int e = 0; e < VL; ++e) {
+                const int i = u * VL + e;
+                part[i & 3] = Mfma<T>::op(mv[i], xs[ls][(4 * u + grp) * VL + e], part[i & 3]);
+            }
+        const typename Mfma<T>::acc acc = (part[0] + part[1]) + (part[2] + part[3]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int jw = jp + Mfma<T>::row(grp, q);
+            if (jw < u1 && ls < nrhs) W[(long)ls * ldw + jw] = wpre[0][q] - acc[q];
+        }
+    } else if constexpr (MODE == LOWER_T) {
         // W[r][j] -= sum_c L[s0 + c][j] * x[c]: a workgroup owns 64 entries j
         // (one per lane: coalesced rows of L), wave w sums c in [32w, 32w + 32)
         const bool act = jt < u1;
         // partial sums meet in LDS (the staged tiles are no longer read)
-        T(*red)[TMAXR][SB] = reinterpret_cast<T(*)[TMAXR][SB]>(&tl[0][0][0]);
-        for (int r = 0; r < nrhs; ++r) {
+        T(*red)[RDOT][SB] = reinterpret_cast<T(*)[RDOT][SB]>(&tl[0][0][0]);
+#pragma unroll
+        for (int r = 0; r < RDOT; ++r) {
+            if (r >= nrhs) break;
             T a = T(0);
 #pragma unroll
             for (int q = 0; q < CW; ++q) a += mv[q] * xs[r][wave * CW + q];
@@ -282,16 +379,19 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
         }
         __syncthreads();
         if (wave == 0 && act) {
-            for (int r = 0; r < nrhs; ++r) {
+#pragma unroll
+            for (int r = 0; r < RDOT; ++r) {
+                if (r >= nrhs) break;
                 const T a = (red[0][r][lane] + red[1][r][lane]) + (red[2][r][lane] + red[3][r][lane]);
-                const T w0 = r < RPRE ? wpre[r < RPRE ? r : 0][0] : W[(long)r * ldw + jt];
-                W[(long)r * ldw + jt] = w0 - a;
+                W[(long)r * ldw + jt] = wpre[r][0] - a;
             }
         }
     } else {
         // W[r][j] -= sum_c M[j][s0 + c] * x[c]; 16 lanes per row, 4 rows per
         // wave at a time, lane ls holds columns ls, ls + 16, ... (coalesced)
-        for (int r = 0; r < nrhs; ++r) {  // wave-uniform
+#pragma unroll
+        for (int r = 0; r < RDOT; ++r) {
+            if (r >= nrhs) break;
             T v[NIT];
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
@@ -301,16 +401,10 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
                 v[it] = row16_sum(a);  // the 16 lanes of a row are one DPP row
             }
             if (ls == 0) {
-                T w[NIT];
 #pragma unroll
                 for (int it = 0; it < NIT; ++it) {
                     const int j = rbase + it * 4;
-                    w[it] = r < RPRE ? wpre[r < RPRE ? r : 0][it] : (j < u1 ? W[(long)r * ldw + j] : T(0));
-                }
-#pragma unroll
-                for (int it = 0; it < NIT; ++it) {
-                    const int j = rbase + it * 4;
-                    if (j < u1) W[(long)r * ldw + j] = w[it] - v[it];
+                    if (j < u1) W[(long)r * ldw + j] = wpre[r][it] - v[it];
                 }
             }
         }
@@ -352,9 +446,15 @@ static int trsv_run(hipStream_t s, size_t n, const T *m, size_t lda, size_t nrhs
                 sizeof(T) * ((double)(s1 - s0) * (s1 - s0 + 1) / 2 + (double)(u1 - u0) * (s1 - s0) +
                              (double)nr * (2.0 * (u1 - u0) + 2.0 * (s1 - s0)));
             RLG_PROF_W("trsv", s, bytes);
-            hipLaunchKernelGGL((k_trsv_step<T, MODE>), dim3(grid), dim3(256), 0, s, m, (long)lda,
-                               (int)n, (int)q0, (int)nq, (int)nr, w + r0 * ldw, (long)ldw,
-                               x + r0 * ldx, (long)ldx, (int)u0, (int)u1, vec ? 1 : 0);
+            auto go = [&](auto nr_wave) {
+                hipLaunchKernelGGL((k_trsv_step<T, MODE, decltype(nr_wave)::value>), dim3(grid), dim3(256), 0,
+                                   s, m, (long)lda, (int)n, (int)q0, (int)nq, (int)nr, w + r0 * ldw, (long)ldw,
+                                   x + r0 * ldx, (long)ldx, (int)u0, (int)u1, vec ? 1 : 0);
+            };
+            // four waves: as few right-hand sides per wave as hold them all
+            if (nr <= (size_t)RDOT) go(std::integral_constant<int, 1>{});
+            else if (nr <= 8) go(std::integral_constant<int, 2>{});
+            else go(std::integral_constant<int, 4>{});
             RLG_LAUNCHED();
         }
     }
