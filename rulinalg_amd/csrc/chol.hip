@@ -22,6 +22,7 @@
 
 #include "kernels.hpp"
 #include "mfma.hpp"
+#include "recip.hpp"
 #include "wave.hpp"
 
 namespace rlg {
@@ -207,13 +208,6 @@ __device__ __forceinline__ void sqrt_recip(float d, float &s, float &r) {
     s = sqrtf(d);
     r = 1.0f / s;
 }
-// x / s from r = 1 / s: the quotient and one residual correction (Markstein),
-// left out where the residual is not finite.
-template <class T> __device__ __forceinline__ T div_recip(T x, T s, T r) {
-    const T q = x * r, e = fma(-q, s, x);
-    return fabs(e) < T(__builtin_inf()) ? fma(e, r, q) : q;
-}
-
 constexpr int PW = 16;           // panel width inside a block column
 constexpr int CLD = CNB + 2;     // LDS row of 64 (16-byte aligned)
 

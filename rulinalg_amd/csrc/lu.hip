@@ -10,34 +10,35 @@
 // depth-64 GEMM.
 //
 // The panel kernel keeps the whole (n - k) x 64 panel resident in LDS,
-// spread over G workgroups of PR rows each.  Every column costs one
-// exchange: each workgroup publishes its local pivot candidate (|value|,
-// row, and the full 64-wide row) and the content of the current diagonal
-// row as tagged words; every workgroup reads the G candidates, reduces them
-// to the same winner, performs its part of the row swap, and eliminates its
-// rows.  The pivot rule is the reference's: the first row of maximal
-// magnitude at or below the diagonal (strict `>` scan, lu.rs:170-178); the
-// multiplier is a division and the update a separately rounded multiply and
-// subtract (lu.rs:603-616), so a matrix no wider than one panel is factored
-// bit-identically to the reference.
+// spread over G workgroups of PanelRows rows each, and factors it 16 columns at a
+// time with a row's 16 entries in its thread's registers (see k_lu_panel).
+// With more than one workgroup every column costs one exchange: each publishes
+// its pivot candidate (|value|, row, and the row's 16 entries) as tagged words;
+// every workgroup reads the G candidates and reduces them to the same winner.
+// The pivot rule is the reference's: the first row of maximal magnitude at or
+// below the diagonal (strict `>` scan, lu.rs:170-178).  An order of at most 64
+// is factored bit-identically to the reference: there the multiplier is a
+// division and the update a separately rounded multiply and subtract
+// (lu.rs:603-616).
 #include <climits>
 #include <type_traits>
 
 #include "kernels.hpp"
 #include "mfma.hpp"
+#include "recip.hpp"
 #include "wave.hpp"
 
 namespace rlg {
 
 constexpr int PNB = 64;    // inner panel width
-// Panel rows per workgroup (LDS-resident): 256 (133 KB of LDS in FP64, one
-// workgroup per CU, so every workgroup of a panel is resident at once).
-constexpr int PR = 256;
-template <class T> struct PanelRows { static constexpr int value = PR; };
-template <> struct PanelRows<float> { static constexpr int value = 2 * PR; };  // same 133 KB
+constexpr int SPW = 16;    // columns held in registers at a time
+// Panel rows per workgroup (LDS-resident), one per thread: 256 in FP64 (146 KB
+// of LDS, one workgroup per CU, so every workgroup of a panel is resident at
+// once) and 512 in FP32 (the same bytes).
+template <class T> struct PanelRows { static constexpr int value = 256; };
+template <> struct PanelRows<float> { static constexpr int value = 512; };
 constexpr int ONB = 512;   // outer block: depth of the trailing GEMM
 constexpr int SWB = 256;   // swaps per k_laswp launch (its workgroup size)
-constexpr int PTHREADS = 256;
 // At most this many workgroups per panel: one per CU of the device and never
 // more than the exchange area holds.
 constexpr int GMAX = 256;
@@ -52,28 +53,37 @@ template <> __device__ __forceinline__ float eps_of<float>() { return 1.1920929e
 // Words are written and read with agent-scope atomics, and a reader polls
 // until every word it needs carries the current tag, so a value is never
 // used before it is complete and no counter, fence or barrier is involved.
-// A slot holds a header (candidate row, candidate |value|) and a 64-wide row;
-// a value takes one word in FP32 and two (low, high half) in FP64.
+// A candidate slot holds a header, the low word of |value| (read only to settle
+// a tie) and the row's entries in the 16 columns at hand; a pivot-row slot holds
+// a pivot row from those columns on.  A value takes one word in FP32 and two
+// (low, high half) in FP64.  The header is one word, so that a poll is one
+// load: the high word of |value| (rank_hi; 0: no candidate), the row in 17 bits
+// and the low 15 bits of the tag, which suffice since a slot's last content is
+// two columns old.
 typedef unsigned long long xword;
-constexpr int XHDR = 4;  // header words: row, |v| (1 or 2 words), spare
+constexpr int XHDR = 2;  // header and the low word of |value|
+__device__ __forceinline__ xword xhdr(unsigned hi, int row, unsigned tag) {
+    return ((xword)hi << 32) | ((unsigned)row << 15) | (tag & 0x7fffu);
+}
 template <class T> struct XSlot {
     static constexpr int VW = sizeof(T) / 4;                      // words per value
-    static constexpr int words = (XHDR + PNB * VW + 15) & ~15;    // 128-byte multiple
+    static constexpr int words = (XHDR + SPW * VW + 15) & ~15;    // 128-byte multiple
+    static constexpr int parity = GMAX * words;                   // candidates of one column parity
+    static constexpr int rows = SPW * PNB * VW;                   // pivot rows of one 16-column parity
 };
-// Slots per column parity: one per workgroup, then the diagonal-row slot.
-constexpr int XPAR = GMAX + 1;
 
 // Workspace layout (bytes): exchange slots, inverses of the unit-lower
 // diagonal blocks of the current outer block, timeout flag.
 struct LuWork {
-    xword *xch;        // [2][XPAR][XSlot<T>::words]
+    xword *xch;        // candidates [2][GMAX][words], then pivot rows [2][SPW][PNB]
     void *linv;        // [ONB / PNB][PNB][PNB] T
     int *timeout;      // exchange timeout flag
 };
 
 static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 static size_t xch_words(size_t elem) {
-    return 2 * (size_t)XPAR * (elem == 8 ? XSlot<double>::words : XSlot<float>::words);
+    return 2 * (size_t)(elem == 8 ? XSlot<double>::parity + XSlot<double>::rows
+                                  : XSlot<float>::parity + XSlot<float>::rows);
 }
 
 size_t lu_work_bytes(size_t n, size_t elem) {
@@ -152,325 +162,369 @@ __device__ __forceinline__ bool xwait(unsigned &spins, int *timeout) {
     return true;
 }
 
-// Factor the panel A[k:k+m, k:k+w] (w <= PNB) in place.
-//
-// Workgroup g holds rows [g PRT, (g+1) PRT) of the panel in LDS; thread t
-// owns the tile rows t + h PTHREADS and does every local step on them.  The
-// elimination is lazy by one column: pivot j is applied to column j + 1 at
-// once, and to the columns beyond during the next column's exchange, while
-// the workgroup waits for the other candidates anyway.  Column j:
-//   A. every thread finds the first maximum |a[r][j]| over its rows r >= j
-//      (column j is up to date); each wave copies its candidate row, and the
-//      wave holding row j that row, to LDS; barrier;
-//   B. wave 0 picks the workgroup's candidate and brings the copied rows up
-//      to date with pivot j - 1 (the arithmetic the owners apply in place),
-//      then publishes the candidate (row index, |value|, the row) and, if it
-//      holds row j, row j;
-//   C/D1. pivot j - 1 is applied to columns > j of every row; with other
-//      workgroups (G > 1, FP32) wave 0 meanwhile reads all G candidates, picks the
-//      same winner as every other workgroup and fetches the winning row
-//      unless it is its own (and, if it holds the winning row but not row j,
-//      row j), while waves 1-3 update all rows, wave 0's included; alone,
-//      every thread updates its own rows; barrier;
-//   D2. wave 0 swaps the rows it holds and puts the pivot row in LDS;
-//      barrier;
-//   E. every thread turns column j of its rows below j into multipliers and
-//      applies pivot j to column j + 1.
-// The pivot indices stay in LDS until the end: a global store before a
-// workgroup barrier would make the barrier wait for its completion.
+// The header at h once it carries `tag` in every lane (a wave-wide wait, given
+// up like xwait's).  Three loads are kept in flight: a load's round trip is
+// about 570 cycles, so polling one at a time would see a new word that much
+// late.
+__device__ __forceinline__ xword xpoll(const xword *h, unsigned tag, bool &live, int *timeout) {
+    auto has = [&](xword v) { return __all(((unsigned)v & 0x7fffu) == (tag & 0x7fffu)); };
+    xword a = xget(h);
+    __builtin_amdgcn_s_sleep(2);
+    xword b = xget(h);
+    __builtin_amdgcn_s_sleep(2);
+    xword c = xget(h);
+    for (unsigned spins = 0;;) {
+        if (has(a)) return a;
+        a = xget(h);
+        if (has(b)) return b;
+        b = xget(h);
+        if (has(c)) return c;
+        c = xget(h);
+        if (!xwait(spins, timeout)) { live = false; return 0; }
+    }
+}
+// The payload of the word at w once it carries `tag` in every lane, bounded
+// like xpoll.
+__device__ __forceinline__ unsigned xlow(const xword *w, unsigned tag, bool &live, int *timeout) {
+    for (unsigned spins = 0;;) {
+        const xword v = xget(w);
+        if (__all(xtag(v) == tag)) return (unsigned)v;
+        if (!xwait(spins, timeout)) { live = false; return 0; }
+    }
+}
 
-// Tile rows are padded to a 16-byte multiple: 16-byte aligned rows let the
-// row sweeps use 16-byte LDS accesses.
+// Tile rows are padded to a 16-byte multiple: 16-byte aligned rows let a
+// thread move its row with 16-byte LDS accesses, and a wave's rows then cover
+// all banks.
 template <class T> struct TilePad { static constexpr int value = 16 / sizeof(T); };
 template <class T> constexpr int TW = PNB + TilePad<T>::value;
 
-// a[r][c] = a[r][c] - mult * pm[c] for the columns c > j from chunk C0 on,
-// as one straight sweep: the row part is loaded, then stored.  The first
-// 8-column chunk may hold columns <= j.  With EXACT they keep their value,
-// by a select on the computed value, as in the reference, which never
-// touches them (x - mult * 0 would turn a -0 into +0, and a non-finite
-// multiplier would reach them).  Without EXACT they take x - mult * 0 (pm is
-// zero there), which differs from x only in the sign of a zero: the mixed
-// factorization, whose factors only precondition the FP64 refinement, uses
-// that form, which needs fewer registers.  Every column is stored
-// unconditionally: a per-column test around the store gets compiled into a
-// conditional store, one LDS round trip per column.  Columns w..63 of the
-// tile and of pm hold zeros and stay zero.
-template <class T, int C0, bool EXACT>
-__device__ __forceinline__ void elim_row(T (*__restrict__ tile)[TW<T>], const T *__restrict__ pm,
-                                         int r, int j, T mult) {
-#pragma clang fp contract(off)
-    T x[PNB - C0];
-#pragma unroll
-    for (int c = C0; c < PNB; ++c) x[c - C0] = tile[r][c];
-#pragma unroll
-    for (int c = C0; c < PNB; ++c) {
-        const T v = x[c - C0] - mult * pm[c];
-        tile[r][c] = (!EXACT || c >= C0 + 8 || c > j) ? v : x[c - C0];
-    }
-}
-
-// elim_row from the 8-column chunk that holds column j + 1.
+// Factor the panel A[k:k+m, k:k+w] (w <= PNB) in place.
+//
+// Workgroup g loads rows [g PRT, (g+1) PRT) of the panel into LDS, one per
+// thread, and a row stays with its thread: a swap only exchanges two rows'
+// positions (pos), and the rows are written to their positions at the end, when
+// every workgroup has long read its own (each took part in column 0's
+// exchange).  Sixteen columns at a time are held in registers.  Column j:
+//   - each wave finds its first maximum over the rows at positions >= j and
+//     copies that row's 16 entries to LDS; barrier; every wave picks the
+//     workgroup's candidate;
+//   - with other workgroups, wave 0 publishes the candidate (position, |value|,
+//     the entries), reads all G headers, picks the same winner as every
+//     other workgroup and fetches its entries; barrier; the winner's workgroup
+//     publishes the row from these columns on;
+//   - rows at positions > j form their multiplier and subtract the pivot row's
+//     entries right of j, in registers.
+// After 16 columns the pivot rows' part right of them (from LDS, or published)
+// is solved against the 16 x 16 unit-lower block and subtracted from the
+// remaining rows on the matrix cores.
+//
+// Bound by the serial chain per column (search, barrier, exchange), not by the
+// arithmetic.  Rows of 64 kept in LDS with three barriers per column and an
+// update of the whole row per column took, in FP64, 122 us for a panel of 256
+// rows and, on average over the factorization, 188 at order 1,531 and 209 at
+// 16,384; this form takes 68, 148 and 199.
+//
+// EXACT (FP32, and FP64 orders up to 64): divisions, and separately rounded
+// products and differences in the reference's order.
 template <class T, bool EXACT>
-__device__ __forceinline__ void elim_row_from(T (*__restrict__ tile)[TW<T>], const T *__restrict__ pm,
-                                              int r, int j, T mult) {
-    switch ((j + 1) >> 3) {
-        case 0: elim_row<T, 0, EXACT>(tile, pm, r, j, mult); break;
-        case 1: elim_row<T, 8, EXACT>(tile, pm, r, j, mult); break;
-        case 2: elim_row<T, 16, EXACT>(tile, pm, r, j, mult); break;
-        case 3: elim_row<T, 24, EXACT>(tile, pm, r, j, mult); break;
-        case 4: elim_row<T, 32, EXACT>(tile, pm, r, j, mult); break;
-        case 5: elim_row<T, 40, EXACT>(tile, pm, r, j, mult); break;
-        case 6: elim_row<T, 48, EXACT>(tile, pm, r, j, mult); break;
-        case 7: elim_row<T, 56, EXACT>(tile, pm, r, j, mult); break;
-        default: break;  // j = 63: nothing right of column j
-    }
-}
-
-template <class T, bool EXACT>
-__global__ __launch_bounds__(PTHREADS) void k_lu_panel(T *__restrict__ A, long lda, int k, int m,
-                                                       int w, int64_t *__restrict__ ipiv,
-                                                       int64_t *__restrict__ info, int n,
-                                                       xword *__restrict__ xch, int *timeout) {
+__global__ __launch_bounds__(PanelRows<T>::value) void k_lu_panel(
+    T *__restrict__ A, long lda, int k, int m, int w, int64_t *__restrict__ ipiv,
+    int64_t *__restrict__ info, int n, xword *__restrict__ xch, int *timeout) {
     constexpr int PRT = PanelRows<T>::value;
-    constexpr int RPT = PRT / PTHREADS;  // panel rows per thread
-    static_assert(RPT * PTHREADS == PRT, "whole rows per thread");
-    constexpr int NW = PTHREADS / 64;
-    constexpr int VW = XSlot<T>::VW, XS = XSlot<T>::words;
+    constexpr int NW = PRT / 64;
+    using X = XSlot<T>;
     __shared__ __attribute__((aligned(16))) T tile[PRT][TW<T>];
-    __shared__ __attribute__((aligned(16))) T prow[PNB];      // pivot row j
-    // pivot row j with zeros at columns <= j + 1, by column parity (its
-    // pending update is applied during column j + 1's step)
-    __shared__ __attribute__((aligned(16))) T pmask[2][PNB];
-    __shared__ T wrow[NW][PNB];                                // wave candidates' rows
-    __shared__ T jrow[PNB];                                    // row j
-    __shared__ T red_v[NW];
-    __shared__ int red_i[NW];
-    __shared__ int s_piv[PNB];
+    __shared__ __attribute__((aligned(16))) T urow[SPW][TW<T>];      // pivot rows of these columns
+    __shared__ __attribute__((aligned(16))) T cand[2][NW][SPW];      // wave candidates' entries
+    __shared__ __attribute__((aligned(16))) T prow[2][SPW];          // the winner's
+    // wave candidates: ranks of |value| (rank_hi, rank_lo; 0: none), position, thread
+    __shared__ uint4 red[2][NW];
+    __shared__ int s_win[2], s_own[2];          // winner's position; its thread here, or -1
+    __shared__ int s_piv[PNB], s_pos[PRT], s_row[SPW];
 
     const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x;
     const int r0 = g * PRT;
     const int rows = min(PRT, m - r0);
     const int lane = tid & 63, wave = tid >> 6;
 
-    {   // all loads in flight before the LDS stores (PRT x PNB / PTHREADS per thread)
-        constexpr int PER = PRT * PNB / PTHREADS;
-        T v[PER];
+    {   // all loads in flight before the LDS stores (64 values per thread)
+        T v[PNB];
 #pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const int e = q * PTHREADS + tid, r = e / PNB, c = e % PNB;
-            v[q] = (r < rows && c < w) ? A[(long)(k + r0 + r) * lda + k + c] : T(0);
+        for (int q = 0; q < PNB; ++q) {
+            const int r = q * NW + wave;
+            v[q] = (r < rows && lane < w) ? A[(long)(k + r0 + r) * lda + k + lane] : T(0);
         }
 #pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const int e = q * PTHREADS + tid, r = e / PNB, c = e % PNB;
-            if (r < rows) tile[r][c] = v[q];  // columns w..63 zero
-        }
+        for (int q = 0; q < PNB; ++q) tile[q * NW + wave][lane] = v[q];  // zero past w and m
     }
     __syncthreads();
 
-    bool live = true;  // wave 0: false once an exchange has timed out
-    int small = w;     // wave 0: first column whose pivot is below epsilon
-    for (int j = 0; j < w; ++j) {
-        const T *pmprev = pmask[(j + 1) & 1];  // masked pivot row j - 1
-        const bool own_j = j >= r0 && j < r0 + rows;
-
-        // A. this thread's candidate, the wave's, and the rows wave 0 needs
-        T bv = T(0);
-        int bi = INT_MAX;
+    bool live = true;  // false once a wait of this wave has timed out
+    int small = w;     // first column whose pivot is below epsilon
+    int pos = tid < rows ? r0 + tid : -1;
+    for (int cb = 0; cb < w; cb += SPW) {
+        xword *const prows = xch + 2 * X::parity + ((cb / SPW) & 1) * X::rows;
+        T x[SPW];
 #pragma unroll
-        for (int h = 0; h < RPT; ++h) {
-            const int r = tid + h * PTHREADS;
-            const T v = fabs(tile[r][j]);
-            const bool take = (r < rows) & (r0 + r >= j) & better(v, r0 + r, bv, bi);
-            bv = take ? v : bv;
-            bi = take ? r0 + r : bi;
-        }
-        {
-            const int wl = wave_first_max_lane(bv, bi);
-            bv = wl >= 0 ? lane_get(bv, wl) : T(0);
-            bi = wl >= 0 ? lane_get(bi, wl) : INT_MAX;
-        }
-        {   // the wave's candidate row and row j, brought up to date with pivot
-            // j - 1 right of column j (the arithmetic step C applies to the
-            // rows in place); columns <= j are final and stay as they are
-#pragma clang fp contract(off)
-            if (bi != INT_MAX) {
-                const T x = tile[bi - r0][lane];
-                const T v = x - tile[bi - r0][j > 0 ? j - 1 : 0] * pmprev[lane];
-                wrow[wave][lane] = (j > 0 && lane > j) ? v : x;
-            }
-            if (own_j && (((j - r0) % PTHREADS) >> 6) == wave) {
-                const T x = tile[j - r0][lane];
-                const T v = x - tile[j - r0][j > 0 ? j - 1 : 0] * pmprev[lane];
-                jrow[lane] = (j > 0 && lane > j) ? v : x;
-            }
-        }
-        if (lane == 0) { red_v[wave] = bv; red_i[wave] = bi; }
-        __syncthreads();
-
-        // B. the workgroup's candidate row and row j, published
-        T pv = T(0), oj = T(0);
-        if (wave == 0) {
-            int bw = 0;
+        for (int c = 0; c < SPW; ++c) x[c] = tile[tid][cb + c];
+        if (tid < SPW) s_row[tid] = -1;
+        // x[e] is the row's entry in column j + e: a column leaves the registers
+        // when it is done, so one loop body serves all 16 (expanded, they would
+        // be twice the instruction cache)
+#pragma unroll 1
+        for (int j = cb; j < min(cb + SPW, w); ++j) {
+            const int c = j - cb, par = j & 1;
+            const T av = fabs(x[0]);
+            const unsigned hi = pos >= j ? rank_hi(av) : 0u, lo = rank_lo(av);
+            const int wl = first_max_lane(hi, lo, pos);
+            if (lane == max(wl, 0)) {
+                red[par][wave] = uint4{wl < 0 ? 0u : hi, lo, (unsigned)pos, (unsigned)tid};
 #pragma unroll
-            for (int q = 1; q < NW; ++q) {
-                const bool take = better(red_v[q], red_i[q], bv, bi);
-                bv = take ? red_v[q] : bv;
-                bi = take ? red_i[q] : bi;
-                bw = take ? q : bw;
-            }
-            if (bi != INT_MAX) pv = wrow[bw][lane];
-            if (own_j) oj = jrow[lane];
-            if (G > 1 && live) {
-                const unsigned tag = (unsigned)(k + j + 1);
-                xword *base = xch + (size_t)(j & 1) * XPAR * XS;
-                xword *mine = base + (size_t)g * XS, *diag = base + (size_t)GMAX * XS;
-                if (lane < w) {
-                    if (bi != INT_MAX) xput_val(mine + XHDR + lane * VW, tag, pv);
-                    if (own_j) xput_val(diag + XHDR + lane * VW, tag, oj);
-                }
-                if (lane == 0) {
-                    xput(mine, tag, (unsigned)bi);
-                    xput_val(mine + 1, tag, bv);
+                for (int e = 0; e < SPW / 2; ++e) cand[par][wave][e] = x[e];
+                if (c < SPW / 2) {  // later, the rest are past the 16 columns
+#pragma unroll
+                    for (int e = SPW / 2; e < SPW; ++e) cand[par][wave][e] = x[e];
                 }
             }
-        }
-
-        // D1 / C.  With other workgroups to hear from, wave 0 waits for the
-        // exchange (D1) while waves 1-3 apply pivot j - 1 to every row,
-        // wave 0's included (C); alone, each wave updates its own rows.
-        // (FP32 only: with two rows per thread the hand-over spreads evenly;
-        // with one, a wave of 1-3 would do twice its work, measured slower;
-        // FP64 updates its rows first and then exchanges, after the barrier)
-        const bool w0_exchange = RPT > 1 && G > 1;  // uniform
-        int p = bi;
-        T pabs = bv;
-        auto exchange = [&]() {
-            if (live) {
+            __syncthreads();
+            const uint4 rw = red[par][lane % NW];
+            unsigned top = dpp_max<DPP_XOR2>(dpp_max<DPP_XOR1>(rw.x));  // over each NW lanes
+            if constexpr (NW > 4) top = dpp_max<DPP_HALF_MIRROR>(top);
+            const unsigned tied = (unsigned)__ballot(rw.x == top) & ((1u << NW) - 1);
+            int bw = __builtin_ctz(tied);
+            if (tied & (tied - 1)) bw = max(first_max_lane(lane < NW ? rw.x : 0u, rw.y, (int)rw.z), 0);
+            int p = lane_get((int)rw.z, bw), t = lane_get((int)rw.w, bw);
+            const T *pr = cand[par][bw];
+            if (G > 1) {
                 const unsigned tag = (unsigned)(k + j + 1);
-                const xword *base = xch + (size_t)(j & 1) * XPAR * XS;
-                const xword *diag = base + (size_t)GMAX * XS;
-                // every workgroup's candidate, 64 slots per round
-                T v = T(0);
-                int i = INT_MAX, gw = 0;
-                for (int q0 = 0; q0 < G && live; q0 += 64) {
-                    const int q = q0 + lane;
-                    const xword *h = base + (size_t)q * XS;
-                    T qv = T(0);
-                    int qi = INT_MAX;
-                    for (unsigned spins = 0;;) {
-                        bool ok = true;
-                        if (q < G) {
-                            const xword hr = xget(h);
-                            qv = xget_val<T>(h + 1, tag, ok);
-                            qi = (int)(unsigned)hr;
-                            ok = ok && xtag(hr) == tag;
-                        }
-                        if (__all(ok)) break;
-                        if (!xwait(spins, timeout)) { live = false; break; }
+                if (wave == 0) {
+                    xword *const base = xch + par * X::parity;
+                    xword *const slot = base + (size_t)g * X::words;
+                    const unsigned whi = lane_get(rw.x, bw);
+                    if (live && lane == 0)
+                        __hip_atomic_store(slot, xhdr(whi, whi ? p : 0, tag), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                    // lanes 16 (bw mod 4) .. + 15 hold the candidate's entries
+                    const bool holds = (lane >> 4) == (bw & 3);
+                    T own = cand[par][lane >> 4][lane & 15];
+                    if constexpr (NW > 4) {
+                        const T up = cand[par][4 + (lane >> 4)][lane & 15];
+                        own = bw < 4 ? own : up;
                     }
-                    const bool take = (q < G) & better(qv, qi, v, i);
-                    v = take ? qv : v;
-                    i = take ? qi : i;
-                    gw = take ? q : gw;
-                }
-                {
-                    const int wl = wave_first_max_lane(v, i);
-                    if (wl >= 0) {
-                        v = lane_get(v, wl);
-                        i = lane_get(i, wl);
-                        gw = lane_get(gw, wl);
-                    } else if (live) {  // no candidate anywhere: cannot happen; report it
-                        if (lane == 0)
+                    if (live) {
+                        if (holds && whi) xput_val(slot + XHDR + (lane & 15) * X::VW, tag, own);
+                        if (lane == 0) xput(slot + 1, tag, lane_get(rw.y, bw));
+                    }
+                    // every workgroup's header, 64 per round: lanes past G have none
+                    unsigned bh = 0, bl = 0;
+                    int i = INT_MAX, gw = g;
+                    for (int q0 = 0; q0 < G && live; q0 += 64) {
+                        const int q = q0 + lane;
+                        const xword *h = base + (size_t)min(q, G - 1) * X::words;
+                        const xword hw = xpoll(h, tag, live, timeout);
+                        const unsigned qh = q < G ? (unsigned)(hw >> 32) : 0u;
+                        const int qi = (int)((unsigned)hw >> 15);
+                        if (G <= 64) {
+                            bh = qh;
+                            i = qi;
+                            gw = q;
+                        } else {  // a tie between rounds needs the low words now
+                            const unsigned ql = xlow(h + 1, tag, live, timeout);
+                            const bool take = (qh > bh) | ((qh == bh) & ((ql > bl) | ((ql == bl) & (qi < i))));
+                            bh = take ? qh : bh;
+                            bl = take ? ql : bl;
+                            i = take ? qi : i;
+                            gw = take ? q : gw;
+                        }
+                    }
+                    const unsigned mh = wave_max_u32(bh);
+                    const unsigned long long at = __ballot(bh == mh);
+                    int win = __ffsll((long long)at) - 1;
+                    if (__popcll(at) > 1) {
+                        if (G <= 64) bl = xlow(base + (size_t)min(gw, G - 1) * X::words + 1, tag, live, timeout);
+                        win = first_max_lane(bh == mh ? bh : 0u, bl, i);
+                    }
+                    if (live && mh) {
+                        p = lane_get(i, win);
+                        gw = lane_get(gw, win);
+                    } else {  // no candidate anywhere cannot happen; report it
+                        if (live && lane == 0)
                             __hip_atomic_store(timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         live = false;
+                        gw = g;  // the result is discarded: keep indices in range
+                        p = j;
+                        t = -1;
                     }
-                }
-                if (live) {
-                    p = i;
-                    pabs = v;
-                    const bool need_row = gw != g;
-                    const bool need_j = p != j && p >= r0 && p < r0 + rows && !own_j;
-                    if (need_row || need_j) {
-                        for (unsigned spins = 0;;) {
-                            bool ok = true, okj = true;
-                            if (lane < w) {
-                                if (need_row) {
-                                    const T x = xget_val<T>(base + (size_t)gw * XS + XHDR + lane * VW, tag, ok);
-                                    if (ok) pv = x;
-                                }
-                                if (need_j) {
-                                    const T x = xget_val<T>(diag + XHDR + lane * VW, tag, okj);
-                                    if (okj) oj = x;
-                                }
-                            }
-                            if (__all(ok && okj)) break;
-                            if (!xwait(spins, timeout)) { live = false; break; }
+                    if (gw == g) {
+                        if (holds) prow[par][lane & 15] = own;
+                    } else {
+                        T pv = T(0);
+                        for (unsigned spins = 0; live;) {
+                            bool ok = true;
+                            if (lane < SPW) pv = xget_val<T>(base + (size_t)gw * X::words + XHDR + lane * X::VW, tag, ok);
+                            if (__all(ok)) break;
+                            if (!xwait(spins, timeout)) live = false;
                         }
+                        if (lane < SPW) prow[par][lane] = pv;
+                    }
+                    if (lane == 0) {
+                        s_win[par] = p;
+                        s_own[par] = gw == g ? t : -1;
                     }
                 }
-                // after a timeout the result is discarded: keep indices in range
-                if (!live) { p = bi; pabs = bv; }
+                __syncthreads();
+                p = s_win[par];
+                pr = prow[par];
+                t = __builtin_amdgcn_readfirstlane(s_own[par]);
+                // the winner's row from column cb on, for every workgroup's update
+                if (wave == 1 && t >= 0 && cb + SPW < w && cb + lane < PNB)
+                    xput_val(prows + (c * PNB + lane) * X::VW, tag,
+                             lane >= c && lane < SPW ? pr[lane - c] : tile[t][cb + lane]);
             }
-        };
-        if (wave == 0 && w0_exchange) exchange();
-        if (j > 0) {
-            if (!w0_exchange) {
-#pragma unroll
-                for (int h = 0; h < RPT; ++h) {
-                    const int r = tid + h * PTHREADS;
-                    if (r < rows && r0 + r >= j) elim_row_from<T, EXACT>(tile, pmprev, r, j, tile[r][j - 1]);
-                }
-            } else if (wave > 0) {
-                // own rows, then wave 0's 64 RPT rows spread over the 192 threads
-#pragma unroll
-                for (int h = 0; h < RPT; ++h) {
-                    const int r = tid + h * PTHREADS;
-                    if (r < rows && r0 + r >= j) elim_row_from<T, EXACT>(tile, pmprev, r, j, tile[r][j - 1]);
-                }
-                constexpr int XTRA = (64 * RPT + PTHREADS - 64 - 1) / (PTHREADS - 64);
-#pragma unroll
-                for (int q = 0; q < XTRA; ++q) {
-                    const int e = (tid - 64) + q * (PTHREADS - 64);
-                    const int r = (e % 64) + (e / 64) * PTHREADS;
-                    if (e < 64 * RPT && r < rows && r0 + r >= j) elim_row_from<T, EXACT>(tile, pmprev, r, j, tile[r][j - 1]);
-                }
-            }
-        }
-        __syncthreads();
-
-        // D2. (FP64: the exchange,) the swap and the pivot row
-        if (wave == 0) {
-            if (G > 1 && !w0_exchange) exchange();
-            // swap rows j and p where this workgroup holds them (lanes w..63
-            // carry zeros on both sides)
-            if (p != j) {
-                if (own_j) tile[j - r0][lane] = pv;
-                if (p >= r0 && p < r0 + rows) tile[p - r0][lane] = oj;
-            }
-            prow[lane] = pv;
-            pmask[j & 1][lane] = lane > j + 1 ? pv : T(0);
-            if (lane == 0) s_piv[j] = p;
-            if (pabs < eps_of<T>() && small == w) small = j;
-        }
-        __syncthreads();
-
-        // E. multipliers of column j; pivot j on column j + 1
-        {
+            const T piv = pr[0];
+            if (fabs(piv) < eps_of<T>() && small == w) small = j;
+            // a pivot row held here: its entries leave the registers
+            if (wave == 2 && t >= 0 && lane < SPW - c) tile[t][j + lane] = pr[lane];
+            if (tid == 0) s_piv[j] = p;
+            if (pos == p) { pos = j; s_row[c] = tid; }
+            else if (pos == j) pos = p;
+            if (pos > j) {
+                if constexpr (EXACT) {
 #pragma clang fp contract(off)
-            const T piv = prow[j];
-            const T pn = j + 1 < PNB ? prow[j + 1] : T(0);
+                    const T mult = x[0] / piv;
+                    tile[tid][j] = mult;
 #pragma unroll
-            for (int h = 0; h < RPT; ++h) {
-                const int r = tid + h * PTHREADS;
-                if (r < rows && r0 + r > j) {
-                    const T mult = tile[r][j] / piv;
-                    tile[r][j] = mult;
-                    if (j + 1 < PNB) tile[r][j + 1] = tile[r][j + 1] - mult * pn;
+                    for (int e = 1; e < SPW; ++e) x[e - 1] = x[e] - mult * pr[e];
+                } else {
+                    const T mult = div_recip(x[0], piv, recip(piv));
+                    tile[tid][j] = mult;
+#pragma unroll
+                    for (int e = 1; e <= SPW / 2; ++e) x[e - 1] = fma(-mult, pr[e], x[e]);
+                    if (c < SPW / 2) {
+#pragma unroll
+                        for (int e = SPW / 2 + 1; e < SPW; ++e) x[e - 1] = fma(-mult, pr[e], x[e]);
+                    }
                 }
             }
         }
+        s_pos[tid] = pos;
+        if (cb + SPW >= w) break;
+        __syncthreads();
+
+        // the pivot rows from column cb on
+        constexpr int PER = SPW * PNB / PRT;
+        if (G == 1) {
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                const int i = q * NW + wave;
+                if (cb + lane < PNB) urow[i][lane] = tile[s_row[i]][cb + lane];
+            }
+        } else {
+            T v[PER];
+            for (unsigned spins = 0; live;) {
+                bool ok = true;
+#pragma unroll
+                for (int q = 0; q < PER; ++q) {
+                    const int i = q * NW + wave;
+                    bool o = true;
+                    v[q] = T(0);
+                    if (cb + lane < PNB)
+                        v[q] = xget_val<T>(prows + (i * PNB + lane) * X::VW, (unsigned)(k + cb + i + 1), o);
+                    ok = ok && o;
+                }
+                if (__all(ok)) break;
+                if (!xwait(spins, timeout)) { live = false; break; }
+            }
+#pragma unroll
+            for (int q = 0; q < PER; ++q) urow[q * NW + wave][lane] = live ? v[q] : T(0);
+        }
+        __syncthreads();
+        // U12 = L11^-1 A12, one column per lane
+        if (wave == 0 && lane < PNB - SPW - cb) {
+            T u[SPW];
+#pragma unroll
+            for (int i = 0; i < SPW; ++i) u[i] = urow[i][SPW + lane];
+#pragma unroll
+            for (int q = 0; q < SPW - 1; ++q)
+#pragma unroll
+                for (int i = q + 1; i < SPW; ++i) {
+                    if constexpr (EXACT) {
+#pragma clang fp contract(off)
+                        u[i] = u[i] - urow[i][q] * u[q];
+                    } else {
+                        u[i] = fma(-urow[i][q], u[q], u[i]);
+                    }
+                }
+#pragma unroll
+            for (int i = 1; i < SPW; ++i) urow[i][SPW + lane] = u[i];
+        }
+        __syncthreads();
+        if constexpr (EXACT) {
+            // this thread's row, or with at most 64 rows row `lane` and every
+            // NW-th group of columns
+            constexpr int VL = 16 / (int)sizeof(T);
+            typedef T vT __attribute__((ext_vector_type(VL)));
+            const bool few = rows <= 64;
+            const int row = few ? lane : tid;
+            if (s_pos[row] >= cb + SPW) {
+#pragma clang fp contract(off)
+                T mult[SPW];
+#pragma unroll
+                for (int c = 0; c < SPW; ++c) mult[c] = tile[row][cb + c];
+                for (int col = cb + SPW + (few ? wave * VL : 0); col < w; col += few ? NW * VL : VL) {
+                    vT v = *reinterpret_cast<const vT *>(&tile[row][col]);
+#pragma unroll
+                    for (int c = 0; c < SPW; ++c) {
+                        const vT u = *reinterpret_cast<const vT *>(&urow[c][col - cb]);
+#pragma unroll
+                        for (int e = 0; e < VL; ++e) v[e] = v[e] - mult[c] * u[e];
+                    }
+                    *reinterpret_cast<vT *>(&tile[row][col]) = v;
+                }
+            }
+        } else {
+            // this wave's 64 rows: A22 -= L21 U12, four independent 16 x 16 tiles
+            // per 16 columns; rows already chosen keep their values
+            const int lr = lane & 15, lk = lane >> 4;
+            T af[4][4];
+            int ps[4][4];
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    af[rt][s] = tile[wave * 64 + rt * 16 + lr][cb + 4 * s + lk];
+                    ps[rt][s] = s_pos[wave * 64 + rt * 16 + Mfma<T>::row(lk, s)];
+                }
+            for (int ct = cb + SPW; ct < PNB; ct += 16) {
+                T bf[4], cv[4][4];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) bf[s] = urow[4 * s + lk][ct - cb + lr];
+#pragma unroll
+                for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) cv[rt][r] = tile[wave * 64 + rt * 16 + Mfma<T>::row(lk, r)][ct + lr];
+                typename Mfma<T>::acc acc[4] = {};
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll
+                    for (int rt = 0; rt < 4; ++rt) acc[rt] = Mfma<T>::op(af[rt][s], bf[s], acc[rt]);
+#pragma unroll
+                for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const T v = cv[rt][r] - acc[rt][r];
+                        // (a chosen row is not even written: it may be taking its U12)
+                        if (ps[rt][r] >= cb + SPW) tile[wave * 64 + rt * 16 + Mfma<T>::row(lk, r)][ct + lr] = v;
+                    }
+            }
+        }
+        // the pivot rows held here take their U12
+        for (int i = wave; i < SPW; i += NW) {
+            const int t = s_row[i];
+            if (t >= 0 && cb + SPW + lane < PNB) tile[t][cb + SPW + lane] = urow[i][SPW + lane];
+        }
+        __syncthreads();
     }
     __syncthreads();
 
@@ -478,11 +532,10 @@ __global__ __launch_bounds__(PTHREADS) void k_lu_panel(T *__restrict__ A, long l
         if (tid < w) ipiv[k + tid] = (int64_t)k + s_piv[tid];
         if (tid == 0 && small < w && *info == (int64_t)n) *info = k + small;
     }
-    constexpr int PER = PRT * PNB / PTHREADS;
 #pragma unroll 8
-    for (int q = 0; q < PER; ++q) {
-        const int e = q * PTHREADS + tid, r = e / PNB, c = e % PNB;
-        if (r < rows && c < w) A[(long)(k + r0 + r) * lda + k + c] = tile[r][c];
+    for (int q = 0; q < PNB; ++q) {
+        const int r = q * NW + wave;
+        if (r < rows && lane < w) A[(long)(k + s_pos[r]) * lda + k + lane] = tile[r][lane];
     }
 }
 
@@ -756,16 +809,6 @@ __global__ __launch_bounds__(256) void k_trsm_llu(T *__restrict__ A, long lda, i
 // Set by lu_factor_lowp for its duration: FP32 panels are then factored with
 // tournament pivoting (tslu.hip) in this workspace.
 static thread_local void *g_tslu_work = nullptr;
-// Cleared by lu_factor_lowp for its duration: the mixed factorization's
-// panels may turn a -0 left of the pivot column into +0 (see elim_row); the
-// drop-in factorizations keep the reference's zeros exactly.
-static thread_local bool g_panel_exact = true;
-
-template <class T>
-static const void *panel_kernel() {
-    return g_panel_exact ? reinterpret_cast<const void *>(k_lu_panel<T, true>)
-                         : reinterpret_cast<const void *>(k_lu_panel<T, false>);
-}
 
 template <class T>
 static int panel(hipStream_t s, T *a, size_t lda, size_t k, size_t m, size_t w, int64_t *ipiv,
@@ -797,10 +840,11 @@ template <class T>
 static int panel_rows_max(size_t *out) {
     Device *d = nullptr;
     RLG_TRY(current_device(&d));
-    static thread_local int per_cu[2][2] = {{-1, -1}, {-1, -1}};
-    int &bpc = per_cu[sizeof(T) == 8][g_panel_exact];
+    static thread_local int per_cu[2] = {-1, -1};
+    int &bpc = per_cu[sizeof(T) == 8];
     if (bpc < 0)
-        RLG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, panel_kernel<T>(), PTHREADS, 0));
+        RLG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &bpc, reinterpret_cast<const void *>(k_lu_panel<T, sizeof(T) == 4>), PanelRows<T>::value, 0));
     size_t g = (size_t)bpc * (size_t)d->num_cus;
     if (g > (size_t)GMAX) g = GMAX;
     *out = g * PanelRows<T>::value;
@@ -819,6 +863,18 @@ static int panel(hipStream_t s, T *a, size_t lda, size_t k, size_t m, size_t w, 
     const unsigned G = ceil_div(m, PanelRows<T>::value);
     // algorithmic bytes: the m x w panel read once and written once
     RLG_PROF_W("lu_panel", s, 2.0 * (double)m * (double)w * sizeof(T));
+    constexpr unsigned PT = PanelRows<T>::value;
+    constexpr bool EX = sizeof(T) == 4;
+    if (G == 1) {  // no exchange; with the whole matrix in one panel the reference's bits
+        auto go = [&](auto exact) {
+            hipLaunchKernelGGL((k_lu_panel<T, decltype(exact)::value>), dim3(1), dim3(PT), 0, s, a, (long)lda,
+                               (int)k, (int)m, (int)w, ipiv, info, (int)n, lw.xch, lw.timeout);
+        };
+        if (EX || n <= (size_t)PNB) go(std::true_type{});
+        else go(std::integral_constant<bool, EX>{});
+        RLG_LAUNCHED();
+        return RLG_OK;
+    }
     // A cooperative launch: the runtime starts the grid only with every
     // workgroup resident at once (and refuses a grid that cannot be), which
     // the per-column exchange between workgroups relies on.
@@ -828,7 +884,8 @@ static int panel(hipStream_t s, T *a, size_t lda, size_t k, size_t m, size_t w, 
     xword *xch_ = lw.xch;
     int *to_ = lw.timeout;
     void *args[] = {&a_, &lda_, &k_, &m_, &w_, &ipiv, &info, &n_, &xch_, &to_};
-    RLG_HIP(hipLaunchCooperativeKernel(panel_kernel<T>(), dim3(G), dim3(PTHREADS), args, 0, s));
+    RLG_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k_lu_panel<T, EX>), dim3(G), dim3(PT),
+                                       args, 0, s));
     return RLG_OK;
 }
 
@@ -1055,7 +1112,6 @@ int lu_factor_lowp(hipStream_t s, int prec, int pivot, size_t n, float *a, size_
     g_lowp_pack2 = static_cast<char *>(g_lowp_pack) + pack;
     g_lowp_pack_bytes = gemm_lowp_pack_bytes(n, n, ONB);
     g_tslu_work = nullptr;
-    g_panel_exact = false;
     int st = RLG_OK;
     UpdateFn<float> aux = nullptr;
     if (pivot == RLG_PIVOT_TOURNAMENT) {
@@ -1070,7 +1126,6 @@ int lu_factor_lowp(hipStream_t s, int prec, int pivot, size_t n, float *a, size_
     g_lowp_pack2 = nullptr;
     g_lowp_pack_bytes = 0;
     g_tslu_work = nullptr;
-    g_panel_exact = true;
     return st;
 }
 

@@ -86,20 +86,6 @@ int tslu_reset(hipStream_t s, void *work, size_t n) {
     return fill_u32(tslu_carve(work, n).cnt, nodes, 0u, s);
 }
 
-// Maximum of a 32-bit key over the wave (uniform): two quad swaps and two row
-// mirrors, then the four rows' maxima.
-__device__ __forceinline__ unsigned wave_max_u32(unsigned k) {
-    k = max(k, (unsigned)dpp<DPP_XOR1>((int)k));
-    k = max(k, (unsigned)dpp<DPP_XOR2>((int)k));
-    k = max(k, (unsigned)dpp<DPP_HALF_MIRROR>((int)k));
-    k = max(k, (unsigned)dpp<DPP_MIRROR>((int)k));
-    const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)k, 0);
-    const unsigned b = (unsigned)__builtin_amdgcn_readlane((int)k, 16);
-    const unsigned c = (unsigned)__builtin_amdgcn_readlane((int)k, 32);
-    const unsigned d = (unsigned)__builtin_amdgcn_readlane((int)k, 48);
-    return max(max(a, b), max(c, d));
-}
-
 // Shared state of one partial-pivoting run over 256 rows.
 struct GeppShared {
     float cand[2][4][TW];   // each wave's candidate row, by column parity

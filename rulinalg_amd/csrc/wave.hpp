@@ -54,24 +54,23 @@ template <int CTRL> __device__ __forceinline__ double dpp(double x) {
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
-__device__ __forceinline__ unsigned long long lane_get(unsigned long long x, int l) {
-    const int lo = __builtin_amdgcn_readlane((int)x, l);
-    const int hi = __builtin_amdgcn_readlane((int)(x >> 32), l);
-    return ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo;
-}
-template <int CTRL> __device__ __forceinline__ unsigned long long dpp(unsigned long long x) {
-    const int lo = dpp<CTRL>((int)x), hi = dpp<CTRL>((int)(x >> 32));
-    return ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo;
-}
-
-// Maximum of a 64-bit key over the wave (uniform result): two quad swaps
+// Maximum of a 32-bit key over the wave (uniform result): two quad swaps
 // and two row mirrors, then the four rows' maxima from lanes 0, 16, 32, 48.
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long k) {
-    auto mx = [](unsigned long long a, unsigned long long b) { return a > b ? a : b; };
-    k = mx(k, dpp<DPP_XOR1>(k));
-    k = mx(k, dpp<DPP_XOR2>(k));
-    k = mx(k, dpp<DPP_HALF_MIRROR>(k));
-    k = mx(k, dpp<DPP_MIRROR>(k));
+__device__ __forceinline__ unsigned lane_get(unsigned x, int l) {
+    return (unsigned)__builtin_amdgcn_readlane((int)x, l);
+}
+// max(x, x of the lane CTRL names): bound control with a zero fill lets the
+// compiler fuse the move into the maximum.
+template <int CTRL> __device__ __forceinline__ unsigned dpp_max(unsigned x) {
+    const unsigned y = (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, true);
+    return x > y ? x : y;
+}
+__device__ __forceinline__ unsigned wave_max_u32(unsigned k) {
+    auto mx = [](unsigned a, unsigned b) { return a > b ? a : b; };
+    k = dpp_max<DPP_XOR1>(k);
+    k = dpp_max<DPP_XOR2>(k);
+    k = dpp_max<DPP_HALF_MIRROR>(k);
+    k = dpp_max<DPP_MIRROR>(k);
     return mx(mx(lane_get(k, 0), lane_get(k, 16)), mx(lane_get(k, 32), lane_get(k, 48)));
 }
 
@@ -105,33 +104,35 @@ __device__ __forceinline__ bool better(T v2, int i2, T v1, int i1) {
     return (i2 != INT_MAX) & ((i1 == INT_MAX) | (v2 > v1) | (!(v1 > v2) & (i2 < i1)));
 }
 
-// The lane that holds the wave's first maximum under `better` (largest
-// |value|, ties to the smallest row index; i == INT_MAX marks a lane without
-// a candidate), or -1 if no lane has one; uniform.  One 64-bit maximum over
-// the wave: in FP32 the key packs the value's bits (a non-negative float
-// orders like its bits) above the complemented row index, so keys are
-// distinct; in FP64 the key is the value's bits + 1 and a tie is settled by
-// the smallest index among the tied lanes.  A NaN ranks like zero.
-__device__ __forceinline__ int wave_first_max_lane(float v, int i) {
-    unsigned long long key = 0;
-    if (i != INT_MAX) {
-        const unsigned b = (v == v) ? __float_as_uint(v) : 0u;
-        key = ((unsigned long long)b << 32) | (0xFFFFFFFFu - (unsigned)i);
-    }
-    const unsigned long long m = wave_max_u64(key);
-    if (m == 0) return -1;
-    return __ffsll((long long)__ballot(key == m)) - 1;
+// The high word of a magnitude plus one (a non-negative float orders like its
+// bits); a NaN ranks like zero.
+__device__ __forceinline__ unsigned rank_hi(float v) { return (v == v) ? __float_as_uint(v) + 1 : 1u; }
+__device__ __forceinline__ unsigned rank_hi(double v) {
+    return (v == v) ? (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) + 1 : 1u;
 }
-__device__ __forceinline__ int wave_first_max_lane(double v, int i) {
-    unsigned long long key = 0;
-    if (i != INT_MAX) key = (v == v) ? (unsigned long long)__double_as_longlong(v) + 1 : 1;
-    const unsigned long long m = wave_max_u64(key);
-    if (m == 0) return -1;
-    const unsigned long long tied = __ballot(key == m);
+__device__ __forceinline__ unsigned rank_lo(float) { return 0u; }
+__device__ __forceinline__ unsigned rank_lo(double v) {
+    return (v == v) ? (unsigned)(unsigned long long)__double_as_longlong(v) : 0u;
+}
+
+// The lane that holds the wave's first maximum under `better` (largest
+// |value|, ties to the smallest row index i), or -1 if no lane has a candidate;
+// uniform.  A lane without one passes hi = 0, else the ranks of its value.  The
+// high words settle it but for near-ties: one 32-bit maximum over the wave, a
+// fused DPP instruction per step, where a 64-bit one takes a compare and two
+// selects (610 against about 380 cycles).  Then the low words, then the indices.
+__device__ __forceinline__ int first_max_lane(unsigned hi, unsigned lo, int i) {
+    const unsigned mh = wave_max_u32(hi);
+    if (mh == 0) return -1;
+    const unsigned long long tied = __ballot(hi == mh);
     if (__popcll(tied) == 1) return __ffsll((long long)tied) - 1;
-    const int ii = key == m ? i : INT_MAX;
+    const unsigned ml = wave_max_u32(hi == mh ? lo : 0u);
+    const int ii = (hi == mh) & (lo == ml) ? i : INT_MAX;
     const int mi = wave_min_i32(ii);
     return __ffsll((long long)__ballot(ii == mi)) - 1;
+}
+template <class T> __device__ __forceinline__ int wave_first_max_lane(T v, int i) {
+    return first_max_lane(i != INT_MAX ? rank_hi(v) : 0u, rank_lo(v), i);
 }
 
 }  // namespace rlg
