@@ -142,6 +142,14 @@ template <> __device__ __forceinline__ double xget_val<double>(const xword *p, u
     return __longlong_as_double((long long)(((b & 0xffffffffull) << 32) | (a & 0xffffffffull)));
 }
 
+constexpr int XPOLLS = 6;  // header loads in flight, and their spacing in sleeps of 64 cycles
+constexpr int XPOLL_SLEEP = 6, XPOLL_GAP = 2;
+// Up to this many workgroups (16,384 rows in FP64), the candidates' entries are
+// read ahead, this many sleeps after the choice of the workgroup's own.  (From 8
+// to 16 sleeps, and from 3 to 8 header loads, the time of a factorization
+// differs by 1 %.)
+constexpr int XROWS = 64, XROWS_SLEEP = 12;
+
 // One round of a bounded wave-wide wait.  Returns false once the timeout
 // flag is up (checked every 256 rounds) or after 2^22 rounds, when it raises
 // the flag itself: an exchange that cannot complete then ends the kernel,
@@ -163,23 +171,24 @@ __device__ __forceinline__ bool xwait(unsigned &spins, int *timeout) {
 }
 
 // The header at h once it carries `tag` in every lane (a wave-wide wait, given
-// up like xwait's).  Three loads are kept in flight: a load's round trip is
-// about 570 cycles, so polling one at a time would see a new word that much
-// late.
+// up like xwait's).  A word takes about 1,450 cycles from one workgroup to
+// another and a load's round trip is about 1,000, so several loads are kept in
+// flight: polled one at a time, a word would be seen up to a round trip late.
 __device__ __forceinline__ xword xpoll(const xword *h, unsigned tag, bool &live, int *timeout) {
-    auto has = [&](xword v) { return __all(((unsigned)v & 0x7fffu) == (tag & 0x7fffu)); };
-    xword a = xget(h);
-    __builtin_amdgcn_s_sleep(2);
-    xword b = xget(h);
-    __builtin_amdgcn_s_sleep(2);
-    xword c = xget(h);
+    constexpr int N = XPOLLS;
+    xword v[N];
+    __builtin_amdgcn_s_sleep(XPOLL_SLEEP);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        if (i) __builtin_amdgcn_s_sleep(XPOLL_GAP);
+        v[i] = xget(h);
+    }
     for (unsigned spins = 0;;) {
-        if (has(a)) return a;
-        a = xget(h);
-        if (has(b)) return b;
-        b = xget(h);
-        if (has(c)) return c;
-        c = xget(h);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (__all(((unsigned)v[i] & 0x7fffu) == (tag & 0x7fffu))) return v[i];
+            v[i] = xget(h);
+        }
         if (!xwait(spins, timeout)) { live = false; return 0; }
     }
 }
@@ -209,10 +218,12 @@ template <class T> constexpr int TW = PNB + TilePad<T>::value;
 //   - each wave finds its first maximum over the rows at positions >= j and
 //     copies that row's 16 entries to LDS; barrier; every wave picks the
 //     workgroup's candidate;
-//   - with other workgroups, wave 0 publishes the candidate (position, |value|,
-//     the entries), reads all G headers, picks the same winner as every
-//     other workgroup and fetches its entries; barrier; the winner's workgroup
-//     publishes the row from these columns on;
+//   - with other workgroups, wave 0 publishes a header (position, |value|),
+//     reads all G headers and picks the same winner as every other workgroup;
+//     meanwhile wave 1 publishes the candidate's entries and waves 1.. read the
+//     other candidates' (at order 4,096 8 % of the factorization
+//     less than fetching the winner's entries after the choice);
+//     barrier; the winner's workgroup publishes the row from these columns on;
 //   - rows at positions > j form their multiplier and subtract the pivot row's
 //     entries right of j, in registers.
 // After 16 columns the pivot rows' part right of them (from LDS, or published)
@@ -223,7 +234,7 @@ template <class T> constexpr int TW = PNB + TilePad<T>::value;
 // arithmetic.  Rows of 64 kept in LDS with three barriers per column and an
 // update of the whole row per column took, in FP64, 122 us for a panel of 256
 // rows and, on average over the factorization, 188 at order 1,531 and 209 at
-// 16,384; this form takes 68, 148 and 199.
+// 16,384; this form takes 68, 148 and 184.
 //
 // EXACT (FP32, and FP64 orders up to 64): divisions, and separately rounded
 // products and differences in the reference's order.
@@ -237,10 +248,11 @@ __global__ __launch_bounds__(PanelRows<T>::value) void k_lu_panel(
     __shared__ __attribute__((aligned(16))) T tile[PRT][TW<T>];
     __shared__ __attribute__((aligned(16))) T urow[SPW][TW<T>];      // pivot rows of these columns
     __shared__ __attribute__((aligned(16))) T cand[2][NW][SPW];      // wave candidates' entries
-    __shared__ __attribute__((aligned(16))) T prow[2][SPW];          // the winner's
+    __shared__ __attribute__((aligned(16))) T rows_in[XROWS][SPW];   // other workgroups'
     // wave candidates: ranks of |value| (rank_hi, rank_lo; 0: none), position, thread
     __shared__ uint4 red[2][NW];
-    __shared__ int s_win[2], s_own[2];          // winner's position; its thread here, or -1
+    __shared__ int4 s_win[2];     // the winner's position, workgroup, and thread here or -1
+    __shared__ int s_got[XROWS];  // whether rows_in[] is complete
     __shared__ int s_piv[PNB], s_pos[PRT], s_row[SPW];
 
     const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x;
@@ -298,23 +310,14 @@ __global__ __launch_bounds__(PanelRows<T>::value) void k_lu_panel(
             const T *pr = cand[par][bw];
             if (G > 1) {
                 const unsigned tag = (unsigned)(k + j + 1);
+                xword *const base = xch + par * X::parity;
+                xword *const slot = base + (size_t)g * X::words;
+                const unsigned whi = lane_get(rw.x, bw);
                 if (wave == 0) {
-                    xword *const base = xch + par * X::parity;
-                    xword *const slot = base + (size_t)g * X::words;
-                    const unsigned whi = lane_get(rw.x, bw);
-                    if (live && lane == 0)
+                    if (live && lane == 0) {
                         __hip_atomic_store(slot, xhdr(whi, whi ? p : 0, tag), __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
-                    // lanes 16 (bw mod 4) .. + 15 hold the candidate's entries
-                    const bool holds = (lane >> 4) == (bw & 3);
-                    T own = cand[par][lane >> 4][lane & 15];
-                    if constexpr (NW > 4) {
-                        const T up = cand[par][4 + (lane >> 4)][lane & 15];
-                        own = bw < 4 ? own : up;
-                    }
-                    if (live) {
-                        if (holds && whi) xput_val(slot + XHDR + (lane & 15) * X::VW, tag, own);
-                        if (lane == 0) xput(slot + 1, tag, lane_get(rw.y, bw));
+                        xput(slot + 1, tag, lane_get(rw.y, bw));
                     }
                     // every workgroup's header, 64 per round: lanes past G have none
                     unsigned bh = 0, bl = 0;
@@ -356,27 +359,58 @@ __global__ __launch_bounds__(PanelRows<T>::value) void k_lu_panel(
                         p = j;
                         t = -1;
                     }
-                    if (gw == g) {
-                        if (holds) prow[par][lane & 15] = own;
-                    } else {
-                        T pv = T(0);
-                        for (unsigned spins = 0; live;) {
-                            bool ok = true;
-                            if (lane < SPW) pv = xget_val<T>(base + (size_t)gw * X::words + XHDR + lane * X::VW, tag, ok);
-                            if (__all(ok)) break;
-                            if (!xwait(spins, timeout)) live = false;
-                        }
-                        if (lane < SPW) prow[par][lane] = pv;
-                    }
                     if (lane == 0) {
-                        s_win[par] = p;
-                        s_own[par] = gw == g ? t : -1;
+                        s_win[par] = int4{p, gw, gw == g ? t : -1, 0};
+                        if (G > XROWS) s_got[0] = 0;
+                    }
+                } else {
+                    if (wave == 1 && whi && lane < SPW) xput_val(slot + XHDR + lane * X::VW, tag, pr[lane]);
+                    // Meanwhile the candidates' entries: the choice takes about as
+                    // long as they take to arrive.
+                    if (G <= XROWS) {
+                        constexpr int WPR = SPW * X::VW, PW = 64 / WPR;  // words per row, rows per load
+                        constexpr int LD = (XROWS + PW * (NW - 1) - 1) / (PW * (NW - 1));
+                        unsigned *const rw32 = reinterpret_cast<unsigned *>(&rows_in[0][0]);
+                        __builtin_amdgcn_s_sleep(XROWS_SLEEP);
+                        xword v[LD];
+#pragma unroll
+                        for (int q = 0; q < LD; ++q) {
+                            const int r = (q * (NW - 1) + wave - 1) * PW + lane / WPR;
+                            v[q] = r < G ? xget(base + (size_t)r * X::words + XHDR + lane % WPR) : 0;
+                        }
+#pragma unroll
+                        for (int q = 0; q < LD; ++q) {
+                            const int r = (q * (NW - 1) + wave - 1) * PW + lane / WPR;
+                            const unsigned long long good = __ballot(xtag(v[q]) == tag);
+                            constexpr unsigned long long one = WPR == 64 ? ~0ull : (1ull << WPR) - 1;
+                            if (r < G) {
+                                rw32[r * WPR + lane % WPR] = (unsigned)v[q];
+                                if (lane % WPR == 0) s_got[r] = ((good >> (lane / WPR * WPR)) & one) == one;
+                            }
+                        }
                     }
                 }
                 __syncthreads();
-                p = s_win[par];
-                pr = prow[par];
-                t = __builtin_amdgcn_readfirstlane(s_own[par]);
+                const int4 sw = s_win[par];
+                p = __builtin_amdgcn_readfirstlane(sw.x);
+                t = __builtin_amdgcn_readfirstlane(sw.z);
+                const int gw = __builtin_amdgcn_readfirstlane(sw.y);
+                if (gw != g) {
+                    pr = rows_in[G <= XROWS ? gw : 0];
+                    if (!__builtin_amdgcn_readfirstlane(s_got[G <= XROWS ? gw : 0])) {  // not there yet
+                        if (wave == 0) {
+                            T pv = T(0);
+                            for (unsigned spins = 0; live;) {
+                                bool ok = true;
+                                if (lane < SPW) pv = xget_val<T>(base + (size_t)gw * X::words + XHDR + lane * X::VW, tag, ok);
+                                if (__all(ok)) break;
+                                if (!xwait(spins, timeout)) live = false;
+                            }
+                            if (lane < SPW) rows_in[G <= XROWS ? gw : 0][lane] = pv;
+                        }
+                        __syncthreads();
+                    }
+                }
                 // the winner's row from column cb on, for every workgroup's update
                 if (wave == 1 && t >= 0 && cb + SPW < w && cb + lane < PNB)
                     xput_val(prows + (c * PNB + lane) * X::VW, tag,
