@@ -34,6 +34,7 @@ template <class T>
 int upload_matrix(hipStream_t s, T *dst, size_t ldd, const T *src, size_t lds, size_t rows,
                   size_t cols) {
     if (rows == 0 || cols == 0) return RLG_OK;
+    if (ldd == cols) return upload_rows(s, dst, src, lds * sizeof(T), cols * sizeof(T), rows);
     RLG_HIP(hipMemcpy2DAsync(dst, ldd * sizeof(T), src, lds * sizeof(T), cols * sizeof(T), rows,
                              hipMemcpyHostToDevice, s));
     return RLG_OK;
@@ -43,6 +44,7 @@ template <class T>
 int download_matrix(hipStream_t s, T *dst, size_t ldd, const T *src, size_t lds, size_t rows,
                     size_t cols) {
     if (rows == 0 || cols == 0) return RLG_OK;
+    if (lds == cols) return download_rows(s, dst, ldd * sizeof(T), src, cols * sizeof(T), rows);
     RLG_HIP(hipMemcpy2DAsync(dst, ldd * sizeof(T), src, lds * sizeof(T), cols * sizeof(T), rows,
                              hipMemcpyDeviceToHost, s));
     return RLG_OK;
@@ -74,10 +76,10 @@ int gemm_host(size_t a_rows, size_t a_cols, const T *a, size_t lda, size_t b_row
     RLG_TRY(current_device(&d));
     hipStream_t s = d->stream;
     const size_t m = a_rows, k = a_cols, n = b_cols;
-    DevBuf da, db, dc;
-    RLG_TRY(da.alloc(m * k * sizeof(T)));
-    RLG_TRY(db.alloc(k * n * sizeof(T)));
-    RLG_TRY(dc.alloc(m * n * sizeof(T)));
+    CallBuf da, db, dc;
+    RLG_TRY(da.alloc(m * k * sizeof(T), s));
+    RLG_TRY(db.alloc(k * n * sizeof(T), s));
+    RLG_TRY(dc.alloc(m * n * sizeof(T), s));
     RLG_TRY(upload_matrix<T>(s, da.as<T>(), k, a, lda, m, k));
     RLG_TRY(upload_matrix<T>(s, db.as<T>(), n, b, ldb, k, n));
     if (k == 0) {
@@ -95,16 +97,16 @@ int gemm_host(size_t a_rows, size_t a_cols, const T *a, size_t lda, size_t b_row
 // ---------------------------------------------------------------- LU
 
 template <class T>
-int lu_finish(hipStream_t s, rlg_lu *h, int64_t *ipiv_d, int64_t *info_d, void *work) {
+int lu_finish(hipStream_t s, rlg_lu *h, int64_t *ipiv_d, void *work) {
     const size_t n = h->n;
-    int64_t info = 0;
-    int timeout = 0;
-    h->ipiv.assign(n, 0);
+    // the pivots, *info and the timeout flag in one copy
+    RLG_TRY(widen_flag(lu_timeout_flag(work, n, sizeof(T)), ipiv_d + n + 1, s));
+    h->ipiv.assign(n + 2, 0);
     h->raw.assign(n, 0);
-    if (n) RLG_HIP(hipMemcpyAsync(h->ipiv.data(), ipiv_d, n * 8, hipMemcpyDeviceToHost, s));
-    RLG_HIP(hipMemcpyAsync(&info, info_d, 8, hipMemcpyDeviceToHost, s));
-    RLG_HIP(hipMemcpyAsync(&timeout, lu_timeout_flag(work, n, sizeof(T)), 4, hipMemcpyDeviceToHost, s));
+    RLG_HIP(hipMemcpyAsync(h->ipiv.data(), ipiv_d, (n + 2) * 8, hipMemcpyDeviceToHost, s));
     RLG_HIP(hipStreamSynchronize(s));
+    const int64_t info = h->ipiv[n], timeout = h->ipiv[n + 1];
+    h->ipiv.resize(n);
     if (timeout) {
         set_error("LU panel barrier timed out (workgroups not co-resident)");
         return RLG_E_DEVICE;
@@ -124,13 +126,12 @@ int lu_finish(hipStream_t s, rlg_lu *h, int64_t *ipiv_d, int64_t *info_d, void *
 template <class T>
 int lu_factor_handle(hipStream_t s, rlg_lu *h) {
     const size_t n = h->n;
-    PoolBuf ipiv, info, work;
-    RLG_TRY(ipiv.alloc(n * 8, s));
-    RLG_TRY(info.alloc(8, s));
+    PoolBuf ipiv, work;  // n pivots, *info, the timeout flag
+    RLG_TRY(ipiv.alloc((n + 2) * 8, s));
     RLG_TRY(work.alloc(lu_work_bytes(n, sizeof(T)), s));
-    RLG_TRY(lu_factor<T>(s, n, static_cast<T *>(h->a), h->lda, ipiv.as<int64_t>(), info.as<int64_t>(),
+    RLG_TRY(lu_factor<T>(s, n, static_cast<T *>(h->a), h->lda, ipiv.as<int64_t>(), ipiv.as<int64_t>() + n,
                          work.p));
-    return lu_finish<T>(s, h, ipiv.as<int64_t>(), info.as<int64_t>(), work.p);
+    return lu_finish<T>(s, h, ipiv.as<int64_t>(), work.p);
 }
 
 template <class T>
@@ -330,14 +331,14 @@ int rlg_matvec_f64(size_t m, size_t n, const double *a, size_t lda, size_t v_len
     Device *d;
     RLG_TRY(current_device(&d));
     hipStream_t s = d->stream;
-    DevBuf da, dv, dy;
-    RLG_TRY(da.alloc(m * n * 8));
-    RLG_TRY(dv.alloc(n * 8));
-    RLG_TRY(dy.alloc(m * 8));
+    CallBuf da, dv, dy;
+    RLG_TRY(da.alloc(m * n * 8, s));
+    RLG_TRY(dv.alloc(n * 8, s));
+    RLG_TRY(dy.alloc(m * 8, s));
     RLG_TRY(upload_matrix<double>(s, da.as<double>(), n, a, lda, m, n));
-    RLG_HIP(hipMemcpyAsync(dv.p, v, n * 8, hipMemcpyHostToDevice, s));
+    RLG_HIP(hipMemcpyAsync(dv.as<double>(), v, n * 8, hipMemcpyHostToDevice, s));
     RLG_TRY(gemv_f64(s, m, n, da.as<double>(), n, dv.as<double>(), dy.as<double>()));
-    RLG_HIP(hipMemcpyAsync(y, dy.p, m * 8, hipMemcpyDeviceToHost, s));
+    RLG_HIP(hipMemcpyAsync(y, dy.as<double>(), m * 8, hipMemcpyDeviceToHost, s));
     RLG_HIP(hipStreamSynchronize(s));
     return RLG_OK;
 }
@@ -561,11 +562,7 @@ int rlg_lu_det_f64(const rlg_lu *lu, double *det) {
     std::vector<double> diag(n);
     Device *d;
     RLG_TRY(current_device(&d));
-    // the diagonal as one strided copy (row pitch lda + 1)
-    if (n)
-        RLG_HIP(hipMemcpy2DAsync(diag.data(), 8, lu->a, (lu->lda + 1) * 8, 8, n,
-                                 hipMemcpyDeviceToHost, d->stream));
-    RLG_HIP(hipStreamSynchronize(d->stream));
+    RLG_TRY(download_diag<double>(d->stream, diag.data(), static_cast<const double *>(lu->a), lu->lda, n));
     // lu.rs:291-300: fold the diagonal from one, times the parity of p.
     double u_det = 1.0;
     for (size_t i = 0; i < n; ++i) u_det = u_det * diag[i];
@@ -667,10 +664,7 @@ int rlg_chol_det_f64(const rlg_chol *ch, double *det) {
     std::vector<double> diag(n);
     Device *d;
     RLG_TRY(current_device(&d));
-    if (n)
-        RLG_HIP(hipMemcpy2DAsync(diag.data(), 8, ch->a, (ch->lda + 1) * 8, 8, n,
-                                 hipMemcpyDeviceToHost, d->stream));
-    RLG_HIP(hipStreamSynchronize(d->stream));
+    RLG_TRY(download_diag<double>(d->stream, diag.data(), static_cast<const double *>(ch->a), ch->lda, n));
     double l_det = 1.0;  // cholesky.rs:175-180
     for (size_t i = 0; i < n; ++i) l_det = l_det * diag[i];
     *det = l_det * l_det;

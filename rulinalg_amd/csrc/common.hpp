@@ -124,6 +124,27 @@ struct PoolBuf {
     template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
+// Operands of one host-pointer call: pooled up to 64 MB (hipMalloc and hipFree
+// took longer than a small product), beyond that allocated and freed.  At the
+// call's end the free list keeps at most 1 GB in buffers of that size; the
+// oldest are freed.
+struct CallBuf {
+    static constexpr size_t POOLED = 64u << 20, MOST = 1u << 30;
+    PoolBuf pooled;
+    DevBuf own;
+    ~CallBuf();
+    int alloc(size_t n, hipStream_t s) { return n <= POOLED ? pooled.alloc(n, s) : own.alloc(n); }
+    template <class T> T *as() const { return static_cast<T *>(own.p ? own.p : pooled.p); }
+};
+
+// Copies between host rows of `width` bytes, `pitch` apart, and a contiguous
+// device buffer.  One linear copy: a 2D copy of pageable memory moves one row at
+// a time, 9 us each (256 rows of 2 KB: 2.4 ms against 25 us).  Rows that are not
+// contiguous on the host go through a temporary buffer.  A download of such rows
+// waits for the stream; otherwise both are asynchronous like hipMemcpyAsync.
+int upload_rows(hipStream_t s, void *dst, const void *src, size_t pitch, size_t width, size_t rows);
+int download_rows(hipStream_t s, void *dst, size_t pitch, const void *src, size_t width, size_t rows);
+
 // The streams that ran work reading a factor handle's device memory, so that
 // freeing the handle waits for exactly those streams.
 struct StreamUse {
@@ -185,5 +206,9 @@ inline unsigned ceil_div(size_t a, size_t b) { return (unsigned)((a + b - 1) / b
 int fill_u32(uint32_t *p, size_t count, uint32_t v, hipStream_t s);
 int fill_i64(int64_t *p, size_t count, int64_t v, hipStream_t s);
 int copy_f64(double *dst, const double *src, size_t count, hipStream_t s);
+// *dst = *src, as a word of the pivots' array.
+int widen_flag(const int *src, int64_t *dst, hipStream_t s);
+// The diagonal of a device matrix to the host; waits for the stream.
+template <class T> int download_diag(hipStream_t s, T *dst, const T *a, size_t lda, size_t n);
 
 }  // namespace rlg

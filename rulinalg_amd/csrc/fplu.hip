@@ -380,9 +380,7 @@ int fplu_factor_handle(hipStream_t s, rlg_fplu *h) {
     h->p = inverse_of(rp);
     h->q = inverse_of(rq);
     std::vector<T> dg(n);
-    if (n)
-        RLG_HIP(hipMemcpy2DAsync(dg.data(), sizeof(T), h->a, (h->lda + 1) * sizeof(T), sizeof(T), n,
-                                 hipMemcpyDeviceToHost, s));
+    RLG_TRY(download_diag<T>(s, dg.data(), static_cast<const T *>(h->a), h->lda, n));
     RLG_TRY(h->rp_d.alloc(n * 8, s));
     RLG_TRY(h->q_d.alloc(n * 8, s));
     RLG_TRY(h->rq_d.alloc(n * 8, s));
@@ -415,12 +413,7 @@ int fplu_decompose_host(size_t rows, size_t cols, const T *a, size_t lda, rlg_fp
     int st = h->own.alloc(rows * rows * sizeof(T), s);
     if (st == RLG_OK) {
         h->a = h->own.p;
-        if (rows)
-            if (hipMemcpy2DAsync(h->a, rows * sizeof(T), a, lda * sizeof(T), rows * sizeof(T), rows,
-                                 hipMemcpyHostToDevice, s) != hipSuccess) {
-                set_error("upload failed");
-                st = RLG_E_DEVICE;
-            }
+        st = upload_rows(s, h->a, a, lda * sizeof(T), rows * sizeof(T), rows);
     }
     if (st == RLG_OK) st = fplu_factor_handle<T>(s, h);
     if (st != RLG_OK) { delete h; return st; }
@@ -485,11 +478,9 @@ int fplu_solve_host(const rlg_fplu *h, size_t b_len, size_t nrhs, const T *b, si
     PoolBuf db, dx;
     RLG_TRY(db.alloc(nrhs * n * sizeof(T), s));
     RLG_TRY(dx.alloc(nrhs * n * sizeof(T), s));
-    RLG_HIP(hipMemcpy2DAsync(db.p, n * sizeof(T), b, ldb * sizeof(T), n * sizeof(T), nrhs, hipMemcpyHostToDevice,
-                             s));
+    RLG_TRY(upload_rows(s, db.p, b, ldb * sizeof(T), n * sizeof(T), nrhs));
     RLG_TRY(fplu_solve_dev<T>(s, h, nrhs, db.as<T>(), n, dx.as<T>(), n, true_solution));
-    RLG_HIP(hipMemcpy2DAsync(x, ldx * sizeof(T), dx.p, n * sizeof(T), n * sizeof(T), nrhs, hipMemcpyDeviceToHost,
-                             s));
+    RLG_TRY(download_rows(s, x, ldx * sizeof(T), dx.p, n * sizeof(T), nrhs));
     RLG_HIP(hipStreamSynchronize(s));
     return RLG_OK;
 }
@@ -503,8 +494,11 @@ int fplu_unpack(const rlg_fplu *h, T *l, T *u) {
     Device *d;
     RLG_TRY(current_device(&d));
     std::vector<T> lu(n * n);
-    RLG_HIP(hipMemcpy2DAsync(lu.data(), n * sizeof(T), h->a, h->lda * sizeof(T), n * sizeof(T), n,
-                             hipMemcpyDeviceToHost, d->stream));
+    if (h->lda == n)
+        RLG_TRY(download_rows(d->stream, lu.data(), n * sizeof(T), h->a, n * sizeof(T), n));
+    else
+        RLG_HIP(hipMemcpy2DAsync(lu.data(), n * sizeof(T), h->a, h->lda * sizeof(T), n * sizeof(T), n,
+                                 hipMemcpyDeviceToHost, d->stream));
     RLG_HIP(hipStreamSynchronize(d->stream));
     // unit_lower_triangular_part (lu.rs:644-663), nullify_lower_triangular_part
     // (src/internal_utils.rs:5-12)

@@ -764,16 +764,16 @@ int rlg_solve_mixed_f64(size_t n, const double *a, size_t lda, size_t nrhs, cons
     Device *d;
     RLG_TRY(current_device(&d));
     hipStream_t s = d->stream;
-    DevBuf da, db, dx;
-    RLG_TRY(da.alloc(n * n * 8));
-    RLG_TRY(db.alloc(nrhs * n * 8));
-    RLG_TRY(dx.alloc(nrhs * n * 8));
-    RLG_HIP(hipMemcpy2DAsync(da.p, n * 8, a, lda * 8, n * 8, n, hipMemcpyHostToDevice, s));
-    RLG_HIP(hipMemcpy2DAsync(db.p, n * 8, b, ldb * 8, n * 8, nrhs, hipMemcpyHostToDevice, s));
+    CallBuf da, db, dx;
+    RLG_TRY(da.alloc(n * n * 8, s));
+    RLG_TRY(db.alloc(nrhs * n * 8, s));
+    RLG_TRY(dx.alloc(nrhs * n * 8, s));
+    RLG_TRY(upload_rows(s, da.as<char>(), a, lda * 8, n * 8, n));
+    RLG_TRY(upload_rows(s, db.as<char>(), b, ldb * 8, n * 8, nrhs));
     int st = rlg_solve_mixed_f64_dev(n, da.as<double>(), n, nrhs, db.as<double>(), n, dx.as<double>(),
                                      n, opts, rep, s);
     if (st != RLG_OK && st != RLG_E_NOT_CONVERGED) return st;
-    RLG_HIP(hipMemcpy2DAsync(x, ldx * 8, dx.p, n * 8, n * 8, nrhs, hipMemcpyDeviceToHost, s));
+    RLG_TRY(download_rows(s, x, ldx * 8, dx.as<char>(), n * 8, nrhs));
     RLG_HIP(hipStreamSynchronize(s));
     return st;
 }

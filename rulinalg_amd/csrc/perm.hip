@@ -111,16 +111,14 @@ static int permute_host(bool by_rows, size_t perm_len, const size_t *perm, size_
     RLG_TRY(dp.alloc(perm_len * 8, s));
     RLG_TRY(dinv.alloc(perm_len * 8, s));
     std::vector<int64_t> p64(perm, perm + perm_len);
-    RLG_HIP(hipMemcpy2DAsync(da.p, cols * sizeof(T), a, lda * sizeof(T), cols * sizeof(T), rows,
-                             hipMemcpyHostToDevice, s));
+    RLG_TRY(upload_rows(s, da.p, a, lda * sizeof(T), cols * sizeof(T), rows));
     RLG_HIP(hipMemcpyAsync(dp.p, p64.data(), perm_len * 8, hipMemcpyHostToDevice, s));
     if (by_rows)
         RLG_TRY(permute_rows_dev<T>(s, rows, dp.as<int64_t>(), cols, da.as<T>(), cols, dout.as<T>(), cols));
     else
         RLG_TRY(permute_cols_dev<T>(s, rows, cols, dp.as<int64_t>(), da.as<T>(), cols, dout.as<T>(), cols,
                                     dinv.as<int64_t>()));
-    RLG_HIP(hipMemcpy2DAsync(out, ldo * sizeof(T), dout.p, cols * sizeof(T), cols * sizeof(T), rows,
-                             hipMemcpyDeviceToHost, s));
+    RLG_TRY(download_rows(s, out, ldo * sizeof(T), dout.p, cols * sizeof(T), rows));
     RLG_HIP(hipStreamSynchronize(s));
     return RLG_OK;
 }

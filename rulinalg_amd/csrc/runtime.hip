@@ -1,6 +1,7 @@
 // Runtime support: thread-local errors, per-device context, the event
 // profiler, small utility kernels and the device-memory C entry points.
 #include <cstdarg>
+#include <cstdlib>
 #include <map>
 
 #include "common.hpp"
@@ -156,6 +157,14 @@ std::vector<PoolEntry> &pool_entries() {
 }
 }  // namespace
 
+static void free_entry(PoolEntry &e) {
+    for (hipEvent_t ev : e.ready) {
+        (void)hipEventSynchronize(ev);
+        (void)hipEventDestroy(ev);
+    }
+    (void)hipFree(e.p);
+}
+
 int PoolBuf::alloc(size_t n, hipStream_t s) {
     release();
     if (n == 0) n = 256;
@@ -222,17 +231,89 @@ void PoolBuf::release_after(const std::vector<hipStream_t> &streams) {
     bytes = 0;
 }
 
+CallBuf::~CallBuf() {
+    if (!pooled.p) return;
+    pooled.release();
+    // sizes that keep growing leave buffers too small to be taken again
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    auto &v = pool_entries();
+    size_t held = 0;
+    for (auto &e : v) held += e.bytes <= POOLED ? e.bytes : 0;
+    for (size_t i = 0; i < v.size() && held > MOST;) {
+        if (v[i].bytes > POOLED) { ++i; continue; }
+        held -= v[i].bytes;
+        free_entry(v[i]);
+        v.erase(v.begin() + (long)i);
+    }
+}
+
 void pool_trim() {
     std::lock_guard<std::mutex> lk(g_pool_mu);
     auto &v = pool_entries();
-    for (auto &e : v) {
-        for (hipEvent_t ev : e.ready) {
-            (void)hipEventSynchronize(ev);
-            (void)hipEventDestroy(ev);
-        }
-        (void)hipFree(e.p);
-    }
+    for (auto &e : v) free_entry(e);
     v.clear();
+}
+
+// ------------------------------------------------------------------ host copies
+
+namespace {
+constexpr size_t STAGE = 32u << 20;  // bytes of host rows packed at a time
+}
+
+int upload_rows(hipStream_t s, void *dst, const void *src, size_t pitch, size_t width, size_t rows) {
+    if (!width || !rows) return RLG_OK;
+    if (!dst || !src) RLG_HIP(hipErrorInvalidValue);
+    if (pitch < width) RLG_HIP(hipErrorInvalidPitchValue);
+    if (pitch == width || rows == 1) {
+        RLG_HIP(hipMemcpyAsync(dst, src, width * rows, hipMemcpyHostToDevice, s));
+        return RLG_OK;
+    }
+    const size_t step = width < STAGE ? STAGE / width : 1;
+    char *tmp = static_cast<char *>(std::malloc((rows < step ? rows : step) * width));
+    if (!tmp) {
+        (void)hipStreamSynchronize(s);  // copies enqueued before
+        set_error("out of host memory");
+        return RLG_E_OOM;
+    }
+    hipError_t e = hipSuccess;
+    for (size_t r = 0; r < rows && e == hipSuccess; r += step) {
+        const size_t k = rows - r < step ? rows - r : step;
+        for (size_t i = 0; i < k; ++i)
+            std::memcpy(tmp + i * width, static_cast<const char *>(src) + (r + i) * pitch, width);
+        e = hipMemcpyAsync(static_cast<char *>(dst) + r * width, tmp, k * width, hipMemcpyHostToDevice, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+    }
+    std::free(tmp);
+    RLG_HIP(e);
+    return RLG_OK;
+}
+
+int download_rows(hipStream_t s, void *dst, size_t pitch, const void *src, size_t width, size_t rows) {
+    if (!width || !rows) return RLG_OK;
+    if (!dst || !src) RLG_HIP(hipErrorInvalidValue);
+    if (pitch < width) RLG_HIP(hipErrorInvalidPitchValue);
+    if (pitch == width || rows == 1) {
+        RLG_HIP(hipMemcpyAsync(dst, src, width * rows, hipMemcpyDeviceToHost, s));
+        return RLG_OK;
+    }
+    const size_t step = width < STAGE ? STAGE / width : 1;
+    char *tmp = static_cast<char *>(std::malloc((rows < step ? rows : step) * width));
+    if (!tmp) {
+        (void)hipStreamSynchronize(s);  // copies enqueued before
+        set_error("out of host memory");
+        return RLG_E_OOM;
+    }
+    hipError_t e = hipSuccess;
+    for (size_t r = 0; r < rows && e == hipSuccess; r += step) {
+        const size_t k = rows - r < step ? rows - r : step;
+        e = hipMemcpyAsync(tmp, static_cast<const char *>(src) + r * width, k * width, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        for (size_t i = 0; i < k && e == hipSuccess; ++i)
+            std::memcpy(static_cast<char *>(dst) + (r + i) * pitch, tmp + i * width, width);
+    }
+    std::free(tmp);
+    RLG_HIP(e);
+    return RLG_OK;
 }
 
 // ------------------------------------------------------------------ kernels
@@ -262,6 +343,34 @@ int fill_i64(int64_t *p, size_t count, int64_t v, hipStream_t s) {
     RLG_LAUNCHED();
     return RLG_OK;
 }
+
+// dst[i] = a[i * lda + i], and the panel's timeout flag as a word behind the
+// pivots, so that each reaches the host in one linear copy
+template <class T> __global__ void k_diag(const T *a, size_t lda, size_t n, T *dst) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = a[i * lda + i];
+}
+__global__ void k_widen(const int *src, int64_t *dst) { *dst = *src; }
+
+int widen_flag(const int *src, int64_t *dst, hipStream_t s) {
+    hipLaunchKernelGGL(k_widen, dim3(1), dim3(1), 0, s, src, dst);
+    RLG_LAUNCHED();
+    return RLG_OK;
+}
+
+template <class T> int download_diag(hipStream_t s, T *dst, const T *a, size_t lda, size_t n) {
+    if (!n) return RLG_OK;
+    PoolBuf d;
+    RLG_TRY(d.alloc(n * sizeof(T), s));
+    hipLaunchKernelGGL(k_diag<T>, dim3(ceil_div(n, 256)), dim3(256), 0, s, a, lda, n, d.as<T>());
+    RLG_LAUNCHED();
+    RLG_HIP(hipMemcpyAsync(dst, d.p, n * sizeof(T), hipMemcpyDeviceToHost, s));
+    RLG_HIP(hipStreamSynchronize(s));
+    return RLG_OK;
+}
+template int download_diag<double>(hipStream_t, double *, const double *, size_t, size_t);
+template int download_diag<float>(hipStream_t, float *, const float *, size_t, size_t);
+
 int copy_f64(double *dst, const double *src, size_t count, hipStream_t s) {
     if (!count) return RLG_OK;
     hipLaunchKernelGGL(k_copy_f64, dim3(ceil_div(count, 256)), dim3(256), 0, s, dst, src, count);
