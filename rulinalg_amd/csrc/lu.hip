@@ -996,7 +996,7 @@ static int update_lowp(hipStream_t s, size_t m, size_t n, size_t k, const float 
 
 // The look-ahead's update on the second stream.  Its workgroups reserve LDS
 // they do not use, so that one of them and one workgroup of the panel chain
-// (tournament, row swaps, block-row solve, depth-64 update: at most 67 KB)
+// (tournament, row swaps, block-row solve, depth-64 update: at most 70 KB)
 // share a CU, where two of them would fill its 160 KB: the split FP16
 // kernel stages 80 KB, the FP32 one 66 KB.
 constexpr size_t LU_SPLIT_PAD = 8 << 10, LU_F32_PAD = 24 << 10;

@@ -9,8 +9,8 @@
 // Two launches factor the m x w panel A[k:k+m, k:k+w] (w <= 64):
 //
 // k_tslu_tourney, one 256-thread workgroup per 256-row leaf:
-//   1. each workgroup runs partial pivoting on its leaf (one row per thread,
-//      in registers) and writes the row numbers of its w winners;
+//   1. each workgroup runs partial pivoting on its leaf and writes the row
+//      numbers of its w winners;
 //   2. every tree node merges up to four children: the workgroup that
 //      completes the last child (an atomic arrival count per node) loads the
 //      children's winners' original rows and runs partial pivoting on those
@@ -36,6 +36,7 @@ namespace rlg {
 constexpr int TW = 64;    // panel width
 constexpr int TLR = 256;  // rows per leaf = threads per workgroup
 constexpr int TF = 4;     // children per tree node: 4 x 64 candidates = 256 rows
+constexpr int TG = 16;    // columns held in registers at a time
 static_assert(TF * TW == TLR, "a merge has as many rows as a leaf");
 
 // Tree of L leaves: level 0 has L nodes, level l + 1 has ceil(n_l / TF).
@@ -86,122 +87,317 @@ int tslu_reset(hipStream_t s, void *work, size_t n) {
     return fill_u32(tslu_carve(work, n).cnt, nodes, 0u, s);
 }
 
-// Shared state of one partial-pivoting run over 256 rows.
-struct GeppShared {
-    float cand[2][4][TW];   // each wave's candidate row, by column parity
-    unsigned key[2][4];     // its |value| bits + 1 (0: the wave has no row left)
-    int id[2][4];           // its row number
-    int order[TW];          // row number of pivot j (-1: none)
+// Shared memory of the tournament kernel (69 KB, so that one workgroup fits
+// beside one of the look-ahead's update): the 256 x 64 tile and the
+// partial-pivoting state, and at the root, in the tile's place, the pivot block
+// and the two triangles being inverted.
+struct TourneyShared {
+    union {
+        float tile[TLR * TW];      // see `at`
+        struct {
+            float F[TW][TW + 1];
+            float L[TW][TW + 1];   // L11, then L11^-1
+            float Ut[TW][TW + 1];  // U11^T, then (U11^-1)^T
+            float tmp[2][32][33];
+        };
+    };
+    float u[TG][TW - TG];          // U12 of a group of columns
+    unsigned long long act[4];     // rows of the tile not yet chosen
+    int id[TLR];                   // row numbers (-1: none)
+    int slot[TW];                  // tile row of pivot j (-1: none)
+    int order[TW];                 // its row number
+    int s_last;
 };
 
-// Partial pivoting on the 256 rows held one per thread (a[] = the row, id =
-// its row number or -1): at column j every wave proposes its largest
-// |a[j]| among the rows not yet chosen, the largest of the four proposals
-// is pivot j (ties: the lower wave, then the lower lane; the pivot choice is
-// free for the tournament), and the other rows are eliminated with it.  On
-// return the chosen row of step j holds its multipliers left of column j and
-// its U row from column j on; `step` is that j for the chosen rows, -1 for
-// the others.  One workgroup barrier per column.
-__device__ __forceinline__ void gepp256(float (&a)[TW], int id, int w, GeppShared &sh, int &step) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    step = -1;
-    static_for<TW>([&](auto jc) __attribute__((always_inline)) {
-        constexpr int j = decltype(jc)::value;
-        if (j < w) {
-            constexpr int par = j & 1;
-            const bool active = id >= 0 && step < 0;
-            const unsigned key = active ? __float_as_uint(fabsf(a[j])) + 1u : 0u;
-            const unsigned wmax = wave_max_u32(key);
-            if (wmax != 0u) {
-                const unsigned long long hit = __ballot(key == wmax);
-                const int wl = __ffsll((long long)hit) - 1;
-                if (lane == wl) {
-                    constexpr int c0 = j & ~3;
-#pragma unroll
-                    for (int c = c0; c < TW; c += 4)
-                        *reinterpret_cast<float4 *>(&sh.cand[par][wave][c]) =
-                            make_float4(a[c], a[c + 1], a[c + 2], a[c + 3]);
-                    sh.id[par][wave] = id;
-                }
-            }
-            if (lane == 0) sh.key[par][wave] = wmax;
-            __syncthreads();
-            unsigned best = sh.key[par][0];
-            int ww = 0;
-#pragma unroll
-            for (int q = 1; q < 4; ++q) {
-                const unsigned kq = sh.key[par][q];
-                if (kq > best) { best = kq; ww = q; }
-            }
-            const int pid = best ? sh.id[par][ww] : -1;
-            if (tid == 0) sh.order[j] = pid;
-            if (best && id == pid) {
-                step = j;
-            } else if (best && active) {
-                const float p = sh.cand[par][ww][j];
-                const float m = p != 0.f ? a[j] * __builtin_amdgcn_rcpf(p) : 0.f;
-                a[j] = m;
-#pragma unroll
-                for (int c = j + 1; c < TW; ++c) a[c] = fmaf(-m, sh.cand[par][ww][c], a[c]);
-            }
-        } else {
-            if (tid == 0) sh.order[j] = -1;
-        }
-    });
-    __syncthreads();
+// Entry (row, col) of the tile.  The 16-byte pieces of a row are permuted by its
+// number, so that 16 consecutive rows read at one column touch all banks.
+__device__ __forceinline__ int at(int row, int col) {
+    return row * TW + (((col >> 2) ^ (row & 15)) << 2) + (col & 3);
 }
 
-// Row `id` of the panel (columns k .. k+w-1, zeros beyond) into a[].
-__device__ __forceinline__ void load_row(float (&a)[TW], const float *__restrict__ A, long lda, int k,
-                                         int id, int w, bool vec) {
-    if (id < 0) {
+// The value again, unknown to the compiler: addresses made from it are formed
+// where they are used, not ahead of a loop and kept in scratch memory.
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// The value, known to be the same in every lane.
+__device__ __forceinline__ unsigned long long uniform(unsigned long long v) {
+    return ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+           (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+}
+// b where this lane's bit of the (uniform) mask is clear, else a.
+template <class V> __device__ __forceinline__ V bit_of(unsigned long long mask, V a, V b) {
+    return __builtin_amdgcn_inverse_ballot_w64(mask) ? a : b;
+}
+
+// Rows sh.id[] of the panel into the tile (columns k .. k+w-1, zeros beyond).
+__device__ __forceinline__ void load_rows(TourneyShared &sh, const float *__restrict__ A, long lda, int k, int w,
+                                          bool vec) {
+    const int tid = opaque(threadIdx.x), c = (tid & 15) * 4, r0 = tid >> 4;
+    float4 v[16];
 #pragma unroll
-        for (int c = 0; c < TW; ++c) a[c] = 0.f;
-        return;
-    }
-    const float *r = A + (long)id * lda + k;
-    if (vec && w == TW) {
-#pragma unroll
-        for (int c = 0; c < TW; c += 4) {
-            const float4 v = *reinterpret_cast<const float4 *>(r + c);
-            a[c] = v.x; a[c + 1] = v.y; a[c + 2] = v.z; a[c + 3] = v.w;
+    for (int q = 0; q < 16; ++q) {
+        const int id = sh.id[q * 16 + r0];
+        const float *r = A + (long)id * lda + k + c;
+        v[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (id < 0) continue;
+        if (vec && w == TW) {
+            v[q] = *reinterpret_cast<const float4 *>(r);
+        } else {
+            if (c < w) v[q].x = r[0];
+            if (c + 1 < w) v[q].y = r[1];
+            if (c + 2 < w) v[q].z = r[2];
+            if (c + 3 < w) v[q].w = r[3];
         }
-    } else {
-#pragma unroll
-        for (int c = 0; c < TW; ++c) a[c] = c < w ? r[c] : 0.f;
     }
+#pragma unroll
+    for (int q = 0; q < 16; ++q) *reinterpret_cast<float4 *>(&sh.tile[at(q * 16 + r0, c)]) = v[q];
+}
+
+// Columns cb .. cb+15 of the tile and the pivot rows' part right of them, by one
+// wave: lane l holds rows l, l + 64, l + 128 and l + 192 in registers, so that a
+// column needs no barrier.  The pivot is the largest |value| of the rows not yet
+// chosen (ties: any; the choice is free for the tournament).  Every lane sets
+// its best row's entries aside while the maximum is found, so that no branch
+// (about 120 cycles) follows it; the winner's reach all lanes through scalar
+// registers, and the other rows form their multipliers and are eliminated.
+__device__ __forceinline__ void factor_group(TourneyShared &sh, int cb, int w) {
+    const int lane = opaque(threadIdx.x & 63);
+    float x[4][TG];
+    unsigned long long act[4];  // rows not yet chosen
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        act[r] = uniform(sh.act[r]);
+#pragma unroll
+        for (int q = 0; q < TG; q += 4) {
+            const float4 v = *reinterpret_cast<const float4 *>(&sh.tile[at(r * 64 + lane, cb + q)]);
+            x[r][q] = v.x; x[r][q + 1] = v.y; x[r][q + 2] = v.z; x[r][q + 3] = v.w;
+        }
+    }
+    int mine = -1;  // lane c: the tile row of pivot cb + c
+    // U12 = L11^-1 A12, one column per lane, a row behind the pivots: its entry
+    // of A and its multipliers, which each column leaves in the tile
+    const int rest = TW - TG - cb, col = min(cb + TG + lane, TW - 1);
+    float u12[TG], an = 0.f;
+    float4 ln[TG / 4] = {};
+    auto solve = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        u12[i] = an;
+#pragma unroll
+        for (int q = 0; q < i; ++q) {
+            const float l = q % 4 == 0 ? ln[q / 4].x : q % 4 == 1 ? ln[q / 4].y : q % 4 == 2 ? ln[q / 4].z : ln[q / 4].w;
+            u12[i] = fmaf(-l, u12[q], u12[i]);
+        }
+    };
+    float m[4] = {}, u[TG] = {};  // of the pivot before: its elimination is completed
+    unsigned key[4];              // while the next maximum is found
+#pragma unroll
+    for (int r = 0; r < 4; ++r) key[r] = bit_of(act[r], (__float_as_uint(x[r][0]) << 1) | 1u, 0u);
+    static_for<TG>([&](auto cc) __attribute__((always_inline)) {
+        constexpr int c = decltype(cc)::value;
+        constexpr int N = c > 0 ? 4 * (TG - 1 - c) : 0;  // multiply-adds left of the pivot before
+        auto eliminate = [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+#pragma unroll
+            for (int f = i * N / 6; f < (i + 1) * N / 6; ++f)
+                x[f % 4][c + 1 + f / 4] = fmaf(-m[f % 4], u[c + 1 + f / 4], x[f % 4][c + 1 + f / 4]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        const bool up0 = key[1] > key[0], up1 = key[3] > key[2];
+        const unsigned k0 = max(key[0], key[1]), k1 = max(key[2], key[3]);
+        const bool up = k1 > k0;
+        const unsigned kk = max(k0, k1);
+        unsigned d = dpp_max<DPP_SHR<1>>(kk);
+        eliminate(std::integral_constant<int, 0>{});
+        d = dpp_max<DPP_SHR<2>>(d);
+        eliminate(std::integral_constant<int, 1>{});
+        d = dpp_max<DPP_SHR<4>>(d);
+        eliminate(std::integral_constant<int, 2>{});
+        d = dpp_max<DPP_SHR<8>>(d);
+        eliminate(std::integral_constant<int, 3>{});
+        d = dpp_max<DPP_BCAST15>(d);
+        eliminate(std::integral_constant<int, 4>{});
+        d = dpp_max<DPP_BCAST31>(d);
+        eliminate(std::integral_constant<int, 5>{});
+        const unsigned mx = lane_get(d, 63);
+        const unsigned long long b0 = __ballot(up0), b1 = __ballot(up1), b2 = __ballot(up);
+        float y[TG];
+#pragma unroll
+        for (int e = c; e < TG; ++e) {
+            const float v0 = up0 ? x[1][e] : x[0][e], v1 = up1 ? x[3][e] : x[2][e];
+            y[e] = up ? v1 : v0;
+        }
+        const int l = __builtin_ctzll(__ballot(kk == mx));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = c; e < TG; ++e) u[e] = lane_get(y[e], l);
+        const unsigned long long one = 1ull << l;
+        act[0] &= ~(one & ~b2 & ~b0);
+        act[1] &= ~(one & ~b2 & b0);
+        act[2] &= ~(one & b2 & ~b1);
+        act[3] &= ~(one & b2 & b1);
+        const float rp = u[c] != 0.f ? __builtin_amdgcn_rcpf(u[c]) : 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            // a chosen row keeps its values: its multiplier is zero
+            m[r] = bit_of(act[r], x[r][c] * rp, 0.f);
+            if constexpr (c + 1 < TG) {
+                x[r][c + 1] = fmaf(-m[r], u[c + 1], x[r][c + 1]);
+                key[r] = bit_of(act[r], (__float_as_uint(x[r][c + 1]) << 1) | 1u, 0u);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (c > 0) solve(std::integral_constant<int, c - 1>{});
+        const int o = (int)((b2 >> l) & 1), in = (int)((o ? b1 >> l : b0 >> l) & 1);
+        const int t = (2 * o + in) * 64 + l;
+        mine = lane == c && mx != 0u ? t : mine;  // (0: no row was left)
+        an = sh.tile[at(t, col)];
+#pragma unroll
+        for (int q = 0; q < c; q += 4) ln[q / 4] = *reinterpret_cast<const float4 *>(&sh.tile[at(t, cb + q)]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            x[r][c] = bit_of(act[r], m[r], x[r][c]);
+            if constexpr (c + 1 < TG) sh.tile[at(r * 64 + lane, cb + c)] = x[r][c];
+        }
+    });
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int q = 0; q < TG; q += 4)
+            *reinterpret_cast<float4 *>(&sh.tile[at(r * 64 + lane, cb + q)]) =
+                make_float4(x[r][q], x[r][q + 1], x[r][q + 2], x[r][q + 3]);
+        if (lane == 0) sh.act[r] = act[r];
+    }
+    if (lane < TG) sh.slot[cb + lane] = cb + lane < w ? mine : -1;
+    solve(std::integral_constant<int, TG - 1>{});
+    if (lane < rest) {
+#pragma unroll
+        for (int i = 0; i < TG; ++i) {
+            sh.u[i][lane] = u12[i];
+            const int t = lane_get(mine, i);
+            if (i && t >= 0) sh.tile[at(t, col)] = u12[i];
+        }
+    }
+}
+
+// Partial pivoting on the 256 rows of the tile, 16 columns at a time: wave 0
+// factors them and solves the pivot rows' part right of them, then all waves
+// update the other rows on the matrix cores.  On return the row chosen at step j (sh.slot, sh.order) holds its
+// multipliers left of column j and its U row from column j on.
+//
+// Bound by the serial chain per column, about 130 instructions of one wave (a
+// lone wave issues one in 4.3 to 6 cycles).  One row per thread, with the search
+// and the pivot row going through LDS and a barrier per column, took 250 us for a
+// panel on average over a factorization of order 16384 (four levels at most,
+// beside the trailing update); this form takes 147, and a level on an idle device
+// 33.  Branching to the winner's row instead of setting the best entries aside
+// takes as long.
+__device__ void gepp256(TourneyShared &sh, int w) {
+    using Acc = Mfma<float>::acc;
+    const int wave = threadIdx.x >> 6;
+#pragma unroll 1
+    for (int cb = 0; cb < w; cb += TG) {
+        const int lane = opaque(threadIdx.x & 63), lr = lane & 15, lk = lane >> 4;
+        if (wave == 0) {
+            __builtin_amdgcn_s_setprio(3);  // ahead of another kernel's waves on this SIMD
+            factor_group(sh, cb, w);
+            __builtin_amdgcn_s_setprio(0);
+        }
+        __syncthreads();
+        if (cb + TG >= w) break;
+        // this wave's 64 rows: A22 -= L21 U12, the sums of 16 products kept
+        // apart; chosen rows keep their values (their multipliers count as zero)
+        float af[4][4];
+        const unsigned long long act = sh.act[wave];
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const float v = sh.tile[at(wave * 64 + rt * 16 + lr, cb + 4 * s + lk)];
+                af[rt][s] = (act >> (rt * 16 + lr)) & 1ull ? v : 0.f;
+            }
+#pragma unroll 1
+        for (int ct = cb + TG; ct < TW; ct += 16) {
+            float bf[4], cv[4][4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) bf[s] = sh.u[4 * s + lk][ct - cb - TG + lr];
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) cv[rt][r] = sh.tile[at(wave * 64 + rt * 16 + Mfma<float>::row(lk, r), ct + lr)];
+            Acc acc[4] = {};
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int rt = 0; rt < 4; ++rt) acc[rt] = Mfma<float>::op(af[rt][s], bf[s], acc[rt]);
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    sh.tile[at(wave * 64 + rt * 16 + Mfma<float>::row(lk, r), ct + lr)] = cv[rt][r] - acc[rt][r];
+        }
+        __syncthreads();
+    }
+    const int tid = threadIdx.x;
+    if (tid < TW) {
+        const int t = sh.slot[tid];
+        sh.order[tid] = t >= 0 ? sh.id[t] : -1;
+    }
+    __syncthreads();
 }
 
 // In-place inverses of two lower-triangular 64 x 64 matrices, M0 with a unit
-// diagonal and M1 with its own (the upper parts are zero and stay zero).
-// Each is split in 32 x 32 halves: the two diagonal halves of M0 are
-// inverted by waves 0 and 1 and those of M1 by waves 2 and 3, side by side,
-// lane j forward-substituting column j of the identity with the column in
-// registers; the corners are X21 = -X22 (M21 X11), two 32 x 32 products on
-// the matrix cores per matrix, one 16 x 16 tile per wave.  `tmp` is scratch.
-// Called by the whole workgroup.
+// diagonal and M1 with its own (the upper parts are zero and stay zero).  The
+// eight 16 x 16 diagonal blocks first, two per wave, a lane forward-substituting
+// one column of the identity in registers; then the blocks below them,
+// X21 = -X22 (M21 X11), by halves of 16 and of 32 on the matrix cores.  `tmp` is
+// scratch.  Called by the whole workgroup.
+//
+// Bound by the substitutions' chains: 32 x 32 blocks took 15,500 cycles, these
+// take 8,400.
 __device__ void inv_lower64_pair(float (*M0)[TW + 1], float (*M1)[TW + 1], float (*tmp)[32][33]) {
     using Acc = Mfma<float>::acc;
-    constexpr int H = TW / 2;
+    constexpr int B = 16;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 15, lk = lane >> 4;
-    if (lane < H) {
-        float (*M)[TW + 1] = wave < 2 ? M0 : M1;
+    float (*const Mw)[TW + 1] = wave < 2 ? M0 : M1;
+    if (lane < 2 * B) {
         const bool unit = wave < 2;
-        const int o = (wave & 1) * H, j = lane;
-        float x[H];
+        const int o = ((wave & 1) * 2 + (lane >> 4)) * B, j = lane & 15;
+        float x[B];
 #pragma unroll
-        for (int i = 0; i < H; ++i) {
+        for (int i = 0; i < B; ++i) {
             float s = (i == j) ? 1.f : 0.f;
 #pragma unroll
-            for (int q = 0; q < i; ++q) s -= M[o + i][o + q] * x[q];
-            x[i] = unit ? s : s / M[o + i][o + i];
+            for (int q = 0; q < i; ++q) s -= Mw[o + i][o + q] * x[q];
+            x[i] = unit ? s : s / Mw[o + i][o + i];
         }
-        // every read of the half precedes the wave's writes to it
+        // every read of the block precedes the wave's writes to it
 #pragma unroll
-        for (int i = 0; i < H; ++i) M[o + i][o + j] = x[i];
+        for (int i = 0; i < B; ++i) Mw[o + i][o + j] = x[i];
     }
     __syncthreads();
+    {   // the 32 x 32 half at o of this wave's matrix
+        const int o = (wave & 1) * 2 * B;
+        Acc acc = Acc{0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < B / 4; ++s)
+            acc = Mfma<float>::op(Mw[o + B + lr][o + 4 * s + lk], Mw[o + 4 * s + lk][o + lr], acc);
+        float (*const t)[33] = &tmp[wave >> 1][(wave & 1) * B];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t[Mfma<float>::row(lk, r)][lr] = acc[r];
+        __syncthreads();
+        acc = Acc{0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < B / 4; ++s)
+            acc = Mfma<float>::op(Mw[o + B + lr][o + B + 4 * s + lk], t[4 * s + lk][lr], acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Mw[o + B + Mfma<float>::row(lk, r)][o + lr] = -acc[r];
+    }
+    __syncthreads();
+    constexpr int H = TW / 2;
     const int tr = (wave >> 1) * 16, tc = (wave & 1) * 16;
 #pragma unroll
     for (int q = 0; q < 2; ++q) {   // tmp = M21 X11
@@ -226,39 +422,28 @@ __device__ void inv_lower64_pair(float (*M0)[TW + 1], float (*M1)[TW + 1], float
     __syncthreads();
 }
 
-// Shared memory of the tournament kernel: the partial-pivoting state, and for
-// the root the pivot block and the two triangles being inverted.
-struct TourneyShared {
-    GeppShared g;
-    float F[TW][TW + 1];
-    float L[TW][TW + 1];   // L11, then L11^-1
-    float Ut[TW][TW + 1];  // U11^T, then (U11^-1)^T
-    float tmp[2][32][33];
-    int slot_sel[TW];      // top slot q -> pivot index whose row starts there (-1)
-    int vrow[TW], vsel[TW];
-    int s_last;
-};
-
-__global__ __launch_bounds__(TLR) void k_tslu_tourney(const float *__restrict__ A, long lda, int k, int m,
+__global__ __launch_bounds__(TLR) __attribute__((amdgpu_waves_per_eu(2))) void k_tslu_tourney(const float *__restrict__ A, long lda, int k, int m,
                                                       int w, int64_t *__restrict__ ipiv,
                                                       int64_t *__restrict__ info, int n,
                                                       float *__restrict__ linv, TsluWork tw, int vec) {
-    __shared__ TourneyShared sh;
+    __shared__ __attribute__((aligned(16))) TourneyShared sh;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int L = gridDim.x;
-    float a[TW];
-    int step = -1;
-
-    // ---- leaf
     const int r0 = blockIdx.x * TLR;
-    int id = r0 + tid < m ? k + r0 + tid : -1;
-    load_row(a, A, lda, k, id, w, vec != 0);
-    gepp256(a, id, w, sh.g, step);
-    int level_off = 0, level_n = L, node = blockIdx.x;
-    if (tid < TW) tw.cand[(level_off + node) * TW + tid] = sh.g.order[tid];
+    int id = r0 + tid < m ? k + r0 + tid : -1;  // the leaf's rows
+    int level_off = 0, level_n = gridDim.x, node = blockIdx.x;
+    for (;;) {
+        sh.id[tid] = id;
+        const unsigned long long have = __ballot(id >= 0);
+        if (lane == 0) sh.act[wave] = have;
+        if (tid < TW) sh.slot[tid] = -1;
+        __syncthreads();
+        load_rows(sh, A, lda, k, w, vec != 0);
+        __syncthreads();
+        gepp256(sh, w);
+        if (level_n == 1) break;
+        if (tid < TW) tw.cand[(level_off + node) * TW + tid] = sh.order[tid];
 
-    // ---- merges: the workgroup completing a node's last child merges it
-    while (level_n > 1) {
+        // ---- the workgroup completing a node's last child merges it
         const int parent = node / TF;
         const int next_off = level_off + level_n, next_n = (level_n + TF - 1) / TF;
         const int kids = min(TF, level_n - parent * TF);
@@ -277,33 +462,30 @@ __global__ __launch_bounds__(TLR) void k_tslu_tourney(const float *__restrict__ 
         id = tid / TW < kids ? __hip_atomic_load(&tw.cand[(level_off + child) * TW + (tid % TW)],
                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                              : -1;
-        load_row(a, A, lda, k, id, w, vec != 0);
-        gepp256(a, id, w, sh.g, step);
         level_off = next_off;
         level_n = next_n;
         node = parent;
-        if (level_n > 1 && tid < TW) tw.cand[(level_off + node) * TW + tid] = sh.g.order[tid];
     }
 
     // ---- root: the pivot block, its inverses, the swaps
-    if (step >= 0) {
+    {
+        constexpr int PER = TW * TW / TLR;
+        float f[PER];
 #pragma unroll
-        for (int c = 0; c < TW; ++c) sh.F[step][c] = a[c];
-    }
-    if (tid < TW) {
-        sh.slot_sel[tid] = -1;
-        if (tid >= w)
+        for (int q = 0; q < PER; ++q) {
+            const int r = q * 4 + wave, t = sh.slot[r];
+            f[q] = t >= 0 ? sh.tile[at(t, lane)] : (r == lane && r >= w ? 1.f : 0.f);
+        }
+        __syncthreads();  // the tile has been read
+        // L11 (unit lower) and U11^T, zero-padded to 64 x 64 with unit diagonal
 #pragma unroll
-            for (int c = 0; c < TW; ++c) sh.F[tid][c] = (c == tid) ? 1.f : 0.f;
-    }
-    __syncthreads();
-    // L11 (unit lower) and U11^T, zero-padded to 64 x 64 with unit diagonal
-    for (int e = tid; e < TW * TW; e += TLR) {
-        const int r = e / TW, c = e % TW;
-        const float f = sh.F[r][c];
-        sh.L[r][c] = c < r ? (r < w && c < w ? f : 0.f) : 0.f;
-        sh.Ut[c][r] = c >= r ? (r < w && c < w ? f : (r == c ? 1.f : 0.f)) : 0.f;
-        tw.F[e] = f;
+        for (int q = 0; q < PER; ++q) {
+            const int r = q * 4 + wave, c = lane;
+            sh.F[r][c] = f[q];
+            sh.L[r][c] = c < r ? (r < w && c < w ? f[q] : 0.f) : 0.f;
+            sh.Ut[c][r] = c >= r ? (r < w && c < w ? f[q] : (r == c ? 1.f : 0.f)) : 0.f;
+            tw.F[r * TW + c] = f[q];
+        }
     }
     __syncthreads();
     inv_lower64_pair(sh.L, sh.Ut, sh.tmp);
@@ -314,62 +496,51 @@ __global__ __launch_bounds__(TLR) void k_tslu_tourney(const float *__restrict__ 
         tw.Uinv[e] = in && c >= r ? sh.Ut[c][r] : 0.f;
     }
     if (wave == 0) {
-        // pivot j's row: in the top slot q = row - k when it starts in
-        // k .. k+w-1, else in the next free "outside" slot (half 1)
-        const int selj = lane < w ? sh.g.order[lane] : -1;
-        if (lane < w) tw.sel[lane] = selj;
-        const bool top = selj >= k && selj < k + w;
-        if (lane < w && top) sh.slot_sel[selj - k] = lane;
-        // (a pivot without a row cannot occur when m >= w; it would leave
-        // its step without a swap, and info reports it)
-        const bool out = lane < w && selj >= 0 && !top;
-        const unsigned long long bo = __ballot(out);
-        const int rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bo >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo((unsigned)bo, 0));
-        if (out) { sh.vrow[rank] = selj; sh.vsel[rank] = lane; }
-        const int nout = __popcll(bo);
-        __builtin_amdgcn_wave_barrier();
+        // The reference's sequential swaps: step j exchanges position k + j with
+        // the position that holds pivot j's row now, to(j).  A row outside the top
+        // w positions stays until it is chosen; one at top position q < j has gone
+        // to to(q) by step j, and on from there if that is a top position below j.
+        // Step j moves what position k + j holds then: what the last earlier step
+        // that named that position brought there, or row k + j.
+        const bool has = lane < w;
+        const int selj = has ? sh.order[lane] : -1;
+        if (has) tw.sel[lane] = selj;
+        // (a pivot without a row cannot occur when m >= w; it would leave its
+        // step without a swap, and info reports it)
+        int to = selj < 0 ? k + lane : selj;
+        for (unsigned long long open; (open = __ballot(has && to < k + lane)) != 0;) {
+            const int q = max(to - k, 0) & 63;
+            const int next = __builtin_amdgcn_ds_bpermute(q * 4, to);
+            if (((open >> lane) & 1ull) && !((open >> q) & 1ull)) to = next;
+        }
+        sh.slot[lane] = -1;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-        // slot (lane, half 0) = position k + lane; (lane, half 1) = position vrow[lane]
-        int pos0 = k + lane, con0 = k + lane, sx0 = lane < w ? sh.slot_sel[lane] : -1;
-        int pos1 = lane < nout ? sh.vrow[lane] : -1, con1 = pos1, sx1 = lane < nout ? sh.vsel[lane] : -1;
-        // the reference's sequential swaps: step j exchanges position k + j
-        // with the position that holds pivot j's row now
-        for (int j = 0; j < w; ++j) {
-            const unsigned long long b0 = __ballot(sx0 == j), b1 = __ballot(sx1 == j);
-            if (!b0 && !b1) {
-                if (lane == 0) ipiv[k + j] = k + j;
-                continue;
-            }
-            const int H = b0 ? 0 : 1;
-            const int Ln = __ffsll((long long)(b0 ? b0 : b1)) - 1;
-            const int psl = __builtin_amdgcn_readlane(H ? pos1 : pos0, Ln);
-            const int csl = __builtin_amdgcn_readlane(H ? con1 : con0, Ln);
-            const int ctop = __builtin_amdgcn_readlane(con0, j), xtop = __builtin_amdgcn_readlane(sx0, j);
-            if (lane == 0) ipiv[k + j] = psl;
-            if (!(H == 0 && Ln == j)) {
-                if (lane == j) { con0 = csl; sx0 = j; }
-                if (lane == Ln) {
-                    if (H) { con1 = ctop; sx1 = xtop; }
-                    else { con0 = ctop; sx0 = xtop; }
-                }
-            }
+        if (has && to > k + lane && to < k + w) atomicMax(&sh.slot[to - k], lane);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        int held = lane;  // the top row that position k + lane holds at step `lane`
+        const int before = sh.slot[lane];
+        for (int go = before; __ballot(go >= 0) != 0;) {
+            held = go >= 0 ? go : held;
+            const int next = __builtin_amdgcn_ds_bpermute(held * 4, before);
+            go = go >= 0 ? next : -1;
         }
+        if (has) ipiv[k + lane] = to;
+        // a top row that is a pivot itself does not stay where it was moved to
+        sh.slot[lane] = 0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        if (selj >= k && selj < k + w) sh.slot[selj - k] = 1;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        const int from = has && to >= k + w && !sh.slot[held] ? k + held : -1;
         // rows that end outside the top: the displaced rows
-        const bool mv = lane < nout && con1 != pos1;
+        const bool mv = from >= 0;
         const unsigned long long bm = __ballot(mv);
-        const int at = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bm >> 32),
-                                                      __builtin_amdgcn_mbcnt_lo((unsigned)bm, 0));
-        if (mv) { tw.map[1 + 2 * at] = con1; tw.map[2 + 2 * at] = pos1; }
-        if (lane == 0) {
-            tw.map[0] = __popcll(bm);
-            if (*info == (int64_t)n) {
-                for (int j = 0; j < w; ++j) {
-                    const float d = sh.F[j][j];
-                    if (sh.g.order[j] < 0 || !(fabsf(d) >= 1.1920929e-7f)) { *info = k + j; break; }
-                }
-            }
-        }
+        const int ord = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bm >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo((unsigned)bm, 0));
+        if (mv) { tw.map[1 + 2 * ord] = from; tw.map[2 + 2 * ord] = to; }
+        if (lane == 0) tw.map[0] = __popcll(bm);
+        const bool bad = lane < w && (selj < 0 || !(fabsf(sh.F[lane][lane]) >= 1.1920929e-7f));
+        const unsigned long long first = __ballot(bad);
+        if (lane == 0 && first && *info == (int64_t)n) *info = k + __builtin_ctzll(first);
     }
 }
 

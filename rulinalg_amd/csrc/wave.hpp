@@ -42,6 +42,10 @@ constexpr int DPP_XOR2 = 0x4E;         // quad_perm [2, 3, 0, 1]
 constexpr int DPP_HALF_MIRROR = 0x141; // lane i <-> 7 - i within each 8
 constexpr int DPP_MIRROR = 0x140;      // lane i <-> 15 - i within each 16
 
+template <int N> constexpr int DPP_SHR = 0x110 + N;  // lane i <- lane i - N within each 16
+constexpr int DPP_BCAST15 = 0x142;     // a row's lane 15 -> the next row
+constexpr int DPP_BCAST31 = 0x143;     // lane 31 -> lanes 32..63
+
 template <int CTRL> __device__ __forceinline__ int dpp(int x) {
     return __builtin_amdgcn_update_dpp(x, x, CTRL, 0xF, 0xF, false);
 }
