@@ -714,82 +714,6 @@ __global__ __launch_bounds__(SWB) void k_laswp(T *__restrict__ A, long lda, cons
 // product instead of a 64-step dependent sweep.  L has a unit diagonal and,
 // under partial pivoting, entries of magnitude at most 1.
 
-// Row-major 64 x 64 inv = L^-1, zero outside jb x jb, by halves: with L = [L11 0; L21 L22] in 32 x 32 blocks,
-// L^-1 = [X11 0; -X22 L21 X11, X22], X11 = L11^-1 and X22 = L22^-1.  Waves 0
-// and 1 invert the two diagonal halves side by side, lane j forward-
-// substituting column j of the identity with the column in registers and L
-// from LDS as broadcasts; the corner is then two 32 x 32 matrix-core
-// products, one 16 x 16 tile per wave.  The rows and columns past jb stage
-// as zeros, so they invert to the identity and are masked on the way out.
-template <class T>
-__global__ __launch_bounds__(256) void k_tri_inv(const T *__restrict__ A, long lda, int j0, int jb,
-                                                 T *__restrict__ inv) {
-    using Acc = typename Mfma<T>::acc;
-    constexpr int H = PNB / 2;
-    __shared__ T L[PNB][PNB + 1];  // L, overwritten by L^-1 block by block
-    __shared__ T Tm[H][H + 1];     // L21 X11
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lr = lane & 15, lk = lane >> 4;
-    {
-        constexpr int PER = PNB * PNB / 256;
-        T v[PER];
-#pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const int e = q * 256 + tid, r = e >> 6, c = e & 63;
-            v[q] = (r < jb && c < jb) ? A[(long)(j0 + r) * lda + j0 + c] : T(0);
-        }
-#pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const int e = q * 256 + tid, r = e >> 6, c = e & 63;
-            L[r][c] = v[q];
-        }
-    }
-    __syncthreads();
-    if (wave < 2 && lane < H) {
-        // X11 (wave 0) or X22 (wave 1): every read of the block precedes the
-        // wave's writes to it, and the two blocks do not overlap
-        const int o = wave * H, j = lane;
-        T x[H];
-#pragma unroll
-        for (int i = 0; i < H; ++i) {
-            T s = (i == j) ? T(1) : T(0);
-#pragma unroll
-            for (int q = 0; q < i; ++q) s -= L[o + i][o + q] * x[q];
-            x[i] = s;
-        }
-#pragma unroll
-        for (int i = 0; i < H; ++i) L[o + i][o + j] = x[i];  // zero above the diagonal
-    }
-    __syncthreads();
-    const int tr = (wave >> 1) * 16, tc = (wave & 1) * 16;  // this wave's 16 x 16 tile
-    {   // Tm = L21 X11
-        Acc acc = Acc{0, 0, 0, 0};
-#pragma unroll
-        for (int s = 0; s < H / 4; ++s)
-            acc = Mfma<T>::op(L[H + tr + lr][4 * s + lk], L[4 * s + lk][tc + lr], acc);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) Tm[tr + Mfma<T>::row(lk, r)][tc + lr] = acc[r];
-    }
-    __syncthreads();
-    {   // X21 = -X22 Tm, over L21 (no longer read)
-        Acc acc = Acc{0, 0, 0, 0};
-#pragma unroll
-        for (int s = 0; s < H / 4; ++s)
-            acc = Mfma<T>::op(L[H + tr + lr][H + 4 * s + lk], Tm[4 * s + lk][tc + lr], acc);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) L[H + tr + Mfma<T>::row(lk, r)][tc + lr] = -acc[r];
-    }
-    __syncthreads();
-    {
-        constexpr int PER = PNB * PNB / 256;
-#pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const int e = q * 256 + tid, i = e >> 6, c = e & 63;
-            inv[e] = (i < jb && c < jb && c <= i) ? L[i][c] : T(0);
-        }
-    }
-}
-
 // B := inv * B for one 64-column slab per workgroup, in place: the slab is
 // read whole into LDS before any of it is written.  Wave w computes rows
 // [16 w, 16 w + 16) of the slab as four 16 x 16 accumulators over 16 k-steps.
@@ -842,6 +766,182 @@ __global__ __launch_bounds__(256) void k_trsm_llu(T *__restrict__ A, long lda, i
 
 // Set by lu_factor_lowp for its duration: FP32 panels are then factored with
 // tournament pivoting (tslu.hip) in this workspace.
+// The step between an inner panel and its update, for the other columns of the
+// outer block: the panel's swaps on columns [c0, c1) and [c2, c3), the inverse of
+// its unit-lower block, and the block-row solve B := L^-1 B on the swapped rows
+// of [c2, c3).  A workgroup owns 32 columns on one side (at least one workgroup
+// has the right side, if that inverse is needed): it reads every row its columns
+// move, then writes them.  Wave 0 derives the row moves while wave 1 inverts the
+// diagonal blocks; every workgroup on the right forms the whole inverse, and the
+// first stores it for the outer block row (have_inv: it is there already).
+//
+// Bound by latencies: four dependent trips to memory and about 4,000 cycles of
+// inversion and product.  It takes 13.4 us at order 16384 in FP64 (14.7 at 1531,
+// unaligned), where three launches, for the inverse, the swaps and the solve,
+// took 8.5, 13.6 and 8.
+//
+// L^-1 in blocks: the diagonal ones of IB x IB by forward substitution, a lane
+// per column, then X21 = -X22 (L21 X11) by doubling sizes on the matrix cores.
+// IB is 16 in FP64 (a shorter chain) and 32 in FP32, which keeps the values that
+// the low-precision factorizations were tested with.
+template <class T> struct InvBlock { static constexpr int value = 16; };
+template <> struct InvBlock<float> { static constexpr int value = 32; };
+constexpr int RCOLS = 32;  // columns per workgroup
+template <class T>
+__global__ __launch_bounds__(256) void k_row_step(T *__restrict__ A, long lda, const int64_t *__restrict__ ipiv,
+                                                  int j0, int jb, int c0, int c1, int c2, int c3, T *inv,
+                                                  int have_inv) {
+    using Acc = typename Mfma<T>::acc;
+    constexpr int IB = InvBlock<T>::value, LD = PNB + TilePad<T>::value;
+    __shared__ __attribute__((aligned(16))) T L[PNB][LD];  // L, overwritten by L^-1 block by block
+    __shared__ T Tm[PNB / 2][PNB / 2 + 1];                 // L21 X11
+    __shared__ T X[PNB][RCOLS + 1];
+    __shared__ int P[PNB], src_in[PNB], dst_out[PNB], src_out[PNB], s_out;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int left = (c1 - c0 + RCOLS - 1) / RCOLS;
+    const bool right = (int)blockIdx.x >= left;
+    const int cb = right ? c2 + ((int)blockIdx.x - left) * RCOLS : c0 + (int)blockIdx.x * RCOLS;
+    const int ce = min(cb + RCOLS, right ? c3 : c1);
+
+    if (tid < jb) P[tid] = (int)ipiv[j0 + tid];
+    if (right) {
+        constexpr int PER = PNB * PNB / 256;
+        T v[PER];
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int r = q * 4 + wave, c = lane;
+            v[q] = have_inv ? inv[r * PNB + c] : (r < jb && c < r) ? A[(long)(j0 + r) * lda + j0 + c] : T(0);
+        }
+#pragma unroll
+        for (int q = 0; q < PER; ++q) L[q * 4 + wave][lane] = v[q];
+    }
+    __syncthreads();
+    if (wave == 0) {
+        // the final content of row j0 + lane, and of the row that swap `lane`
+        // is the last to touch beyond the block
+        int so = -1, pt = -1;
+        bool mv = false;
+        if (lane < jb) {
+            pt = P[lane];
+            src_in[lane] = swap_chase(P, j0, pt, lane);
+            if (pt >= j0 + jb && swap_last(P, pt, lane, jb)) {
+                so = swap_chase(P, j0, j0 + lane, lane);
+                mv = so != pt;
+            }
+        }
+        const unsigned long long b = __ballot(mv);
+        if (mv) {
+            const int at = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b, 0));
+            dst_out[at] = pt;
+            src_out[at] = so;
+        }
+        if (lane == 0) s_out = __popcll(b);
+    } else if (wave == 1 && right && !have_inv) {
+        // every read of a block precedes the wave's writes to it
+        const int o = lane / IB * IB, j = lane % IB;
+        T x[IB];
+#pragma unroll
+        for (int i = 0; i < IB; ++i) {
+            T s = (i == j) ? T(1) : T(0);
+#pragma unroll
+            for (int q = 0; q < i; ++q) s -= L[o + i][o + q] * x[q];
+            x[i] = s;
+        }
+#pragma unroll
+        for (int i = 0; i < IB; ++i) L[o + i][o + j] = x[i];  // zero above the diagonal
+    }
+    __syncthreads();
+
+    // the rows: element (q * 8 + tid / 32, tid % 32) of the block's and of the others
+    constexpr int RG = 256 / RCOLS, PER = PNB / RG;
+    const int rg = tid / RCOLS, cl = tid % RCOLS, col = cb + cl;
+    const int outs = s_out;
+    T vi[PER], vo[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int i = q * RG + rg;
+        vi[q] = i < jb && col < ce ? A[(long)src_in[i] * lda + col] : T(0);
+        vo[q] = i < outs && col < ce ? A[(long)src_out[i] * lda + col] : T(0);
+    }
+    if (right && !have_inv) {
+        if constexpr (IB == 16) {
+            const int o = wave * 32;
+            const bool on = wave < 2;
+            if (on) {
+                Acc acc = Acc{0, 0, 0, 0};
+#pragma unroll
+                for (int s = 0; s < 4; ++s) acc = Mfma<T>::op(L[o + 16 + lr][o + 4 * s + lk], L[o + 4 * s + lk][o + lr], acc);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) Tm[16 * wave + Mfma<T>::row(lk, r)][lr] = acc[r];
+            }
+            __syncthreads();
+            if (on) {
+                Acc acc = Acc{0, 0, 0, 0};
+#pragma unroll
+                for (int s = 0; s < 4; ++s) acc = Mfma<T>::op(L[o + 16 + lr][o + 16 + 4 * s + lk], Tm[16 * wave + 4 * s + lk][lr], acc);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) L[o + 16 + Mfma<T>::row(lk, r)][o + lr] = -acc[r];
+            }
+            __syncthreads();
+        }
+        constexpr int H = PNB / 2;
+        const int tr = (wave >> 1) * 16, tc = (wave & 1) * 16;  // this wave's 16 x 16 tile
+        {   // Tm = L21 X11
+            Acc acc = Acc{0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < H / 4; ++s) acc = Mfma<T>::op(L[H + tr + lr][4 * s + lk], L[4 * s + lk][tc + lr], acc);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) Tm[tr + Mfma<T>::row(lk, r)][tc + lr] = acc[r];
+        }
+        __syncthreads();
+        {   // X21 = -X22 Tm, over L21 (no longer read)
+            Acc acc = Acc{0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < H / 4; ++s)
+                acc = Mfma<T>::op(L[H + tr + lr][H + 4 * s + lk], Tm[4 * s + lk][tc + lr], acc);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) L[H + tr + Mfma<T>::row(lk, r)][tc + lr] = -acc[r];
+        }
+        __syncthreads();
+        // the rows and columns past jb were staged as zeros: they inverted to the
+        // identity, and become zeros again
+#pragma unroll
+        for (int q = 0; q < PNB * PNB / 256; ++q) {
+            const int i = q * 4 + wave, c = lane;
+            const T v = i < jb && c < jb && c <= i ? L[i][c] : T(0);
+            L[i][c] = v;
+            if ((int)blockIdx.x == left) inv[i * PNB + c] = v;
+        }
+    }
+    if (right) {
+#pragma unroll
+        for (int q = 0; q < PER; ++q) X[q * RG + rg][cl] = vi[q];
+    }
+    __syncthreads();  // every row has been read
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int i = q * RG + rg;
+        if (!right && i < jb && col < ce && src_in[i] != j0 + i) A[(long)(j0 + i) * lda + col] = vi[q];
+        if (i < outs && col < ce) A[(long)dst_out[i] * lda + col] = vo[q];
+    }
+    if (!right) return;
+    // wave w: rows [16 w, 16 w + 16) of L^-1 B as two 16 x 16 tiles
+    Acc acc[2] = {};
+#pragma unroll
+    for (int s = 0; s < PNB / 4; ++s)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+            acc[t] = Mfma<T>::op(L[16 * wave + lr][4 * s + lk], X[4 * s + lk][16 * t + lr], acc[t]);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * wave + Mfma<T>::row(lk, r), c = cb + 16 * t + lr;
+            if (row < jb && c < ce) A[(long)(j0 + row) * lda + c] = acc[t][r];
+        }
+}
+
 static thread_local void *g_tslu_work = nullptr;
 
 template <class T>
@@ -949,12 +1049,17 @@ static T *linv_of(const LuWork &lw, size_t j0) {
 }
 
 template <class T>
-static int tri_inv(hipStream_t s, const T *a, size_t lda, size_t j0, size_t jb, const LuWork &lw) {
-    if (jb <= 1) return RLG_OK;
-    // algorithmic bytes: the unit-lower block read, the 64 x 64 inverse written
-    RLG_PROF_W("tri_inv", s, ((double)jb * jb / 2 + (double)PNB * PNB) * sizeof(T));
-    hipLaunchKernelGGL(k_tri_inv<T>, dim3(1), dim3(256), 0, s, a, (long)lda, (int)j0, (int)jb,
-                       linv_of<T>(lw, j0));
+static int row_step(hipStream_t s, T *a, size_t lda, const int64_t *ipiv, size_t n, size_t j0, size_t jb, size_t c0,
+                    size_t c3, const LuWork &lw, bool have_inv) {
+    const size_t left = ceil_div(j0 - c0, RCOLS), right = ceil_div(c3 - j0 - jb, RCOLS);
+    // the last panel's inverse has no use; others' serve the outer block row too
+    const size_t blocks = left + (right || j0 + jb == n || have_inv ? right : 1);
+    if (blocks == 0) return RLG_OK;
+    // algorithmic bytes: at most 2 jb rows of these columns read and written, the
+    // block read and its inverse written
+    RLG_PROF_W("row_step", s, (4.0 * (double)jb * (double)(c3 - c0 - jb) + 2.0 * PNB * PNB) * sizeof(T));
+    hipLaunchKernelGGL(k_row_step<T>, dim3((unsigned)blocks), dim3(256), 0, s, a, (long)lda, ipiv, (int)j0, (int)jb,
+                       (int)c0, (int)j0, (int)(j0 + jb), (int)c3, linv_of<T>(lw, j0), (int)have_inv);
     RLG_LAUNCHED();
     return RLG_OK;
 }
@@ -1030,12 +1135,9 @@ static int outer_panel(hipStream_t s, size_t n, T *a, size_t lda, int64_t *ipiv,
         const size_t jb = k0 + kb - j0 < (size_t)PNB ? k0 + kb - j0 : PNB;
         bool linv_done = false;
         RLG_TRY(panel_any<T>(s, a, lda, j0, n - j0, jb, ipiv, info, n, lw, &linv_done));
-        // L^-1 of the panel's diagonal block, for its two block-row solves
-        if (j0 + jb < n && !linv_done) RLG_TRY(tri_inv<T>(s, a, lda, j0, jb, lw));
-        // inner swaps on the other columns of the outer block
-        RLG_TRY(laswp<T>(s, a, lda, ipiv, j0, jb, k0, j0, j0 + jb, k0 + kb));
+        // swaps and block-row solve on the other columns of the outer block
+        RLG_TRY(row_step<T>(s, a, lda, ipiv, n, j0, jb, k0, k0 + kb, lw, linv_done));
         if (j0 + jb < k0 + kb) {
-            RLG_TRY(trsm_llu<T>(s, a, lda, j0, jb, j0 + jb, k0 + kb, lw));
             RLG_TRY(update_native<T>(s, n - j0 - jb, k0 + kb - j0 - jb, jb, a + (j0 + jb) * lda + j0,
                                      lda, a + j0 * lda + j0 + jb, lda, a + (j0 + jb) * lda + j0 + jb,
                                      lda));
