@@ -44,6 +44,15 @@
 
 namespace rlg {
 
+// The value again, unknown to the compiler: addresses made from it are formed
+// where they are used, not ahead of a loop and kept in scratch memory.
+__device__ __forceinline__ int opaque(int v) {
+#ifdef __AMDGCN__
+    asm volatile("" : "+v"(v));
+#endif
+    return v;
+}
+
 constexpr int BTH = 256;
 constexpr int BMAXN = RLG_BATCH_MAX_N;
 constexpr int PANEL = 8704;       // doubles: 512 x 17
@@ -78,12 +87,13 @@ struct Smem {
     int red_i[BTH / 64];
     int piv[32];
     double div[32];
-    // LU column step j (buffers by the parity of j): each wave's pivot
-    // candidate (|value|, row, the whole row) and row j of the panel
-    double cand_v[2][BTH / 64];
-    int cand_i[2][BTH / 64];
+    // LU column step j (buffers by the parity of j): each wave's pivot candidate,
+    // the ranks of its |value| (rank_hi, rank_lo; 0: none), its position and panel
+    // row, and that row from column j on
+    unsigned cand_hi[2][BTH / 64], cand_lo[2][BTH / 64];
+    int cand_p[2][BTH / 64], cand_t[2][BTH / 64];
     double cand[2][BTH / 64][32];
-    double jrow[2][32];
+    alignas(16) double l11[32 * 32];  // L11 of the panel by columns, for the block row
     int mdst[64], msrc[64];     // net row moves of a panel's swaps
     int mcnt;
     int info;
@@ -91,9 +101,8 @@ struct Smem {
 };
 
 constexpr int BNW = BTH / 64;  // waves per workgroup
-constexpr int TSTRIP = 4;      // 16 x 16 tiles per wave step of the Cholesky SYRK update
-constexpr int TSTRIP_LU = 8;   // and of the LU trailing update (measured 15 % faster than 4;
-                               // the SYRK's strips end at the diagonal, where 8 wastes tiles)
+constexpr int TSTRIP = 8;      // 16 x 16 tiles per wave step of the Cholesky SYRK update
+constexpr int TSTRIP_LU = 8;   // and of the LU trailing update
 
 // Copy the m x kb block at A[k.., k..] (ld n) into the LDS panel P (ld LD), or
 // back (TO_A); eight loads in flight per thread before their stores.  With
@@ -129,7 +138,8 @@ __device__ __forceinline__ void panel_move(T *__restrict__ A, int n, int k, int 
 // just before it; a row x beyond the block is final after the last swap that
 // names it, and then holds what row s held just before swap s.  "What row x
 // held before swap t" is found by scanning the earlier swaps downwards.
-// Called by every thread; wave 0 (kb <= 32 lanes) fills sm.mdst / sm.msrc.
+// Called by every thread; wave 0 (kb <= 32 lanes) fills sm.mdst / sm.msrc, which
+// hold room for 64 moves.
 __device__ __forceinline__ int bchase(const int *piv, int x, int t) {
     for (int s = t - 1; s >= 0; --s)
         if (piv[s] == x) x = s;
@@ -155,7 +165,13 @@ __device__ __forceinline__ void panel_moves(int kb, const int *piv, int *mdst, i
         const int below_o = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(b_out >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b_out, 0));
         if (d_in >= 0) { mdst[below] = d_in; msrc[below] = s_in; }
         if (d_out >= 0) { mdst[n_in + below_o] = d_out; msrc[n_in + below_o] = s_out; }
-        if (t == 0) *mcnt = n_in + __popcll(b_out);
+        // the list padded to whole groups of 8 with its last move
+        const int cnt = n_in + __popcll(b_out);
+        const unsigned long long last = b_out ? b_out : b_in;
+        const int ll = last ? 63 - __builtin_clzll(last) : 0;
+        const int d_last = lane_get(b_out ? d_out : d_in, ll), s_last = lane_get(b_out ? s_out : s_in, ll);
+        if (cnt && t >= cnt && t < ((cnt + 7) & ~7)) { mdst[t] = d_last; msrc[t] = s_last; }
+        if (t == 0) *mcnt = cnt;
     }
 }
 
@@ -166,109 +182,125 @@ __device__ __forceinline__ void panel_moves(int kb, const int *piv, int *mdst, i
 // B holds L^-1 P B.  Pivots go to piv_out[0..n).  Returns the first failing
 // step or n.
 template <class T, int NB>
-__device__ int lu_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs,
+__device__ __attribute__((noinline)) int lu_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs,
                         int64_t *__restrict__ piv_out, Smem &sm) {
     T *P = reinterpret_cast<T *>(sm.panel);
     constexpr int LD = NB + 1;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) sm.info = n;
+    // (arguments of a called function count as different in every lane: the
+    // branches on them would be masks)
+    n = __builtin_amdgcn_readfirstlane(n);
+    nrhs = __builtin_amdgcn_readfirstlane(nrhs);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (threadIdx.x == 0) sm.info = n;
     __syncthreads();
     for (int k = 0; k < n; k += NB) {
+        int tid = opaque(threadIdx.x), lane = tid & 63;
         const int kb = min(NB, n - k), m = n - k;
         panel_move<T, LD, false, false>(A, n, k, m, kb, P);
         __syncthreads();
-        // Column j of the panel, one barrier: before it, each wave's best
-        // candidate for column j (|value|, row and the whole row) and row j
-        // are copied to buffers of the column's parity; after it every
-        // thread picks the same pivot row p from the four candidates, threads
-        // 0..kb-1 write the pivot row into row j, and each thread eliminates
-        // its own rows, taking the pivot row and (for row p) row j from the
-        // copies, then searches column j + 1 over its rows and the waves
-        // publish the next candidates into the other parity's buffers.
-        // Thread t owns the panel rows t + q BTH and is the only one to write
-        // them, apart from row j.  Rows are read across threads only through
-        // the copies, which a wave makes from rows its own lanes wrote (for
-        // column 0, from the loaded panel, after the barrier that follows
-        // the load).
+        // The panel's rows in registers, thread t holding rows t + q BTH; a row
+        // stays with its thread, a swap exchanges two rows' positions.  Column j,
+        // one barrier: each wave's best candidate (largest |value| among the rows
+        // at positions >= j, ties to the lowest) is copied to buffers of the
+        // column's parity; after it every thread picks the same pivot row from
+        // the four candidates and eliminates its own rows at positions > j.
+        // Multipliers go to P, to the row's own place, and a pivot row's entries
+        // when it is chosen.  x[e] is column j + e.
+        //
+        // Bound by the chain of a column: with the rows in LDS, read and written
+        // whole for every column, one took 4,000 cycles at order 512 and 3,300 at
+        // 128; this form takes 2,560 and 2,300.
         constexpr int RQ = NB == 32 ? 1 : 2;  // NB = 32 only for m <= 247
         T *cand = reinterpret_cast<T *>(&sm.cand[0][0][0]);  // [2][BNW][NB]
-        T *jrows = reinterpret_cast<T *>(&sm.jrow[0][0]);     // [2][NB]
-        // publish this wave's candidate (bv, bi: the lane's own) for the
-        // column of parity `par`, and (wave 0) row `jn` set aside
-        auto publish = [&](T bv, int bi, int par, int jn) __attribute__((always_inline)) {
-            const int wl = wave_first_max_lane(bv, bi);
-            bv = wl >= 0 ? lane_get(bv, wl) : T(0);
-            bi = wl >= 0 ? lane_get(bi, wl) : INT_MAX;
-            if (lane < NB)
-                cand[(par * BNW + wave) * NB + lane] = (bi != INT_MAX && lane < kb) ? P[bi * LD + lane] : T(0);
-            if (lane == 0) { sm.cand_v[par][wave] = (double)bv; sm.cand_i[par][wave] = bi; }
-            if (wave == 0 && lane < NB) jrows[par * NB + lane] = lane < kb ? P[jn * LD + lane] : T(0);
-        };
-        {
-            T bv = T(0);
-            int bi = INT_MAX;
+        T x[RQ][NB];
+        int pos[RQ];
 #pragma unroll
-            for (int q = 0; q < RQ; ++q) {
-                const int r = tid + q * BTH;
-                const T v = r < m ? fabs(P[r * LD]) : T(0);
-                const bool take = (r < m) & better(v, r, bv, bi);
-                bv = take ? v : bv;
-                bi = take ? r : bi;
-            }
-            publish(bv, bi, 0, 0);
+        for (int q = 0; q < RQ; ++q) {
+            const int r = tid + q * BTH;
+            pos[q] = r < m ? r : -1;
+#pragma unroll
+            for (int c = 0; c < NB; ++c) x[q][c] = r < m ? P[r * LD + c] : T(0);  // past kb: not used
         }
-        __syncthreads();
+#pragma unroll 1
         for (int j = 0; j < kb; ++j) {
 #pragma clang fp contract(off)
             const int par = j & 1;
-            T pa = (T)sm.cand_v[par][0];
-            int p = sm.cand_i[par][0], ww = 0;
-#pragma unroll
-            for (int q = 1; q < BNW; ++q) {
-                const bool take = better((T)sm.cand_v[par][q], sm.cand_i[par][q], pa, p);
-                pa = take ? (T)sm.cand_v[par][q] : pa;
-                p = take ? sm.cand_i[par][q] : p;
-                ww = take ? q : ww;
+            // this thread's candidate
+            T av = fabs(x[0][0]);
+            unsigned hi = pos[0] >= j ? rank_hi(av) : 0u, lo = rank_lo(av);
+            int bp = pos[0], bt = tid;
+            bool second = false;
+            if (RQ == 2) {
+                const T a1 = fabs(x[RQ - 1][0]);
+                const unsigned h1 = pos[RQ - 1] >= j ? rank_hi(a1) : 0u, l1 = rank_lo(a1);
+                second = (h1 > hi) | ((h1 == hi) & ((l1 > lo) | ((l1 == lo) & (pos[RQ - 1] < bp))));
+                hi = second ? h1 : hi;
+                lo = second ? l1 : lo;
+                bp = second ? pos[RQ - 1] : bp;
+                bt = second ? tid + BTH : bt;
             }
-            p = __builtin_amdgcn_readfirstlane(p);  // the same in every lane
-            ww = __builtin_amdgcn_readfirstlane(ww);
-            const T *prow = cand + (par * BNW + ww) * NB;  // row p (zeros at columns >= kb)
-            const T *jrow = jrows + par * NB;              // row j (zeros at columns >= kb)
-            const T piv = prow[j];
+            const int wl = first_max_lane(hi, lo, bp);
+            if (lane == (wl > 0 ? wl : 0)) {
+                sm.cand_hi[par][wave] = wl < 0 ? 0u : hi;
+                sm.cand_lo[par][wave] = lo;
+                sm.cand_p[par][wave] = bp;
+                sm.cand_t[par][wave] = bt;
+#pragma unroll
+                for (int e = 0; e < NB; ++e) cand[(par * BNW + wave) * NB + e] = second ? x[RQ - 1][e] : x[0][e];
+            }
+            __syncthreads();
+            const unsigned ch = sm.cand_hi[par][lane % BNW], cl = sm.cand_lo[par][lane % BNW];
+            const int cp = sm.cand_p[par][lane % BNW], ct = sm.cand_t[par][lane % BNW];
+            const unsigned top = dpp_max<DPP_XOR2>(dpp_max<DPP_XOR1>(ch));  // over each 4 lanes
+            const unsigned tied = (unsigned)__ballot(ch == top) & ((1u << BNW) - 1);
+            int bw = __builtin_ctz(tied);
+            if (tied & (tied - 1)) {
+                const int fl = first_max_lane(lane < BNW ? ch : 0u, cl, cp);
+                bw = fl > 0 ? fl : 0;
+            }
+            const int p = lane_get(cp, bw), t = lane_get(ct, bw);
+            const T *pr = cand + (par * BNW + bw) * NB;
+            const T piv = pr[0];
             if (tid == 0) {
                 sm.piv[j] = p;
-                if (pa < beps<T>() && sm.info == n) sm.info = k + j;
+                if (fabs(piv) < beps<T>() && sm.info == n) sm.info = k + j;
             }
-            if (tid < kb) P[j * LD + tid] = prow[tid];
-            T bv = T(0);
-            int bi = INT_MAX;
+            if (wave == 1 && j + lane < kb) P[t * LD + j + lane] = pr[lane];
 #pragma unroll
             for (int q = 0; q < RQ; ++q) {
-                const int r = tid + q * BTH;
-                if (r < m && r > j) {
-                    const T *src = r == p ? jrow : P + r * LD;  // row r after the swap
-                    const T mult = src[j] / piv;
-                    T x[NB], pm[NB];
+                pos[q] = pos[q] == p ? j : (pos[q] == j ? p : pos[q]);
+                if (pos[q] > j) {
+                    const T mult = x[q][0] / piv;
+                    P[(tid + q * BTH) * LD + j] = mult;
 #pragma unroll
-                    for (int c = 0; c < NB; ++c) {
-                        x[c] = src[c];
-                        pm[c] = c > j ? prow[c] : T(0);
-                    }
+                    for (int e = 1; e <= NB / 2; ++e) x[q][e - 1] = x[q][e] - mult * pr[e];
+                    if (j < NB / 2) {
 #pragma unroll
-                    for (int c = 0; c < NB; ++c) P[r * LD + c] = x[c] - mult * pm[c];
-                    P[r * LD + j] = mult;
-                    if (j + 1 < kb) {
-                        const T v = fabs(P[r * LD + j + 1]);
-                        const bool take = better(v, r, bv, bi);
-                        bv = take ? v : bv;
-                        bi = take ? r : bi;
+                        for (int e = NB / 2 + 1; e < NB; ++e) x[q][e - 1] = x[q][e] - mult * pr[e];
                     }
                 }
             }
-            if (j + 1 < kb) publish(bv, bi, par ^ 1, j + 1);
-            __syncthreads();
         }
+        __syncthreads();
+        // the rows that moved to their positions in P
+#pragma unroll
+        for (int q = 0; q < RQ; ++q)
+            if (pos[q] >= 0 && pos[q] != tid + q * BTH) {
+#pragma unroll
+                for (int c = 0; c < NB; ++c) x[q][c] = P[(tid + q * BTH) * LD + c];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < RQ; ++q)
+            if (pos[q] >= 0 && pos[q] != tid + q * BTH) {
+#pragma unroll
+                for (int c = 0; c < NB; ++c) P[pos[q] * LD + c] = x[q][c];
+            }
+        tid = opaque(tid);
         if (tid < kb) piv_out[k + tid] = k + sm.piv[tid];
+        __syncthreads();
+        T *L11 = reinterpret_cast<T *>(sm.l11);
+        for (int e = tid; e < NB * NB; e += BTH) L11[e] = P[(e % NB) * LD + e / NB];  // past kb: not used
         panel_move<T, LD, true, false>(A, n, k, m, kb, P);
         // row swaps on the columns outside the panel and on the RHS, as the
         // net moves of the panel's swaps: every source read before any write
@@ -286,90 +318,145 @@ __device__ int lu_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs,
                 else { base = B + (long)(q - k - right) * n + k; rs = 1; }
                 T v[2 * NB];
 #pragma unroll
-                for (int e = 0; e < 2 * NB; ++e)
-                    if (e < mc) v[e] = base[sm.msrc[e] * rs];
+                for (int g = 0; g < 2 * NB; g += 8)
+                    if (g < mc) {
 #pragma unroll
-                for (int e = 0; e < 2 * NB; ++e)
-                    if (e < mc) base[sm.mdst[e] * rs] = v[e];
+                        for (int e = g; e < g + 8; ++e) v[e] = base[sm.msrc[e] * rs];
+                    }
+#pragma unroll
+                for (int g = 0; g < 2 * NB; g += 8)
+                    if (g < mc) {
+#pragma unroll
+                        for (int e = g; e < g + 8; ++e) base[sm.mdst[e] * rs] = v[e];
+                    }
             }
         }
         __syncthreads();
+        tid = opaque(tid);
         // block row: U12 = L11^-1 A12 and Y1 = L11^-1 B1, one column per thread,
-        // column sweep as gaussian_elimination applies it (lu.rs:603-616)
+        // column sweep as gaussian_elimination applies it (lu.rs:603-616), with
+        // L11 from a copy by columns, two entries per read
         for (int q = tid; q < right + nrhs; q += BTH) {
             T u[NB];
             T *base;
             long stride;
             if (q < right) { base = A + (long)k * n + k + kb + q; stride = n; }
             else { base = B + (long)(q - right) * n + k; stride = 1; }
+            if (kb == NB) {
 #pragma unroll
-            for (int i = 0; i < NB; ++i) u[i] = i < kb ? base[i * stride] : T(0);
+                for (int i = 0; i < NB; ++i) u[i] = base[i * stride];
+            } else {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) u[i] = i < kb ? base[i * stride] : T(0);
+            }
             {
 #pragma clang fp contract(off)
                 // unguarded: in a last panel narrower than NB the entries
-                // u[kb..] take garbage from LDS rows past the panel and are
-                // never stored
+                // u[kb..] take garbage from rows past the panel and are never
+                // stored
+                typedef T v2 __attribute__((ext_vector_type(2)));
 #pragma unroll
                 for (int c = 0; c < NB; ++c) {
                     // one column of L11 at a time: scheduled freely, the
                     // unrolled sweep would hold all of L11 in registers
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int i = c + 1; i < NB; ++i) u[i] = u[i] - P[i * LD + c] * u[c];
+                    for (int i = (c + 1) & ~1; i < NB; i += 2) {
+                        const v2 l = *reinterpret_cast<const v2 *>(&L11[c * NB + i]);
+                        if (i > c) u[i] = u[i] - l.x * u[c];
+                        u[i + 1] = u[i + 1] - l.y * u[c];
+                    }
                 }
             }
+            if (kb == NB) {
 #pragma unroll
-            for (int i = 1; i < NB; ++i)
-                if (i < kb) base[i * stride] = u[i];
+                for (int i = 1; i < NB; ++i) base[i * stride] = u[i];
+            } else {
+#pragma unroll
+                for (int i = 1; i < NB; ++i)
+                    if (i < kb) base[i * stride] = u[i];
+            }
         }
         __syncthreads();
-        // trailing update A22 -= L21 * U12 on MFMA tiles: a wave takes a strip
-        // of TSTRIP_LU tiles along a tile row and issues all of the strip's
-        // global loads (C tiles and U12 fragments) before its MFMAs
+        // Trailing update A22 -= L21 * U12 on MFMA tiles (kb = NB here): a wave
+        // takes every BNW-th tile row of a strip of TSTRIP_LU tile columns, with
+        // the strip's U12 in registers and the next tile row's entries in flight.
+        // Entries past the edge are read from the last row or column and not
+        // stored.  (Loading U12 anew for each tile row and nothing ahead, the
+        // update took 3.3 M cycles at order 512; this takes 2.3 M.)
+        tid = opaque(tid);
+        lane = tid & 63;
         const int mt = m - kb;  // rows / cols of A22
         if (mt > 0) {
             using Acc = typename BMfma<T>::acc;
-            constexpr int KS = NB / 4;
-            const int tiles = (mt + 15) / 16, strips = (tiles + TSTRIP_LU - 1) / TSTRIP_LU;
+            constexpr int KS = NB / 4, S = TSTRIP_LU;
+            const int tiles = (mt + 15) / 16;
             const int lr = lane & 15, lk = lane >> 4;
             T *C = A + (long)(k + kb) * n + k + kb;
             const T *U = A + (long)k * n + k + kb;
-            for (int t = wave; t < tiles * strips; t += BNW) {
-                const int ti = t / strips, tj0 = (t - ti * strips) * TSTRIP_LU;
-                Acc acc[TSTRIP_LU];
-                T bf[TSTRIP_LU][KS];
+            for (int tj0 = 0; tj0 < tiles; tj0 += S) {
+                const int ns = tiles - tj0 < S ? tiles - tj0 : S;
+                T bf[S][KS];
+                int gj[S];
 #pragma unroll
-                for (int s = 0; s < TSTRIP_LU; ++s) {
-                    const int gj = (tj0 + s) * 16 + lr;
+                for (int s = 0; s < S; ++s) {
+                    const int g = (tj0 + s) * 16 + lr;
+                    gj[s] = g < mt ? g : mt - 1;
+                    if (s < ns) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int gi = ti * 16 + BMfma<T>::row(lk, r);
-                        acc[s][r] = (gi < mt && gj < mt) ? C[(long)gi * n + gj] : T(0);
-                    }
-#pragma unroll
-                    for (int q = 0; q < KS; ++q) {
-                        const int kk = 4 * q + lk;
-                        bf[s][q] = (gj < mt && kk < kb) ? U[(long)kk * n + gj] : T(0);
+                        for (int q = 0; q < KS; ++q) bf[s][q] = U[(long)(4 * q + lk) * n + gj[s]];
                     }
                 }
-                T af[KS];
-#pragma unroll
-                for (int q = 0; q < KS; ++q) {
-                    const int kk = 4 * q + lk, ai = ti * 16 + lr;
-                    af[q] = (ai < mt && kk < kb) ? -P[(kb + ai) * LD + kk] : T(0);
-                }
-#pragma unroll
-                for (int s = 0; s < TSTRIP_LU; ++s)
-#pragma unroll
-                    for (int q = 0; q < KS; ++q) acc[s] = BMfma<T>::op(af[q], bf[s][q], acc[s]);
-#pragma unroll
-                for (int s = 0; s < TSTRIP_LU; ++s) {
-                    const int gj = (tj0 + s) * 16 + lr;
+                auto load = [&](int ti, Acc(&c)[S]) __attribute__((always_inline)) {
+                    const T *row[4];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        const int gi = ti * 16 + BMfma<T>::row(lk, r);
-                        if (gi < mt && gj < mt) C[(long)gi * n + gj] = acc[s][r];
+                        const int g = ti * 16 + BMfma<T>::row(lk, r);
+                        row[r] = C + (long)(g < mt ? g : mt - 1) * n;
                     }
+#pragma unroll
+                    for (int s = 0; s < S; ++s)
+                        if (s < ns) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) c[s][r] = row[r][gj[s]];
+                        }
+                };
+                Acc acc[S], nxt[S];
+                if (wave < tiles) load(wave, acc);
+                for (int ti = wave; ti < tiles; ti += BNW) {
+                    // read and negated before the next loads are issued, which a
+                    // wait for LDS would wait for
+                    T af[KS];
+                    const int ai = ti * 16 + lr < mt ? ti * 16 + lr : mt - 1;
+#pragma unroll
+                    for (int q = 0; q < KS; ++q) af[q] = -P[(kb + ai) * LD + 4 * q + lk];
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (ti + BNW < tiles) load(ti + BNW, nxt);
+#pragma unroll
+                    for (int s = 0; s < S; ++s)
+                        if (s < ns) {
+#pragma unroll
+                            for (int q = 0; q < KS; ++q) acc[s] = BMfma<T>::op(af[q], bf[s][q], acc[s]);
+                        }
+                    const bool whole = ti * 16 + 16 <= mt && (tj0 + ns) * 16 <= mt;
+                    T *const out = C + (long)(ti * 16) * n;
+                    if (whole) {
+#pragma unroll
+                        for (int s = 0; s < S; ++s)
+                            if (s < ns) {
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) out[(long)BMfma<T>::row(lk, r) * n + gj[s]] = acc[s][r];
+                            }
+                    } else {
+#pragma unroll
+                        for (int s = 0; s < S; ++s)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r)
+                                if (ti * 16 + BMfma<T>::row(lk, r) < mt && (tj0 + s) * 16 + lr < mt)
+                                    out[(long)BMfma<T>::row(lk, r) * n + gj[s]] = acc[s][r];
+                    }
+#pragma unroll
+                    for (int s = 0; s < S; ++s) acc[s] = nxt[s];
                 }
             }
             // RHS rows below the block: B[r][k+kb+i] -= sum_c L21[i][c] * Y1[r][c]
@@ -401,11 +488,13 @@ enum { TS_LOWER_UNIT = 0, TS_LOWER = 1, TS_UPPER = 2, TS_LOWER_T = 3 };
 // transpose_back_substitution divides and then subtracts x[i] * l[i][j]
 // (cholesky.rs:329-361).
 template <class T, int MODE>
-__device__ void tri_solve(const T *__restrict__ A, int n, T *__restrict__ X, int nrhs, Smem &sm) {
+__device__ __attribute__((noinline)) void tri_solve(const T *__restrict__ A, int n, T *__restrict__ X, int nrhs, Smem &sm) {
     constexpr int TB = 32, DL = TB + 1;
     T *D = reinterpret_cast<T *>(sm.panel);
     T *XB = D + TB * DL;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    n = __builtin_amdgcn_readfirstlane(n);
+    nrhs = __builtin_amdgcn_readfirstlane(nrhs);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool fwd = MODE == TS_LOWER_UNIT || MODE == TS_LOWER;
     const int nblk = (n + TB - 1) / TB;
     for (int bi = 0; bi < nblk; ++bi) {
@@ -492,13 +581,18 @@ __device__ void tri_solve(const T *__restrict__ A, int n, T *__restrict__ X, int
 // Left-looking Cholesky of A in place (lower triangle), RHS forward-solved
 // along the way (B := L^-1 B).  Returns the first failing column or n.
 template <class T, int NB>
-__device__ int chol_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs, Smem &sm) {
+__device__ __attribute__((noinline)) int chol_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs, Smem &sm) {
     T *P = reinterpret_cast<T *>(sm.panel);
     constexpr int LD = NB + 1;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) sm.info = n;
+    // (arguments of a called function count as different in every lane: the
+    // branches on them would be masks)
+    n = __builtin_amdgcn_readfirstlane(n);
+    nrhs = __builtin_amdgcn_readfirstlane(nrhs);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (threadIdx.x == 0) sm.info = n;
     __syncthreads();
     for (int k = 0; k < n; k += NB) {
+        int tid = opaque(threadIdx.x), lane = tid & 63;
         const int kb = min(NB, n - k), m = n - k;
         panel_move<T, LD, false, true>(A, n, k, m, kb, P);
         __syncthreads();
@@ -567,6 +661,8 @@ __device__ int chol_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs,
                 if (i < kb) x[i] = xv[i];
         }
         __syncthreads();
+        tid = opaque(tid);
+        lane = tid & 63;
         const int mt = m - kb;
         if (mt > 0) {
             for (int q = tid; q < mt * nrhs; q += BTH) {
@@ -581,53 +677,72 @@ __device__ int chol_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs,
                     if (c < kb) s = s - P[(kb + i) * LD + c] * yv[c];
                 br[k + kb + i] = s;
             }
-            // SYRK on lower tiles: A22 -= L21 L21^T, in strips of TSTRIP tiles
-            // along a tile row (tiles right of the diagonal tile skipped), the
-            // strip's C tiles loaded before its MFMAs
+            // SYRK on lower tiles: A22 -= L21 L21^T (kb = NB here), as the LU's
+            // trailing update: every BNW-th tile row of a strip of tile columns
+            // per wave, the strip's operand in registers and the next tile row's
+            // entries in flight.  (With strips of four read anew for each tile
+            // row it took 2.2 M cycles at order 512; this takes 1.3 M.)
             using Acc = typename BMfma<T>::acc;
-            constexpr int KS = NB / 4;
+            constexpr int KS = NB / 4, S = TSTRIP;
             const int tiles = (mt + 15) / 16;
             const int lr = lane & 15, lk = lane >> 4;
             T *C = A + (long)(k + kb) * n + k + kb;
-            int t = 0;
-            for (int ti = 0; ti < tiles; ++ti) {
-                T af[KS];
+            for (int tj0 = 0; tj0 < tiles; tj0 += S) {
+                T bf[S][KS];
+                int gj[S];
 #pragma unroll
-                for (int q = 0; q < KS; ++q) {
-                    const int kk = 4 * q + lk, ai = ti * 16 + lr;
-                    af[q] = (ai < mt && kk < kb) ? -P[(kb + ai) * LD + kk] : T(0);
+                for (int s = 0; s < S; ++s) {
+                    const int g = (tj0 + s) * 16 + lr;
+                    gj[s] = g < mt ? g : mt - 1;
+#pragma unroll
+                    for (int q = 0; q < KS; ++q) bf[s][q] = P[(kb + gj[s]) * LD + 4 * q + lk];
                 }
-                for (int tj0 = 0; tj0 <= ti; tj0 += TSTRIP, ++t) {
-                    if (t % BNW != wave) continue;
-                    Acc acc[TSTRIP];
+                auto load = [&](int ti, Acc(&c)[S]) __attribute__((always_inline)) {
+                    const T *row[4];
 #pragma unroll
-                    for (int s = 0; s < TSTRIP; ++s) {
-                        const int gj = (tj0 + s) * 16 + lr;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int gi = ti * 16 + BMfma<T>::row(lk, r);
-                            acc[s][r] = (tj0 + s <= ti && gi < mt && gj < mt) ? C[(long)gi * n + gj] : T(0);
-                        }
+                    for (int r = 0; r < 4; ++r) {
+                        const int g = ti * 16 + BMfma<T>::row(lk, r);
+                        row[r] = C + (long)(g < mt ? g : mt - 1) * n;
                     }
 #pragma unroll
-                    for (int s = 0; s < TSTRIP; ++s) {
-                        const int gj = (tj0 + s) * 16 + lr;
+                    for (int s = 0; s < S; ++s)
+                        if (tj0 + s <= ti) {
 #pragma unroll
-                        for (int q = 0; q < KS; ++q) {
-                            const int kk = 4 * q + lk;
-                            const T bf = (gj < mt && kk < kb) ? P[(kb + gj) * LD + kk] : T(0);
-                            acc[s] = BMfma<T>::op(af[q], bf, acc[s]);
+                            for (int r = 0; r < 4; ++r) c[s][r] = row[r][gj[s]];
                         }
+                };
+                Acc acc[S], nxt[S];
+                if (tj0 + wave < tiles) load(tj0 + wave, acc);
+                for (int ti = tj0 + wave; ti < tiles; ti += BNW) {
+                    T af[KS];
+                    const int ai = ti * 16 + lr < mt ? ti * 16 + lr : mt - 1;
+#pragma unroll
+                    for (int q = 0; q < KS; ++q) af[q] = -P[(kb + ai) * LD + 4 * q + lk];
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (ti + BNW < tiles) load(ti + BNW, nxt);
+#pragma unroll
+                    for (int s = 0; s < S; ++s)
+                        if (tj0 + s <= ti) {
+#pragma unroll
+                            for (int q = 0; q < KS; ++q) acc[s] = BMfma<T>::op(af[q], bf[s][q], acc[s]);
+                        }
+                    T *const out = C + (long)(ti * 16) * n;
+                    if (ti * 16 + 16 <= mt && tj0 + S <= ti) {
+#pragma unroll
+                        for (int s = 0; s < S; ++s)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) out[(long)BMfma<T>::row(lk, r) * n + gj[s]] = acc[s][r];
+                    } else {
+#pragma unroll
+                        for (int s = 0; s < S; ++s)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                const int gi = ti * 16 + BMfma<T>::row(lk, r);
+                                if (gi < mt && (tj0 + s) * 16 + lr <= gi) out[(long)BMfma<T>::row(lk, r) * n + gj[s]] = acc[s][r];
+                            }
                     }
 #pragma unroll
-                    for (int s = 0; s < TSTRIP; ++s) {
-                        const int gj = (tj0 + s) * 16 + lr;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int gi = ti * 16 + BMfma<T>::row(lk, r);
-                            if (tj0 + s <= ti && gi < mt && gj < mt && gj <= gi) C[(long)gi * n + gj] = acc[s][r];
-                        }
-                    }
+                    for (int s = 0; s < S; ++s) acc[s] = nxt[s];
                 }
             }
         }
