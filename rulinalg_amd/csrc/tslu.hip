@@ -104,7 +104,7 @@ struct TourneyShared {
     float u[TG][TW - TG];          // U12 of a group of columns
     unsigned long long act[4];     // rows of the tile not yet chosen
     int id[TLR];                   // row numbers (-1: none)
-    int slot[TW];                  // tile row of pivot j (-1: none)
+    int slot[TW];                  // tile row of pivot j (-1: not known yet, -2: none)
     int order[TW];                 // its row number
     int s_last;
 };
@@ -156,13 +156,18 @@ __device__ __forceinline__ void load_rows(TourneyShared &sh, const float *__rest
     for (int q = 0; q < 16; ++q) *reinterpret_cast<float4 *>(&sh.tile[at(q * 16 + r0, c)]) = v[q];
 }
 
-// Columns cb .. cb+15 of the tile and the pivot rows' part right of them, by one
-// wave: lane l holds rows l, l + 64, l + 128 and l + 192 in registers, so that a
+__device__ __forceinline__ void publish_slot(TourneyShared &sh, int i, int t) {
+    if ((threadIdx.x & 63) == 0)
+        __hip_atomic_store(&sh.slot[i], t, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Columns cb .. cb+15 of the tile, by one wave: lane l holds rows l, l + 64, l + 128 and l + 192 in registers, so that a
 // column needs no barrier.  The pivot is the largest |value| of the rows not yet
 // chosen (ties: any; the choice is free for the tournament).  Every lane sets
 // its best row's entries aside while the maximum is found, so that no branch
 // (about 120 cycles) follows it; the winner's reach all lanes through scalar
 // registers, and the other rows form their multipliers and are eliminated.
+// Every column goes to the tile as it is done, then its pivot's row to sh.slot.
 __device__ __forceinline__ void factor_group(TourneyShared &sh, int cb, int w) {
     const int lane = opaque(threadIdx.x & 63);
     float x[4][TG];
@@ -176,21 +181,7 @@ __device__ __forceinline__ void factor_group(TourneyShared &sh, int cb, int w) {
             x[r][q] = v.x; x[r][q + 1] = v.y; x[r][q + 2] = v.z; x[r][q + 3] = v.w;
         }
     }
-    int mine = -1;  // lane c: the tile row of pivot cb + c
-    // U12 = L11^-1 A12, one column per lane, a row behind the pivots: its entry
-    // of A and its multipliers, which each column leaves in the tile
-    const int rest = TW - TG - cb, col = min(cb + TG + lane, TW - 1);
-    float u12[TG], an = 0.f;
-    float4 ln[TG / 4] = {};
-    auto solve = [&](auto ic) __attribute__((always_inline)) {
-        constexpr int i = decltype(ic)::value;
-        u12[i] = an;
-#pragma unroll
-        for (int q = 0; q < i; ++q) {
-            const float l = q % 4 == 0 ? ln[q / 4].x : q % 4 == 1 ? ln[q / 4].y : q % 4 == 2 ? ln[q / 4].z : ln[q / 4].w;
-            u12[i] = fmaf(-l, u12[q], u12[i]);
-        }
-    };
+    int prev = -2;                // the pivot before: its tile row (-2: none)
     float m[4] = {}, u[TG] = {};  // of the pivot before: its elimination is completed
     unsigned key[4];              // while the next maximum is found
 #pragma unroll
@@ -249,51 +240,67 @@ __device__ __forceinline__ void factor_group(TourneyShared &sh, int cb, int w) {
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (c > 0) solve(std::integral_constant<int, c - 1>{});
+        // (the columns before are in the tile by now: the release does not wait)
+        if constexpr (c > 0) publish_slot(sh, cb + c - 1, prev);
         const int o = (int)((b2 >> l) & 1), in = (int)((o ? b1 >> l : b0 >> l) & 1);
         const int t = (2 * o + in) * 64 + l;
-        mine = lane == c && mx != 0u ? t : mine;  // (0: no row was left)
-        an = sh.tile[at(t, col)];
-#pragma unroll
-        for (int q = 0; q < c; q += 4) ln[q / 4] = *reinterpret_cast<const float4 *>(&sh.tile[at(t, cb + q)]);
+        prev = mx != 0u && cb + c < w ? t : -2;  // (0: no row was left)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             x[r][c] = bit_of(act[r], m[r], x[r][c]);
-            if constexpr (c + 1 < TG) sh.tile[at(r * 64 + lane, cb + c)] = x[r][c];
+            sh.tile[at(r * 64 + lane, cb + c)] = x[r][c];
         }
     });
+    publish_slot(sh, cb + TG - 1, prev);
+    if (lane == 0) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-#pragma unroll
-        for (int q = 0; q < TG; q += 4)
-            *reinterpret_cast<float4 *>(&sh.tile[at(r * 64 + lane, cb + q)]) =
-                make_float4(x[r][q], x[r][q + 1], x[r][q + 2], x[r][q + 3]);
-        if (lane == 0) sh.act[r] = act[r];
-    }
-    if (lane < TG) sh.slot[cb + lane] = cb + lane < w ? mine : -1;
-    solve(std::integral_constant<int, TG - 1>{});
-    if (lane < rest) {
-#pragma unroll
-        for (int i = 0; i < TG; ++i) {
-            sh.u[i][lane] = u12[i];
-            const int t = lane_get(mine, i);
-            if (i && t >= 0) sh.tile[at(t, col)] = u12[i];
-        }
+        for (int r = 0; r < 4; ++r) sh.act[r] = act[r];
     }
 }
 
+// The pivot rows' part right of columns cb .. cb+15 (cb < 48), U12 = L11^-1 A12,
+// one column per lane: by another wave behind factor_group, a row as soon as its
+// pivot is known.  factor_group waits for nothing, so the wait ends; it is bounded
+// all the same.
+__device__ __forceinline__ void solve_group(TourneyShared &sh, int cb) {
+    const int lane = opaque(threadIdx.x & 63);
+    const int rest = TW - TG - cb, col = min(cb + TG + lane, TW - 1);
+    float u12[TG];
+    static_for<TG>([&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        int t = -1;
+        for (int spin = 0; t == -1 && spin < (1 << 20); ++spin) {
+            t = __hip_atomic_load(&sh.slot[cb + i], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (t == -1) __builtin_amdgcn_s_sleep(1);
+        }
+        t = __builtin_amdgcn_readfirstlane(t);
+        const int r = max(t, 0);
+        float l[TG], v = sh.tile[at(r, col)];
+#pragma unroll
+        for (int q = 0; q < i; ++q) l[q] = sh.tile[at(r, cb + q)];
+#pragma unroll
+        for (int q = 0; q < i; ++q) v = fmaf(-l[q], u12[q], v);
+        u12[i] = v;
+        if (lane < rest) {
+            sh.u[i][lane] = v;
+            if (i && t >= 0) sh.tile[at(r, col)] = v;
+        }
+    });
+}
+
 // Partial pivoting on the 256 rows of the tile, 16 columns at a time: wave 0
-// factors them and solves the pivot rows' part right of them, then all waves
-// update the other rows on the matrix cores.  On return the row chosen at step j (sh.slot, sh.order) holds its
-// multipliers left of column j and its U row from column j on.
+// factors them, wave 1 solves the pivot rows' part right of them meanwhile, then
+// all waves update the other rows on the matrix cores.  On return the row chosen
+// at step j (sh.slot, sh.order) holds its multipliers left of column j and its U
+// row from column j on.
 //
-// Bound by the serial chain per column, about 130 instructions of one wave (a
+// Bound by the serial chain per column, about 115 instructions of one wave (a
 // lone wave issues one in 4.3 to 6 cycles).  One row per thread, with the search
 // and the pivot row going through LDS and a barrier per column, took 250 us for a
 // panel on average over a factorization of order 16384 (four levels at most,
-// beside the trailing update); this form takes 147, and a level on an idle device
-// 33.  Branching to the winner's row instead of setting the best entries aside
-// takes as long.
+// beside the trailing update); this form takes 142, and a level on an idle device
+// 32 instead of 58.  Branching to the winner's row instead of setting the best
+// entries aside takes as long; with the solve in the same wave, 147.
 __device__ void gepp256(TourneyShared &sh, int w) {
     using Acc = Mfma<float>::acc;
     const int wave = threadIdx.x >> 6;
@@ -303,6 +310,10 @@ __device__ void gepp256(TourneyShared &sh, int w) {
         if (wave == 0) {
             __builtin_amdgcn_s_setprio(3);  // ahead of another kernel's waves on this SIMD
             factor_group(sh, cb, w);
+            __builtin_amdgcn_s_setprio(0);
+        } else if (wave == 1 && cb + TG < w) {
+            __builtin_amdgcn_s_setprio(3);
+            solve_group(sh, cb);
             __builtin_amdgcn_s_setprio(0);
         }
         __syncthreads();
