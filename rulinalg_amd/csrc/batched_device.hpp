@@ -177,6 +177,9 @@ __device__ __forceinline__ void panel_moves(int kb, const int *piv, int *mdst, i
 
 // ---------------------------------------------------------------- LU
 
+// (The phases stay called functions: with all of them forced inline, and their
+// registers spilled, the kernel faulted the GPU, for a cause not shown.)
+//
 // Factor the n x n matrix A (ld = n, type T) in place with RHS vectors B
 // (nrhs x n, may be null) carried along as extra columns, so that on return
 // B holds L^-1 P B.  Pivots go to piv_out[0..n).  Returns the first failing

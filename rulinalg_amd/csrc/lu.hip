@@ -234,7 +234,7 @@ template <class T> constexpr int TW = PNB + TilePad<T>::value;
 // arithmetic.  Rows of 64 kept in LDS with three barriers per column and an
 // update of the whole row per column took, in FP64, 122 us for a panel of 256
 // rows and, on average over the factorization, 188 at order 1,531 and 209 at
-// 16,384; this form takes 68, 148 and 184.
+// 16,384; this form takes 68, 137 and 184.
 //
 // EXACT (FP32, and FP64 orders up to 64): divisions, and separately rounded
 // products and differences in the reference's order.
@@ -776,8 +776,8 @@ __global__ __launch_bounds__(256) void k_trsm_llu(T *__restrict__ A, long lda, i
 // first stores it for the outer block row (have_inv: it is there already).
 //
 // Bound by latencies: four dependent trips to memory and about 4,000 cycles of
-// inversion and product.  It takes 13.4 us at order 16384 in FP64 (14.7 at 1531,
-// unaligned), where three launches, for the inverse, the swaps and the solve,
+// inversion and product.  It takes 17 us in FP64 (12 in FP32) on average at order
+// 16384, where three launches, for the inverse, the swaps and the solve,
 // took 8.5, 13.6 and 8.
 //
 // L^-1 in blocks: the diagonal ones of IB x IB by forward substitution, a lane
