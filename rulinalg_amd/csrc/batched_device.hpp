@@ -44,15 +44,6 @@
 
 namespace rlg {
 
-// The value again, unknown to the compiler: addresses made from it are formed
-// where they are used, not ahead of a loop and kept in scratch memory.
-__device__ __forceinline__ int opaque(int v) {
-#ifdef __AMDGCN__
-    asm volatile("" : "+v"(v));
-#endif
-    return v;
-}
-
 constexpr int BTH = 256;
 constexpr int BMAXN = RLG_BATCH_MAX_N;
 constexpr int PANEL = 8704;       // doubles: 512 x 17

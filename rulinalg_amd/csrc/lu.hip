@@ -573,6 +573,266 @@ __global__ __launch_bounds__(PanelRows<T>::value) void k_lu_panel(
     }
 }
 
+// ---------------------------------------------------------------- panels of up to 256 rows
+
+// The panel A[k:k+m, k:k+w] with m <= 64 R <= 256, in FP64, by one workgroup:
+// k_lu_panel's arithmetic (the same bits), but one wave holds 16 columns of all
+// rows in registers, R rows per lane, so that a column needs no barrier and no LDS
+// on its chain; a second wave solves the pivot rows' part right of the group
+// meanwhile, and the four update the rest on the matrix cores.
+//
+// Bound by the chain of a column, 120 instructions of one wave for R = 1 and 400
+// for R = 4.  A row per thread, with two LDS round trips and a barrier per column,
+// took 68 us for any number of rows; this takes 34, 47, 57 and 68 us for R = 1 to
+// 4 (an order of 256 is factored in 347 instead of 417 us).  One loop body for the
+// 16 columns, the entries moving down a register per column, is 3 to 6 us slower:
+// it eliminates more entries than there are.
+constexpr size_t ONE_ROWS = 256;
+template <int R> struct OneShared {
+    double tile[R * 64 * PNB];           // see one_at
+    double u[SPW][PNB - SPW];            // U12 of a group of columns
+    unsigned long long act[R];           // rows not yet chosen
+    int slot[PNB];                       // row of pivot j (-1: not known yet)
+    int piv[PNB], pos[R * 64];
+};
+// Entry (row, col) of the tile: the 16-byte pieces of a row are permuted by its
+// number, so that 16 consecutive rows read at one column touch all banks.
+__device__ __forceinline__ int one_at(int row, int col) {
+    return row * PNB + (((col >> 1) ^ (row & 15)) << 1) + (col & 1);
+}
+// Columns cb .. cb+15, by wave 0; pos[r] is the position of row 64 r + lane.  The
+// pivot is the first maximum (see first_max_lane).  Every lane sets its best row's
+// entries aside, and the winner's reach all lanes through scalar registers.  A
+// chosen row's entries go to the tile when it is chosen (its registers are
+// eliminated on, with a multiplier of zero), the others' multipliers column by
+// column; then the row goes to sh.slot.
+template <int R>
+__device__ __forceinline__ void one_factor(OneShared<R> &sh, int cb, int w, int (&pos)[R]) {
+    typedef double v2 __attribute__((ext_vector_type(2)));
+    const int lane = opaque(threadIdx.x & 63);
+    double x[R][SPW];
+    unsigned long long act[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        act[r] = uniform(sh.act[r]);
+#pragma unroll
+        for (int q = 0; q < SPW; q += 2) {
+            const v2 v = *reinterpret_cast<const v2 *>(&sh.tile[one_at(r * 64 + lane, cb + q)]);
+            x[r][q] = v.x;
+            x[r][q + 1] = v.y;
+        }
+    }
+    static_for<SPW>([&](auto cc) __attribute__((always_inline)) {
+        constexpr int c = decltype(cc)::value;
+        const int j = cb + c;
+        if (j >= w) return;
+        unsigned key[R], d = 0u;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            key[r] = bit_of(act[r], rank_hi(fabs(x[r][c])), 0u);
+            d = max(d, key[r]);
+        }
+        double y[SPW];  // the entries of this lane's best row, its number and position
+        int best = 0, at = 0;
+        auto aside = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int e = c; e < SPW; ++e) y[e] = x[0][e];
+            best = 0;
+            at = pos[0];
+            unsigned most = key[0];
+#pragma unroll
+            for (int r = 1; r < R; ++r) {
+                const bool up = key[r] > most;
+#pragma unroll
+                for (int e = c; e < SPW; ++e) y[e] = up ? x[r][e] : y[e];
+                best = up ? r : best;
+                at = up ? pos[r] : at;
+                most = max(most, key[r]);
+            }
+        };
+        d = dpp_max<DPP_SHR<1>>(d);
+        d = dpp_max<DPP_SHR<2>>(d);
+        d = dpp_max<DPP_SHR<4>>(d);
+        d = dpp_max<DPP_SHR<8>>(d);
+        d = dpp_max<DPP_BCAST15>(d);
+        d = dpp_max<DPP_BCAST31>(d);
+        const unsigned mx = lane_get(d, 63);
+        aside();
+        unsigned long long hit[R];
+        int hits = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            hit[r] = __ballot(key[r] == mx);
+            hits += __popcll(hit[r]);
+        }
+        if (__builtin_expect(hits != 1, 0)) {  // equal high words: the low words, then the positions
+            unsigned lo[R], ml = 0u;
+            int mi = INT_MAX;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                lo[r] = key[r] == mx ? rank_lo(fabs(x[r][c])) : 0u;
+                ml = max(ml, lo[r]);
+            }
+            ml = wave_max_u32(ml);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (key[r] == mx && lo[r] == ml) mi = min(mi, pos[r]);
+            mi = wave_min_i32(mi);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                key[r] = key[r] == mx && lo[r] == ml && pos[r] == mi ? 1u : 0u;
+                hit[r] = __ballot(key[r] != 0u);
+            }
+            aside();
+        }
+        unsigned long long any = hit[0];
+#pragma unroll
+        for (int r = 1; r < R; ++r) any |= hit[r];
+        const int l = __builtin_ctzll(any);
+        double u[SPW];
+#pragma unroll
+        for (int e = c; e < SPW; ++e) u[e] = lane_get(y[e], l);
+        const int t = lane_get(best, l) * 64 + l, pl = lane_get(at, l);
+        if (lane == l) {
+            if (c & 1) sh.tile[one_at(t, j)] = y[c];
+#pragma unroll
+            for (int e = (c + 1) & ~1; e < SPW; e += 2)
+                *reinterpret_cast<v2 *>(&sh.tile[one_at(t, cb + e)]) = v2{y[e], y[e + 1]};
+        }
+        const double piv = u[c];
+        const double rc = recip(piv);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            act[r] &= ~hit[r];
+            pos[r] = pos[r] == pl ? j : (pos[r] == j ? pl : pos[r]);
+            const double mult = div_recip(x[r][c], piv, rc);
+            if (bit_of(act[r], true, false)) sh.tile[one_at(r * 64 + lane, j)] = mult;
+            const double m = bit_of(act[r], mult, 0.0);
+#pragma unroll
+            for (int e = c + 1; e < SPW; ++e) x[r][e] = fma(-m, u[e], x[r][e]);
+        }
+        if (lane == 0) {
+            sh.piv[j] = pl;
+            __hip_atomic_store(&sh.slot[j], t, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+    });
+    if (lane == 0) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) sh.act[r] = act[r];
+    }
+}
+
+// U12 = L11^-1 A12 of columns cb .. cb+15, one column per lane, by another wave
+// behind one_factor, which waits for nothing: the wait ends, and is bounded.
+template <int R> __device__ __forceinline__ void one_solve(OneShared<R> &sh, int cb) {
+    const int lane = opaque(threadIdx.x & 63);
+    const int rest = PNB - SPW - cb, col = min(cb + SPW + lane, PNB - 1);
+    double u12[SPW];
+    static_for<SPW>([&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        int t = -1;
+        for (int spin = 0; t == -1 && spin < (1 << 20); ++spin) {
+            t = __hip_atomic_load(&sh.slot[cb + i], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (t == -1) __builtin_amdgcn_s_sleep(1);
+        }
+        const int r = max(__builtin_amdgcn_readfirstlane(t), 0);
+        double l[SPW], v = sh.tile[one_at(r, col)];
+#pragma unroll
+        for (int q = 0; q < i; ++q) l[q] = sh.tile[one_at(r, cb + q)];
+#pragma unroll
+        for (int q = 0; q < i; ++q) v = fma(-l[q], u12[q], v);
+        u12[i] = v;
+        if (lane < rest) {
+            sh.u[i][lane] = v;
+            sh.tile[one_at(r, col)] = v;
+        }
+    });
+}
+
+template <int R>
+__global__ __launch_bounds__(256) void k_lu_panel_one(double *__restrict__ A, long lda, int k, int m, int w,
+                                                      int64_t *__restrict__ ipiv, int64_t *__restrict__ info, int n) {
+    __shared__ __attribute__((aligned(16))) OneShared<R> sh;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    {   // all loads in flight before the LDS stores
+        const int lane = tid & 63;
+        constexpr int PER = R * 16;
+        double v[PER];
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int r = q * 4 + wave;
+            v[q] = (r < m && lane < w) ? A[(long)(k + r) * lda + k + lane] : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < PER; ++q) sh.tile[one_at(q * 4 + wave, lane)] = v[q];  // zero past w and m
+    }
+    const unsigned long long have = __ballot(tid < m);
+    if ((tid & 63) == 0 && wave < R) sh.act[wave] = have;
+    if (tid < PNB) sh.slot[tid] = -1;
+    __syncthreads();
+
+    int pos[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) pos[r] = r * 64 + (tid & 63);
+#pragma unroll 1
+    for (int cb = 0; cb < w; cb += SPW) {
+        if (wave == 0) one_factor(sh, cb, w, pos);
+        else if (wave == 1 && cb + SPW < w) one_solve(sh, cb);
+        __syncthreads();
+        if (cb + SPW >= w) break;
+        if (wave < R) {
+            // this wave's 64 rows: A22 -= L21 U12; rows already chosen keep their values
+            const int lane = opaque(tid & 63), lr = lane & 15, lk = lane >> 4;
+            const unsigned long long act = uniform(sh.act[wave]);
+            double af[4][4];
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) af[rt][s] = sh.tile[one_at(wave * 64 + rt * 16 + lr, cb + 4 * s + lk)];
+#pragma unroll 1
+            for (int ct = cb + SPW; ct < PNB; ct += 16) {
+                double bf[4], cv[4][4];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) bf[s] = sh.u[4 * s + lk][ct - cb - SPW + lr];
+#pragma unroll
+                for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        cv[rt][r] = sh.tile[one_at(wave * 64 + rt * 16 + Mfma<double>::row(lk, r), ct + lr)];
+                Mfma<double>::acc acc[4] = {};
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll
+                    for (int rt = 0; rt < 4; ++rt) acc[rt] = Mfma<double>::op(af[rt][s], bf[s], acc[rt]);
+#pragma unroll
+                for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int row = rt * 16 + Mfma<double>::row(lk, r);
+                        if ((act >> row) & 1ull) sh.tile[one_at(wave * 64 + row, ct + lr)] = cv[rt][r] - acc[rt][r];
+                    }
+            }
+        }
+        __syncthreads();
+    }
+    const int lane = opaque(tid & 63);
+    if (wave == 0) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) sh.pos[r * 64 + lane] = pos[r];
+        // the first pivot below epsilon (every column has one: m >= w)
+        const double d = lane < w ? sh.tile[one_at(sh.slot[lane], lane)] : 1.0;
+        const unsigned long long small = __ballot(fabs(d) < eps_of<double>());
+        if (lane == 0 && small != 0ull && *info == (int64_t)n) *info = k + __builtin_ctzll(small);
+        if (lane < w) ipiv[k + lane] = (int64_t)k + sh.piv[lane];
+    }
+    __syncthreads();
+#pragma unroll 8
+    for (int q = 0; q < R * 16; ++q) {
+        const int r = q * 4 + wave;
+        if (r < m && lane < w) A[(long)(k + sh.pos[r]) * lda + k + lane] = sh.tile[one_at(r, lane)];
+    }
+}
+
 // ---------------------------------------------------------------- row swaps
 
 // Net effect of the swaps ipiv[k0 .. k0+cnt) as a list of (dst, src) rows:
@@ -999,13 +1259,24 @@ static int panel(hipStream_t s, T *a, size_t lda, size_t k, size_t m, size_t w, 
     RLG_PROF_W("lu_panel", s, 2.0 * (double)m * (double)w * sizeof(T));
     constexpr unsigned PT = PanelRows<T>::value;
     constexpr bool EX = sizeof(T) == 4;
-    if (G == 1) {  // no exchange; with the whole matrix in one panel the reference's bits
-        auto go = [&](auto exact) {
-            hipLaunchKernelGGL((k_lu_panel<T, decltype(exact)::value>), dim3(1), dim3(PT), 0, s, a, (long)lda,
-                               (int)k, (int)m, (int)w, ipiv, info, (int)n, lw.xch, lw.timeout);
-        };
-        if (EX || n <= (size_t)PNB) go(std::true_type{});
-        else go(std::integral_constant<bool, EX>{});
+    if constexpr (!EX) {
+        // one workgroup: the fewer rows per lane, the shorter the chain (see the kernel)
+        if (m <= ONE_ROWS && n > (size_t)PNB) {
+            auto one = [&](auto rows) {
+                hipLaunchKernelGGL((k_lu_panel_one<decltype(rows)::value>), dim3(1), dim3(256), 0, s, a, (long)lda,
+                                   (int)k, (int)m, (int)w, ipiv, info, (int)n);
+            };
+            if (m <= 64) one(std::integral_constant<int, 1>{});
+            else if (m <= 128) one(std::integral_constant<int, 2>{});
+            else if (m <= 192) one(std::integral_constant<int, 3>{});
+            else one(std::integral_constant<int, 4>{});
+            RLG_LAUNCHED();
+            return RLG_OK;
+        }
+    }
+    if (G == 1) {  // no exchange; in FP64 the whole matrix (n <= 64), to the reference's bits
+        hipLaunchKernelGGL((k_lu_panel<T, true>), dim3(1), dim3(PT), 0, s, a, (long)lda, (int)k, (int)m, (int)w,
+                           ipiv, info, (int)n, lw.xch, lw.timeout);
         RLG_LAUNCHED();
         return RLG_OK;
     }

@@ -115,23 +115,6 @@ __device__ __forceinline__ int at(int row, int col) {
     return row * TW + (((col >> 2) ^ (row & 15)) << 2) + (col & 3);
 }
 
-// The value again, unknown to the compiler: addresses made from it are formed
-// where they are used, not ahead of a loop and kept in scratch memory.
-__device__ __forceinline__ int opaque(int v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
-// The value, known to be the same in every lane.
-__device__ __forceinline__ unsigned long long uniform(unsigned long long v) {
-    return ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
-           (unsigned)__builtin_amdgcn_readfirstlane((int)v);
-}
-// b where this lane's bit of the (uniform) mask is clear, else a.
-template <class V> __device__ __forceinline__ V bit_of(unsigned long long mask, V a, V b) {
-    return __builtin_amdgcn_inverse_ballot_w64(mask) ? a : b;
-}
-
 // Rows sh.id[] of the panel into the tile (columns k .. k+w-1, zeros beyond).
 __device__ __forceinline__ void load_rows(TourneyShared &sh, const float *__restrict__ A, long lda, int k, int w,
                                           bool vec) {

@@ -58,6 +58,27 @@ template <int CTRL> __device__ __forceinline__ double dpp(double x) {
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
+// The value again, unknown to the compiler: addresses made from it are formed
+// where they are used, not ahead of a loop and kept in scratch memory.
+__device__ __forceinline__ int opaque(int v) {
+#ifdef __AMDGCN__
+    asm volatile("" : "+v"(v));
+#endif
+    return v;
+}
+
+#ifdef __AMDGCN__
+// The value, known to be the same in every lane.
+__device__ __forceinline__ unsigned long long uniform(unsigned long long v) {
+    return ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+           (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+}
+// b where this lane's bit of the (uniform) mask is clear, else a.
+template <class V> __device__ __forceinline__ V bit_of(unsigned long long mask, V a, V b) {
+    return __builtin_amdgcn_inverse_ballot_w64(mask) ? a : b;
+}
+#endif
+
 // Maximum of a 32-bit key over the wave (uniform result): two quad swaps
 // and two row mirrors, then the four rows' maxima from lanes 0, 16, 32, 48.
 __device__ __forceinline__ unsigned lane_get(unsigned x, int l) {
