@@ -33,6 +33,13 @@
 // FP64 at order 4096, per launch of 128 rows: 14.6 -> 9.1 us (upper, one
 // right-hand side), 10.3 -> 8.6 (unit lower); at order 16384 with 16
 // right-hand sides 56 -> 17.9 and 39.5 -> 17.2 us.
+//
+// The loads come next: with a test and a 64-bit product per load, a wave spends
+// some 500 instructions before the first barrier.  Whole blocks and rows load
+// without tests, from addresses a scalar apart: solves of order 4096 4 % faster
+// (LU 541 -> 520 us, 16 right-hand sides 1,017 -> 980; Cholesky 588 -> 567).
+// Taking four entries at a time from the lanes, and their solution redundantly in
+// each, is slower (541 -> 594 us): the chain is bound by instructions issued.
 #include <limits>
 
 #include "kernels.hpp"
@@ -78,11 +85,13 @@ __device__ __forceinline__ void tile_load(T (&v)[TPER], const T *__restrict__ M,
     constexpr int VL = TVL<T>;
     typedef T vT __attribute__((ext_vector_type(VL)));
     if (vec && rs == SB && cs == SB) {
+        constexpr int RPU = 256 / (SB / VL);  // rows per load: their addresses differ by a scalar
+        const int i0 = threadIdx.x / (SB / VL), j0 = (threadIdx.x % (SB / VL)) * VL;
+        const T *p = M + (long)(rb + i0) * lda + cb + j0;
 #pragma unroll
         for (int u = 0; u < TPER / VL; ++u) {
-            const int e = u * 256 + threadIdx.x;  // vector index
-            const int i = e / (SB / VL), j0 = (e % (SB / VL)) * VL;
-            const vT x = *reinterpret_cast<const vT *>(M + (long)(rb + i) * lda + cb + j0);
+            const int i = u * RPU + i0;
+            const vT x = *reinterpret_cast<const vT *>(p + u * (RPU * lda));
 #pragma unroll
             for (int t = 0; t < VL; ++t) {
                 const int j = j0 + t;
@@ -189,24 +198,43 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
     // product form: the wave's 16 rows (row ls of them per lane), the lane's
     // columns 4 VL u + VL grp + e, and the W entries of its accumulator
     const int jp = u0 + (int)blockIdx.x * RPW + wave * 16;
+    // full block and rows: no test per load, and row addresses a scalar apart
+    static_assert(RPW == CPW, "one test for both forms");
+    const bool full = S == TSB * SB && u0 + ((int)blockIdx.x + 1) * RPW <= u1;
     T mv[PRODUCT ? CW : MODE == LOWER_T ? CW : NIT * NC];
     T wpre[PRODUCT ? 1 : RDOT][PRODUCT ? 4 : MODE == LOWER_T ? 1 : NIT];
     if constexpr (PRODUCT) {
         typedef T vT __attribute__((ext_vector_type(VL)));
         const int j = jp + ls;
+        if (full && (vec || MODE == LOWER_T)) {
+            const T *p = MODE == LOWER_T ? M + (long)(s0 + grp * VL) * lda + j : M + (long)j * lda + s0 + grp * VL;
 #pragma unroll
-        for (int u = 0; u < CW / VL; ++u) {
-            const int c = (4 * u + grp) * VL;
-            if (MODE != LOWER_T && vec && c + VL <= S) {
-                const vT x = j < u1 ? *reinterpret_cast<const vT *>(M + (long)j * lda + s0 + c) : vT(T(0));
+            for (int u = 0; u < CW / VL; ++u) {
+                if constexpr (MODE == LOWER_T) {
 #pragma unroll
-                for (int e = 0; e < VL; ++e) mv[u * VL + e] = x[e];
-            } else {
+                    for (int e = 0; e < VL; ++e) mv[u * VL + e] = p[(4 * u * VL + e) * lda];
+                } else {
+                    const vT x = *reinterpret_cast<const vT *>(p + 4 * u * VL);
 #pragma unroll
-                for (int e = 0; e < VL; ++e)
-                    mv[u * VL + e] = j < u1 && c + e < S
-                                         ? M[MODE == LOWER_T ? (long)(s0 + c + e) * lda + j : (long)j * lda + s0 + c + e]
-                                         : T(0);
+                    for (int e = 0; e < VL; ++e) mv[u * VL + e] = x[e];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < CW / VL; ++u) {
+                const int c = (4 * u + grp) * VL;
+                if (MODE != LOWER_T && vec && c + VL <= S) {
+                    const vT x = j < u1 ? *reinterpret_cast<const vT *>(M + (long)j * lda + s0 + c) : vT(T(0));
+#pragma unroll
+                    for (int e = 0; e < VL; ++e) mv[u * VL + e] = x[e];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < VL; ++e)
+                        mv[u * VL + e] =
+                            j < u1 && c + e < S
+                                ? M[MODE == LOWER_T ? (long)(s0 + c + e) * lda + j : (long)j * lda + s0 + c + e]
+                                : T(0);
+                }
             }
         }
 #pragma unroll
@@ -216,14 +244,32 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
         }
     } else if constexpr (MODE == LOWER_T) {
         const bool act = jt < u1;
+        if (full) {
+            const T *p = M + (long)(s0 + wave * CW) * lda + jt;
 #pragma unroll
-        for (int q = 0; q < CW; ++q) {
-            const int c = wave * CW + q;
-            mv[q] = (act && c < S) ? M[(long)(s0 + c) * lda + jt] : T(0);
+            for (int q = 0; q < CW; ++q) mv[q] = p[q * lda];
+        } else {
+#pragma unroll
+            for (int q = 0; q < CW; ++q) {
+                const int c = wave * CW + q;
+                mv[q] = (act && c < S) ? M[(long)(s0 + c) * lda + jt] : T(0);
+            }
         }
 #pragma unroll
         for (int r = 0; r < RDOT; ++r)
             wpre[r][0] = (wave == 0 && act && r < nrhs) ? W[(long)r * ldw + jt] : T(0);
+    } else if (full) {
+        const T *p = M + (long)rbase * lda + s0 + ls, *wp = W + rbase;
+#pragma unroll
+        for (int it = 0; it < NIT; ++it)
+#pragma unroll
+            for (int k = 0; k < NC; ++k) mv[it * NC + k] = p[it * (4 * lda) + 16 * k];
+#pragma unroll
+        for (int r = 0; r < RDOT; ++r) {
+            if (r >= nrhs) break;
+#pragma unroll
+            for (int it = 0; it < NIT; ++it) wpre[r][it] = wp[r * ldw + it * 4];
+        }
     } else {
 #pragma unroll
         for (int it = 0; it < NIT; ++it) {
@@ -340,10 +386,8 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
     }
     __syncthreads();
     if (blockIdx.x == 0)
-        for (int e = tid; e < nrhs * S; e += 256) {
-            const int r = e / S, c = e - r * S;
-            X[(long)r * ldx + s0 + c] = xs[r][c];
-        }
+        for (int r = wave; r < nrhs; r += 4)
+            for (int c = lane; c < S; c += 64) X[(long)r * ldx + s0 + c] = xs[r][c];
 
     // ---- 2. remove the solved rows from this workgroup's share of [u0, u1)
     if constexpr (PRODUCT) {
