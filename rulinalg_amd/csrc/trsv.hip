@@ -28,8 +28,10 @@
 // and its right-hand side by the row's diagonal up front, which leaves a
 // broadcast and one fused multiply-add per column on the chain, and a wave
 // sweeps up to four right-hand sides together.  Scaled and swept that way, a
-// value that is not finite could reach entries it must not; a sub-block whose
-// result holds one is swept again with a division and a test per column.
+// value that is not finite could reach entries it must not, and a quotient below
+// the normal numbers would lose a term; a sub-block whose result holds the one or
+// may have lost the other (sweep_lossy) is swept again with a division and a test
+// per column.
 // FP64 at order 4096, per launch of 128 rows: 14.6 -> 9.1 us (upper, one
 // right-hand side), 10.3 -> 8.6 (unit lower); at order 16384 with 16
 // right-hand sides 56 -> 17.9 and 39.5 -> 17.2 us.
@@ -169,6 +171,40 @@ __device__ __forceinline__ T sweep_plain(const T (*t)[SB + TP<T>], T x, T dl, in
     return x;
 }
 
+// The exponent of v, with |v| in [2^(e-1), 2^e); 0 for zero, infinities and NaN.
+__device__ __forceinline__ int exponent(double v) { return __builtin_amdgcn_frexp_exp(v); }
+__device__ __forceinline__ int exponent(float v) { return __builtin_amdgcn_frexp_expf(v); }
+
+// Exponents below which the scaled sweep may lose bits.  A step of it is one fused
+// multiply-add, exact but for its rounding, so what counts is that the quotients
+// m / d are normal (NORMAL) and that no entry is so small that 64 roundings to a
+// multiple of the smallest subnormal number show in it (LOW): neither the entries
+// that are not zero, nor the products whose sum could have come out as zero.
+// ENTRY, SOLVED and RHS are bounds on the three kinds of exponent that together
+// imply both.  (They cost 1 % of a solve of order 4096, 562 to 569 us.)
+template <class T> struct Range;
+template <> struct Range<double> {
+    static constexpr int NORMAL = -1021, LOW = -1009, ENTRY = -500, SOLVED = -500, RHS = -1000;
+};
+template <> struct Range<float> {
+    static constexpr int NORMAL = -125, LOW = -117, ENTRY = -45, SOLVED = -70, RHS = -100;
+};
+// Whether the scaled sweep of a sub-block (x to y) can have lost bits; uniform.
+template <class T, int MODE>
+__device__ __forceinline__ bool sweep_lossy(const T (*t)[SB + TP<T>], T x, T dl, T y, int lane) {
+    using R = Range<T>;
+    const int ed = exponent(dl);
+    int q = 0;  // the smallest quotient's exponent
+#pragma unroll 8
+    for (int c = 0; c < SB; ++c) {
+        const T m = MODE == LOWER_T ? t[c][lane] : t[lane][c];
+        q = min(q, m != T(0) ? exponent(m) - ed : 0);
+    }
+    q = wave_min_i32(q);
+    const int s = wave_min_i32(exponent(y));
+    return q < R::NORMAL || s < R::LOW || q + s < R::LOW || __any(x != T(0) && exponent(x) - ed < R::LOW);
+}
+
 // NR: right-hand sides per wave (wave w sweeps w, w + 4, ...).
 template <class T, int MODE, int NR>
 __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long lda, int n, int q0,
@@ -179,6 +215,7 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
     // [2] the off-diagonal tile inside the stored triangle
     __shared__ __attribute__((aligned(16))) T tl[3][SB][SB + TP<T>];
     __shared__ __attribute__((aligned(16))) T xs[TMAXR][TSB * SB + TP<T>];
+    __shared__ int s_low[4];  // the smallest exponent in each wave's part of the diagonal tiles
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int s0 = q0 * SB, s1 = min(n, (q0 + nq) * SB), S = s1 - s0;
     const int bs0 = min(SB, S), bs1 = S - bs0;  // rows of sub-blocks 0 and 1
@@ -187,7 +224,7 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
     // ---- every read that does not depend on the super-block's solution is
     // issued first, so a launch waits for memory once, not once per phase:
     // the update slice and, for the first right-hand sides, its rows of W;
-    // the three tiles; this wave's first right-hand side on the super-block.
+    // the three tiles; this wave's right-hand sides on the super-block.
     constexpr int NIT = RPW / 16, NC = TSB * SB / 16;  // row forms
     constexpr int CW = TSB * SB / 4;                   // transposed form
     constexpr bool PRODUCT = NR > 1;
@@ -316,12 +353,24 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
             tile_store(tl[1], v1, vf1);
             tile_store(tl[2], v2, vf0 && vf1);
         }
+        if constexpr (MODE != LOWER_UNIT) {
+            int e = 0;
+#pragma unroll
+            for (int q = 0; q < TPER; ++q) e = min(e, exponent(v0[q]));
+            if (nq > 1) {
+#pragma unroll
+                for (int q = 0; q < TPER; ++q) e = min(e, exponent(v1[q]));
+            }
+            e = wave_min_i32(e);
+            if (lane == 0) s_low[wave] = e;
+        }
         __syncthreads();
 
         // ---- 1. the super-block, redundantly in every workgroup.  The loops run
         // all 64 columns: the staged tiles are zero outside the block and x is
         // zero on lanes beyond it, so the columns past it subtract exact zeros.
         if (wave < nrhs) {
+            const int low = MODE != LOWER_UNIT ? min(min(s_low[0], s_low[1]), min(s_low[2], s_low[3])) : 0;
             T sol[2][NR];
 #pragma unroll
             for (int k = 0; k < NR; ++k) sol[0][k] = sol[1][k] = T(0);
@@ -367,8 +416,17 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
                 }
 #pragma unroll
                 for (int k = 0; k < NR; ++k) {
-                    if (__any(!(fabs(y[k]) < std::numeric_limits<T>::infinity())))
-                        y[k] = sweep_plain<T, MODE>(t, x[k], dl, lane);
+                    const bool wild = !(fabs(y[k]) < std::numeric_limits<T>::infinity());
+                    if constexpr (MODE == LOWER_UNIT) {
+                        if (__any(wild)) y[k] = sweep_plain<T, MODE>(t, x[k], dl, lane);
+                    } else {
+                        using R = Range<T>;
+                        const int ed = exponent(dl);
+                        const bool small = low - ed < R::ENTRY || exponent(y[k]) < R::SOLVED ||
+                                           exponent(x[k]) - ed < R::RHS;
+                        if (__any(wild | small) && (__any(wild) || sweep_lossy<T, MODE>(t, x[k], dl, y[k], lane)))
+                            y[k] = sweep_plain<T, MODE>(t, x[k], dl, lane);
+                    }
                     if (lane >= (second ? bs1 : bs0)) y[k] = T(0);
                     sol[qi][k] = y[k];
                 }
