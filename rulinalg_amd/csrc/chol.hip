@@ -189,8 +189,9 @@ __global__ __launch_bounds__(128) void k_chol_block(T *__restrict__ A, long lda,
 // the 64 columns (about 180 cycles each).  Order 4096: 6.27 -> 2.58 ms for the
 // factorization, order 16384: 49.6 -> 33.2 ms (44 TF).
 
-// s = sqrt(d) and r = 1 / s for d >= epsilon (Goldschmidt's iteration from the
-// hardware's reciprocal square root estimate, then one residual step for s).
+// s = sqrt(d) and r = 1 / s for d >= epsilon (two steps of Goldschmidt's iteration
+// from the hardware's reciprocal square root estimate, then one residual step for
+// s); infinity and 0 for an infinite d, whose column is then zero (div_recip).
 __device__ __forceinline__ void sqrt_recip(double d, double &s, double &r) {
     const double y = __builtin_amdgcn_rsq(d);
     double g = d * y, h = 0.5 * y;
@@ -202,7 +203,7 @@ __device__ __forceinline__ void sqrt_recip(double d, double &s, double &r) {
     }
     s = fma(fma(-g, g, d), h, g);
     s = d == __builtin_inf() ? d : s;
-    r = h + h;
+    r = d == __builtin_inf() ? 0.0 : h + h;
 }
 __device__ __forceinline__ void sqrt_recip(float d, float &s, float &r) {
     s = sqrtf(d);
