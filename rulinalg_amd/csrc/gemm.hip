@@ -1033,6 +1033,9 @@ static int gemm_impl(hipStream_t s, const char *cls, size_t m, size_t n, size_t 
     // a shallow product is bound by its C traffic, and at 128 by one workgroup
     // per CU (133 KB of LDS): FP64 16000 x 64 x 448 takes 37 us there, 29 at 64
     if (shallow && edge > 64) edge = 64;
+    // a launch has fewer than 2^32 threads: products of some 2^29 rows and one
+    // column need the wider tile
+    while (edge < GBM && (uint64_t)ceil_div(m, edge) * ceil_div(n, edge) * GTHREADS >> 32) edge *= 2;
     auto go = [&](auto e, auto tb, auto lo, auto v) {
         gemm_launch<T, decltype(e)::value, decltype(tb)::value, decltype(lo)::value, decltype(v)::value>(
             s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, lds_pad, shallow);
