@@ -68,6 +68,11 @@ struct AuxStream {
 
 // ------------------------------------------------------------------ memory
 
+// Frees every pooled buffer that is not in use (all devices).
+void pool_trim();
+// hipMalloc; where memory is short the pool's buffers are given back first.
+int device_alloc(void **p, size_t n);
+
 // RAII device buffer.
 struct DevBuf {
     void *p = nullptr;
@@ -84,12 +89,7 @@ struct DevBuf {
     int alloc(size_t n) {
         release();
         if (n == 0) n = 256;
-        hipError_t e = hipMalloc(&p, n);
-        if (e != hipSuccess) {
-            p = nullptr;
-            set_error("hipMalloc(%zu) failed: %s", n, hipGetErrorString(e));
-            return e == hipErrorOutOfMemory ? RLG_E_OOM : RLG_E_DEVICE;
-        }
+        RLG_TRY(device_alloc(&p, n));
         bytes = n;
         return RLG_OK;
     }
@@ -111,6 +111,7 @@ struct PoolBuf {
     size_t bytes = 0;
     hipStream_t stream = nullptr;
     int dev = 0;
+    bool operand = false;  // a CallBuf's: kept apart from the others
     PoolBuf() = default;
     PoolBuf(const PoolBuf &) = delete;
     PoolBuf &operator=(const PoolBuf &) = delete;
@@ -125,13 +126,14 @@ struct PoolBuf {
 };
 
 // Operands of one host-pointer call: pooled up to 64 MB (hipMalloc and hipFree
-// took longer than a small product), beyond that allocated and freed.  At the
-// call's end the free list keeps at most 1 GB in buffers of that size; the
-// oldest are freed.
+// took longer than a small product), beyond that allocated and freed.  They take
+// and leave buffers of their own in the pool, at most 1 GB per device of them: at
+// the call's end the oldest that no stream uses any more are freed.
 struct CallBuf {
     static constexpr size_t POOLED = 64u << 20, MOST = 1u << 30;
     PoolBuf pooled;
     DevBuf own;
+    CallBuf() { pooled.operand = true; }
     ~CallBuf();
     int alloc(size_t n, hipStream_t s) { return n <= POOLED ? pooled.alloc(n, s) : own.alloc(n); }
     template <class T> T *as() const { return static_cast<T *>(own.p ? own.p : pooled.p); }
@@ -161,8 +163,6 @@ struct StreamUse {
         return streams;
     }
 };
-// Frees every pooled buffer that is not in use (all devices).
-void pool_trim();
 
 // ------------------------------------------------------------------ profiler
 

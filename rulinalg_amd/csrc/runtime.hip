@@ -148,6 +148,7 @@ struct PoolEntry {
     void *p;
     size_t bytes;
     int dev;
+    bool operand;                   // left by a CallBuf
     std::vector<hipEvent_t> ready;  // every stream that used the buffer
 };
 std::mutex g_pool_mu;
@@ -157,12 +158,37 @@ std::vector<PoolEntry> &pool_entries() {
 }
 }  // namespace
 
+// (not under the pool's lock: it may wait for the streams that used the buffer)
 static void free_entry(PoolEntry &e) {
     for (hipEvent_t ev : e.ready) {
         (void)hipEventSynchronize(ev);
         (void)hipEventDestroy(ev);
     }
     (void)hipFree(e.p);
+}
+
+// Whether every stream that used the buffer is past it.
+static bool idle(const PoolEntry &e) {
+    for (hipEvent_t ev : e.ready)
+        if (hipEventQuery(ev) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+    return true;
+}
+
+int device_alloc(void **p, size_t n) {
+    hipError_t e = hipMalloc(p, n);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // else the next launch would seem to have failed
+        pool_trim();
+        e = hipMalloc(p, n);
+    }
+    if (e == hipSuccess) return RLG_OK;
+    (void)hipGetLastError();
+    *p = nullptr;
+    set_error("hipMalloc(%zu) failed: %s", n, hipGetErrorString(e));
+    return e == hipErrorOutOfMemory ? RLG_E_OOM : RLG_E_DEVICE;
 }
 
 int PoolBuf::alloc(size_t n, hipStream_t s) {
@@ -175,7 +201,7 @@ int PoolBuf::alloc(size_t n, hipStream_t s) {
         auto &v = pool_entries();
         size_t best = v.size();
         for (size_t i = 0; i < v.size(); ++i)
-            if (v[i].dev == dev && v[i].bytes >= n && v[i].bytes <= 2 * n &&
+            if (v[i].dev == dev && v[i].operand == operand && v[i].bytes >= n && v[i].bytes <= 2 * n &&
                 (best == v.size() || v[i].bytes < v[best].bytes))
                 best = i;
         if (best != v.size()) {
@@ -190,17 +216,7 @@ int PoolBuf::alloc(size_t n, hipStream_t s) {
             return RLG_OK;
         }
     }
-    hipError_t e = hipMalloc(&p, n);
-    if (e != hipSuccess) {
-        // give back cached buffers and retry once
-        pool_trim();
-        e = hipMalloc(&p, n);
-    }
-    if (e != hipSuccess) {
-        p = nullptr;
-        set_error("hipMalloc(%zu) failed: %s", n, hipGetErrorString(e));
-        return e == hipErrorOutOfMemory ? RLG_E_OOM : RLG_E_DEVICE;
-    }
+    RLG_TRY(device_alloc(&p, n));
     bytes = n;
     return RLG_OK;
 }
@@ -226,7 +242,7 @@ void PoolBuf::release_after(const std::vector<hipStream_t> &streams) {
         if (s != stream)
             if (hipEvent_t ev = mark(s)) evs.push_back(ev);
     std::lock_guard<std::mutex> lk(g_pool_mu);
-    pool_entries().push_back({p, bytes, dev, std::move(evs)});
+    pool_entries().push_back({p, bytes, dev, operand, std::move(evs)});
     p = nullptr;
     bytes = 0;
 }
@@ -235,23 +251,29 @@ CallBuf::~CallBuf() {
     if (!pooled.p) return;
     pooled.release();
     // sizes that keep growing leave buffers too small to be taken again
-    std::lock_guard<std::mutex> lk(g_pool_mu);
-    auto &v = pool_entries();
-    size_t held = 0;
-    for (auto &e : v) held += e.bytes <= POOLED ? e.bytes : 0;
-    for (size_t i = 0; i < v.size() && held > MOST;) {
-        if (v[i].bytes > POOLED) { ++i; continue; }
-        held -= v[i].bytes;
-        free_entry(v[i]);
-        v.erase(v.begin() + (long)i);
+    std::vector<PoolEntry> surplus;
+    {
+        std::lock_guard<std::mutex> lk(g_pool_mu);
+        auto &v = pool_entries();
+        size_t held = 0;
+        for (auto &e : v) held += e.operand && e.dev == pooled.dev ? e.bytes : 0;
+        for (size_t i = 0; i < v.size() && held > MOST;) {
+            if (!v[i].operand || v[i].dev != pooled.dev || !idle(v[i])) { ++i; continue; }
+            held -= v[i].bytes;
+            surplus.push_back(std::move(v[i]));
+            v.erase(v.begin() + (long)i);
+        }
     }
+    for (auto &e : surplus) free_entry(e);
 }
 
 void pool_trim() {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
-    auto &v = pool_entries();
-    for (auto &e : v) free_entry(e);
-    v.clear();
+    std::vector<PoolEntry> all;
+    {
+        std::lock_guard<std::mutex> lk(g_pool_mu);
+        all.swap(pool_entries());
+    }
+    for (auto &e : all) free_entry(e);
 }
 
 // ------------------------------------------------------------------ host copies
@@ -411,8 +433,7 @@ int rlg_dev_alloc(size_t bytes, void **ptr) {
     Device *d;
     RLG_TRY(current_device(&d));
     *ptr = nullptr;
-    RLG_HIP(hipMalloc(ptr, bytes ? bytes : 256));
-    return RLG_OK;
+    return device_alloc(ptr, bytes ? bytes : 256);
 }
 
 int rlg_dev_free(void *ptr) {
