@@ -77,6 +77,7 @@ int gemm_host(size_t a_rows, size_t a_cols, const T *a, size_t lda, size_t b_row
     hipStream_t s = d->stream;
     const size_t m = a_rows, k = a_cols, n = b_cols;
     CallBuf da, db, dc;
+    HostCall call(s);
     RLG_TRY(da.alloc(m * k * sizeof(T), s));
     RLG_TRY(db.alloc(k * n * sizeof(T), s));
     RLG_TRY(dc.alloc(m * n * sizeof(T), s));
@@ -90,8 +91,7 @@ int gemm_host(size_t a_rows, size_t a_cols, const T *a, size_t lda, size_t b_row
     }
     RLG_TRY(gemm_t<T>(s, m, n, k, T(1), da.as<T>(), k, db.as<T>(), n, T(0), dc.as<T>(), n));
     RLG_TRY(download_matrix<T>(s, c, ldc, dc.as<T>(), n, m, n));
-    RLG_HIP(hipStreamSynchronize(s));
-    return RLG_OK;
+    return call.finish();
 }
 
 // ---------------------------------------------------------------- LU
@@ -332,6 +332,7 @@ int rlg_matvec_f64(size_t m, size_t n, const double *a, size_t lda, size_t v_len
     RLG_TRY(current_device(&d));
     hipStream_t s = d->stream;
     CallBuf da, dv, dy;
+    HostCall call(s);
     RLG_TRY(da.alloc(m * n * 8, s));
     RLG_TRY(dv.alloc(n * 8, s));
     RLG_TRY(dy.alloc(m * 8, s));
@@ -339,8 +340,7 @@ int rlg_matvec_f64(size_t m, size_t n, const double *a, size_t lda, size_t v_len
     RLG_HIP(hipMemcpyAsync(dv.as<double>(), v, n * 8, hipMemcpyHostToDevice, s));
     RLG_TRY(gemv_f64(s, m, n, da.as<double>(), n, dv.as<double>(), dy.as<double>()));
     RLG_HIP(hipMemcpyAsync(y, dy.as<double>(), m * 8, hipMemcpyDeviceToHost, s));
-    RLG_HIP(hipStreamSynchronize(s));
-    return RLG_OK;
+    return call.finish();
 }
 
 // ------------------------------------------------------------------ triangular

@@ -139,6 +139,25 @@ struct CallBuf {
     template <class T> T *as() const { return static_cast<T *>(own.p ? own.p : pooled.p); }
 };
 
+// The end of a host-pointer call: its stream is waited for also where the call ends
+// with an error, since copies from the caller's (pinned) memory may be under way and
+// pooled buffers, other than freed ones, wait for nothing.  Declared behind them.
+struct HostCall {
+    hipStream_t s;
+    bool open = true;
+    explicit HostCall(hipStream_t st) : s(st) {}
+    HostCall(const HostCall &) = delete;
+    HostCall &operator=(const HostCall &) = delete;
+    ~HostCall() {
+        if (open) (void)hipStreamSynchronize(s);
+    }
+    int finish() {
+        open = false;
+        RLG_HIP(hipStreamSynchronize(s));
+        return RLG_OK;
+    }
+};
+
 // Copies between host rows of `width` bytes, `pitch` apart, and a contiguous
 // device buffer.  One linear copy: a 2D copy of pageable memory moves one row at
 // a time, 9 us each (256 rows of 2 KB: 2.4 ms against 25 us).  Rows that are not

@@ -765,6 +765,7 @@ int rlg_solve_mixed_f64(size_t n, const double *a, size_t lda, size_t nrhs, cons
     RLG_TRY(current_device(&d));
     hipStream_t s = d->stream;
     CallBuf da, db, dx;
+    HostCall call(s);
     RLG_TRY(da.alloc(n * n * 8, s));
     RLG_TRY(db.alloc(nrhs * n * 8, s));
     RLG_TRY(dx.alloc(nrhs * n * 8, s));
@@ -774,7 +775,7 @@ int rlg_solve_mixed_f64(size_t n, const double *a, size_t lda, size_t nrhs, cons
                                      n, opts, rep, s);
     if (st != RLG_OK && st != RLG_E_NOT_CONVERGED) return st;
     RLG_TRY(download_rows(s, x, ldx * 8, dx.as<char>(), n * 8, nrhs));
-    RLG_HIP(hipStreamSynchronize(s));
+    RLG_TRY(call.finish());
     return st;
 }
 

@@ -32,6 +32,7 @@ bool g_busy = false;                 // work recorded now does not end until it 
 std::atomic<int> g_stalls{0};        // waits for such work
 std::atomic<int> g_locked_frees{0};  // frees during which the pool could not be used
 std::atomic<bool> g_probe{false};
+bool g_fail_launch = false;
 int g_copies = 0;                    // asynchronous copies that read or write host memory, not yet waited for
 thread_local hipError_t g_last = hipSuccess;
 
@@ -112,14 +113,18 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hip
     if (k != hipMemcpyDeviceToDevice) ++g_copies;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) {
+    return ret(g_fail_launch ? hipErrorInvalidConfiguration : hipSuccess);
+}
 
 }  // extern "C"
 
 namespace {
 
 constexpr size_t MB = 1 << 20;
-std::vector<double> g_a(90 * MB / 8, 1.0), g_v(8192, 1.0), g_y(90 * MB / 8 / 1024);
+std::vector<double> g_a(90 * MB / 8, 1.0), g_v(8192, 1.0), g_y(1 << 17);
 
 int fail(const char *what, double v = 0) {
     std::printf("%s (%g)\n", what, v);
@@ -187,11 +192,31 @@ int shortage() {
     return rlg_dev_free(p);
 }
 
+// A call that fails leaves no copy from the caller's memory under way.
+int drained() {
+    rlg_mixed_opts o;
+    rlg_mixed_opts_default(&o);
+    o.factor_prec = 99;
+    const size_t n = 256;
+    if (rlg_solve_mixed_f64(n, g_a.data(), n, 1, g_v.data(), n, g_y.data(), n, &o, nullptr) != RLG_E_INVALID_ARG)
+        return fail("an unknown precision was accepted");
+    if (g_copies) return fail("copies under way after an invalid option", g_copies);
+    g_fail_launch = true;
+    if (rlg_gemm_f64(n, n, g_a.data(), n, n, n, g_a.data(), n, g_y.data(), n) == RLG_OK) return fail("launch");
+    if (g_copies) return fail("copies under way after a failed product", g_copies);
+    if (rlg_matvec_f64(n, n, g_a.data(), n, n, g_v.data(), g_y.data()) == RLG_OK) return fail("launch");
+    if (g_copies) return fail("copies under way after a failed matrix-vector product", g_copies);
+    g_fail_launch = false;
+    const int st = product(4);
+    return g_copies ? fail("copies under way after a call", g_copies) : st;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     const std::string s = argc > 1 ? argv[1] : "";
-    const int st = s == "bounded" ? bounded() : s == "unblocked" ? unblocked() : s == "shortage" ? shortage() : 2;
+    const int st = s == "bounded" ? bounded() : s == "unblocked" ? unblocked() : s == "shortage" ? shortage()
+                   : s == "drained" ? drained() : 2;
     if (st == 0) std::printf("ok\n");
     std::fflush(stdout);
     std::_Exit(st);
