@@ -79,13 +79,16 @@ struct Smem {
     int piv[32];
     double div[32];
     // LU column step j (buffers by the parity of j): each wave's pivot candidate,
-    // the ranks of its |value| (rank_hi, rank_lo; 0: none), its position and panel
+    // the ranks of its |value| (rank_hi, rank_lo, 0 for none), its position and panel
     // row, and that row from column j on
-    unsigned cand_hi[2][BTH / 64], cand_lo[2][BTH / 64];
-    int cand_p[2][BTH / 64], cand_t[2][BTH / 64];
+    unsigned cand_hi[2][BTH / 64];
+    unsigned cand_lo[2][BTH / 64];
+    int cand_p[2][BTH / 64];
+    int cand_t[2][BTH / 64];
     double cand[2][BTH / 64][32];
     alignas(16) double l11[32 * 32];  // L11 of the panel by columns, for the block row
-    int mdst[64], msrc[64];     // net row moves of a panel's swaps
+    int mdst[64];  // net row moves of a panel's swaps
+    int msrc[64];
     int mcnt;
     int info;
     int item;

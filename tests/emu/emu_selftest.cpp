@@ -7,7 +7,8 @@
 // first wave reaches, while the others wait at the next one), halfwave (a lane read by half of a wave), race (a
 // shared-memory value read without a barrier after thread 0 writes it: the
 // result depends on the lane order), oob (a global write one element past
-// the end of its buffer: the address sanitizer aborts).  ORDER as in
+// the end of its buffer: the address sanitizer aborts), gap (a write past one
+// member of a shared structure that stays inside the structure: likewise).  ORDER as in
 // emu::launch.  Prints the per-thread result checksum on success; exit 2 on
 // an emulation error.
 #include <cstdio>
@@ -15,11 +16,18 @@
 #include <cstring>
 #include <string>
 
+#include "emu_gap.hpp"
 #include "emu_runtime.hpp"
 
 namespace {
 
 int g_case = 0;
+
+struct Members {
+    int first[256];
+    emu::Gap EMU_GAP;
+    int second[256];
+};
 
 void k_selftest(int *out) {
     __shared__ int flag;
@@ -55,6 +63,13 @@ void k_selftest(int *out) {
     case 4:  // one element past the end of `out`
         out[tid + 1] = tid;
         break;
+    case 5: {  // past the first member, within the structure
+        __shared__ Members m;
+        int *const first = m.first;
+        first[tid + (tid == 255 ? 1 : 0)] = m.second[tid] = tid;
+        out[tid] = tid;
+        break;
+    }
     }
 }
 
@@ -64,9 +79,9 @@ void body(void *p) { k_selftest(static_cast<int *>(p)); }
 
 int main(int argc, char **argv) {
     if (argc != 3) return 1;
-    const char *names[] = {"clean", "barrier", "halfwave", "race", "oob"};
+    const char *names[] = {"clean", "barrier", "halfwave", "race", "oob", "gap"};
     g_case = -1;
-    for (int i = 0; i < 5; ++i)
+    for (int i = 0; i < 6; ++i)
         if (!std::strcmp(argv[1], names[i])) g_case = i;
     if (g_case < 0) return 1;
     int *out = static_cast<int *>(std::malloc(256 * sizeof(int)));

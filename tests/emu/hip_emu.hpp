@@ -13,6 +13,12 @@
 // still compute) is reported as an error and ends the run.  Between
 // synchronization points lanes run one after another, in an order the
 // driver chooses, so that results which depend on that order expose a race.
+//
+// Memory: every global buffer is an allocation of its exact size under the address
+// sanitizer.  Shared memory is checked too, member by member (emu_gap.hpp): the
+// hardware drops an LDS instruction's access out of range, but phases that are called
+// functions take the structure by a generic pointer, and a generic access beyond the
+// LDS or scratch limit faults the device (an aperture violation).
 #pragma once
 
 #include <math.h>
