@@ -1036,8 +1036,6 @@ __global__ __launch_bounds__(256) void k_trsm_llu(T *__restrict__ A, long lda, i
 
 // ---------------------------------------------------------------- driver
 
-// Set by lu_factor_lowp for its duration: FP32 panels are then factored with
-// tournament pivoting (tslu.hip) in this workspace.
 // The step between an inner panel and its update, for the other columns of the
 // outer block: the panel's swaps on columns [c0, c1) and [c2, c3), the inverse of
 // its unit-lower block, and the block-row solve B := L^-1 B on the swapped rows
@@ -1214,6 +1212,8 @@ __global__ __launch_bounds__(256) void k_row_step(T *__restrict__ A, long lda, c
         }
 }
 
+// Set by lu_factor_lowp for its duration: FP32 panels are then factored with
+// tournament pivoting (tslu.hip) in this workspace.
 static thread_local void *g_tslu_work = nullptr;
 
 template <class T>

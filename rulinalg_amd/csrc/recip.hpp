@@ -15,10 +15,6 @@ __device__ __forceinline__ double recip(double d) {
     for (int i = 0; i < 2; ++i) y = fma(fma(-d, y, 1.0), y, y);
     return fabs(d) < __builtin_inf() ? y : 0.0;
 }
-__device__ __forceinline__ float recip(float d) {
-    const float y = __builtin_amdgcn_rcpf(d);
-    return fabsf(d) < __builtin_inff() ? fmaf(fmaf(-d, y, 1.0f), y, y) : 0.0f;
-}
 // a / d from r = 1 / d; the correction is left out where the residual is not
 // finite.
 template <class T> __device__ __forceinline__ T div_recip(T a, T d, T r) {

@@ -58,8 +58,10 @@ constexpr int CPW = 64;     // entries updated per workgroup (transposed form)
 
 enum TriMode { LOWER_UNIT = 0, LOWER = 1, UPPER = 2, LOWER_T = 3 };
 
-// a / d from r = 1 / d, with one residual correction (Markstein).
-template <class T> __device__ __forceinline__ T div_recip(T a, T d, T r) {
+// a / d from r = 1 / d, with one residual correction (Markstein).  Unlike div_recip it
+// does not look at the residual: a sub-block with a value that is not finite is swept
+// plainly.
+template <class T> __device__ __forceinline__ T scaled(T a, T d, T r) {
     const T q = a * r;
     return fma(fma(-q, d, a), r, q);
 }
@@ -401,9 +403,9 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
                 if constexpr (MODE != LOWER_UNIT) {
                     const T rd = T(1) / dl;
 #pragma unroll
-                    for (int c = 0; c < SB; ++c) m[c] = div_recip(m[c], dl, rd);
+                    for (int c = 0; c < SB; ++c) m[c] = scaled(m[c], dl, rd);
 #pragma unroll
-                    for (int k = 0; k < NR; ++k) y[k] = div_recip(x[k], dl, rd);
+                    for (int k = 0; k < NR; ++k) y[k] = scaled(x[k], dl, rd);
                 } else {
 #pragma unroll
                     for (int k = 0; k < NR; ++k) y[k] = x[k];

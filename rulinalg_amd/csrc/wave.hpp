@@ -123,11 +123,6 @@ __device__ __forceinline__ int wave_min_i32(int k) {
 
 // Candidate order: larger magnitude first; equal magnitudes go to the lower
 // row index, which reproduces the reference's first-maximum scan.
-template <class T>
-__device__ __forceinline__ bool better(T v2, int i2, T v1, int i1) {
-    // branch-free: the exec-mask branches of an if-chain cost more than the tests
-    return (i2 != INT_MAX) & ((i1 == INT_MAX) | (v2 > v1) | (!(v1 > v2) & (i2 < i1)));
-}
 
 // The high word of a magnitude plus one (a non-negative float orders like its
 // bits); a NaN ranks like zero.
@@ -140,8 +135,8 @@ __device__ __forceinline__ unsigned rank_lo(double v) {
     return (v == v) ? (unsigned)(unsigned long long)__double_as_longlong(v) : 0u;
 }
 
-// The lane that holds the wave's first maximum under `better` (largest
-// |value|, ties to the smallest row index i), or -1 if no lane has a candidate;
+// The lane that holds the wave's first maximum (largest |value|, ties to the
+// smallest row index i), or -1 if no lane has a candidate;
 // uniform.  A lane without one passes hi = 0, else the ranks of its value.  The
 // high words settle it but for near-ties: one 32-bit maximum over the wave, a
 // fused DPP instruction per step, where a 64-bit one takes a compare and two
@@ -152,12 +147,9 @@ __device__ __forceinline__ int first_max_lane(unsigned hi, unsigned lo, int i) {
     const unsigned long long tied = __ballot(hi == mh);
     if (__popcll(tied) == 1) return __ffsll((long long)tied) - 1;
     const unsigned ml = wave_max_u32(hi == mh ? lo : 0u);
-    const int ii = (hi == mh) & (lo == ml) ? i : INT_MAX;
+    const int ii = hi == mh && lo == ml ? i : INT_MAX;
     const int mi = wave_min_i32(ii);
     return __ffsll((long long)__ballot(ii == mi)) - 1;
-}
-template <class T> __device__ __forceinline__ int wave_first_max_lane(T v, int i) {
-    return first_max_lane(i != INT_MAX ? rank_hi(v) : 0u, rank_lo(v), i);
 }
 
 }  // namespace rlg
