@@ -345,7 +345,8 @@ struct rlg_server {
     }
 
     void loop() {
-        (void)hipSetDevice(device);
+        // the library's own device of this thread, which the factorizations go by
+        (void)rlg_set_device(device);
         for (;;) {
             bool busy = false;
             // admit into idle slots

@@ -1,4 +1,5 @@
-// The library's buffer pool under host-pointer calls, without a GPU: the HIP calls
+// The library's buffer pool under host-pointer calls, and the device that the native
+// server's thread works on, without a GPU: the HIP calls
 // that librlgpu makes are defined here (device memory is host memory, kernels do
 // nothing, copies are immediate) and checked (test infrastructure).
 //
@@ -33,6 +34,9 @@ std::atomic<int> g_stalls{0};        // waits for such work
 std::atomic<int> g_locked_frees{0};  // frees during which the pool could not be used
 std::atomic<bool> g_probe{false};
 bool g_fail_launch = false;
+std::atomic<int> g_wrong_device{0};  // work for a stream or memory of another device than the thread's
+int g_want_device = -1;              // the device that allocations are to be on (-1: any)
+thread_local int t_device = 0;
 int g_copies = 0;                    // asynchronous copies that read or write host memory, not yet waited for
 thread_local hipError_t g_last = hipSuccess;
 
@@ -61,9 +65,9 @@ bool pool_is_usable() {
 
 extern "C" {
 
-hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
-hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int *n) { *n = 2; return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = t_device; return hipSuccess; }
+hipError_t hipSetDevice(int d) { t_device = d; return hipSuccess; }
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int) {
     std::memset(p, 0, sizeof *p);
     std::strcpy(p->gcnArchName, "gfx950");
@@ -77,6 +81,7 @@ hipError_t hipGetLastError(void) {
     return e;
 }
 hipError_t hipMalloc(void **p, size_t n) {
+    if (g_want_device >= 0 && t_device != g_want_device) ++g_wrong_device;
     std::lock_guard<std::mutex> lk(g_mu);
     if (g_held + n > g_limit) return ret(hipErrorOutOfMemory);
     *p = std::malloc(n);
@@ -95,7 +100,7 @@ hipError_t hipFree(void *p) {
     std::free(p);
     return hipSuccess;
 }
-hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = reinterpret_cast<hipStream_t>(new int(0)); return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = reinterpret_cast<hipStream_t>(new int(t_device)); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { g_copies = 0; return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
@@ -113,7 +118,16 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hip
     if (k != hipMemcpyDeviceToDevice) ++g_copies;
     return hipSuccess;
 }
-hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t) {
+    for (size_t i = 0; i < h; ++i) std::memcpy(static_cast<char *>(d) + i * dp, static_cast<const char *>(s) + i * sp, w);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = std::malloc(n); return hipSuccess; }
+hipError_t hipHostFree(void *p) { std::free(p); return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t s) {
+    if (t_device != *reinterpret_cast<int *>(s)) ++g_wrong_device;
+    return hipSuccess;
+}
 hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
 hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) {
     return ret(g_fail_launch ? hipErrorInvalidConfiguration : hipSuccess);
@@ -211,12 +225,36 @@ int drained() {
     return g_copies ? fail("copies under way after a call", g_copies) : st;
 }
 
+// The server's own thread stays on the device that the server was created on.
+int server() {
+    setenv("RLG_ENABLE_SERVER", "1", 1);
+    if (rlg_set_device(1) != RLG_OK) return fail("rlg_set_device");
+    rlg_server *s = nullptr;
+    if (rlg_server_create(nullptr, &s) != RLG_OK) return fail(rlg_last_error_message());
+    g_want_device = 1;
+    for (int i = 0; i < 4; ++i) {
+        rlg_request q{};
+        rlg_result r{};
+        int64_t t = 0;
+        q.kind = i % 2 ? RLG_KIND_LU : RLG_KIND_CHOL;
+        q.n = 150 + i;
+        q.nrhs = 2;
+        q.a = g_a.data();
+        q.b = g_v.data();
+        // (the kernels do nothing, so a request may well fail)
+        if (rlg_server_submit(s, &q, &t) != RLG_OK || rlg_server_wait(s, t, &r) != RLG_OK) return fail("request");
+        rlg_server_release(s, t);
+    }
+    rlg_server_destroy(s);
+    return g_wrong_device ? fail("launches or allocations on another device", g_wrong_device) : 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     const std::string s = argc > 1 ? argv[1] : "";
     const int st = s == "bounded" ? bounded() : s == "unblocked" ? unblocked() : s == "shortage" ? shortage()
-                   : s == "drained" ? drained() : 2;
+                   : s == "drained" ? drained() : s == "server" ? server() : 2;
     if (st == 0) std::printf("ok\n");
     std::fflush(stdout);
     std::_Exit(st);
