@@ -224,12 +224,12 @@ __device__ __attribute__((noinline)) int lu_fused(T *__restrict__ A, int n, T *_
             const int par = j & 1;
             // this thread's candidate
             T av = fabs(x[0][0]);
-            unsigned hi = pos[0] >= j ? rank_hi(av) : 0u, lo = rank_lo(av);
+            unsigned hi = pos[0] >= j ? rank_hi(av, pos[0] == j) : 0u, lo = rank_lo(av);
             int bp = pos[0], bt = tid;
             bool second = false;
             if (RQ == 2) {
                 const T a1 = fabs(x[RQ - 1][0]);
-                const unsigned h1 = pos[RQ - 1] >= j ? rank_hi(a1) : 0u, l1 = rank_lo(a1);
+                const unsigned h1 = pos[RQ - 1] >= j ? rank_hi(a1, pos[RQ - 1] == j) : 0u, l1 = rank_lo(a1);
                 second = (h1 > hi) | ((h1 == hi) & ((l1 > lo) | ((l1 == lo) & (pos[RQ - 1] < bp))));
                 hi = second ? h1 : hi;
                 lo = second ? l1 : lo;

@@ -288,7 +288,7 @@ __global__ __launch_bounds__(PanelRows<T>::value) void k_lu_panel(
         for (int j = cb; j < min(cb + SPW, w); ++j) {
             const int c = j - cb, par = j & 1;
             const T av = fabs(x[0]);
-            const unsigned hi = pos >= j ? rank_hi(av) : 0u, lo = rank_lo(av);
+            const unsigned hi = pos >= j ? rank_hi(av, pos == j) : 0u, lo = rank_lo(av);
             const int wl = first_max_lane(hi, lo, pos);
             if (lane == max(wl, 0)) {
                 red[par][wave] = uint4{wl < 0 ? 0u : hi, lo, (unsigned)pos, (unsigned)tid};
@@ -629,7 +629,7 @@ __device__ __forceinline__ void one_factor(OneShared<R> &sh, int cb, int w, int 
         unsigned key[R], d = 0u;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            key[r] = bit_of(act[r], rank_hi(fabs(x[r][c])), 0u);
+            key[r] = bit_of(act[r], rank_hi(fabs(x[r][c]), pos[r] == j), 0u);
             d = max(d, key[r]);
         }
         double y[SPW];  // the entries of this lane's best row, its number and position

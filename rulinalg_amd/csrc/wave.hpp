@@ -122,13 +122,17 @@ __device__ __forceinline__ int wave_min_i32(int k) {
 // ---------------------------------------------------------------- pivot search
 
 // Candidate order: larger magnitude first; equal magnitudes go to the lower
-// row index, which reproduces the reference's first-maximum scan.
+// row index.  That is the reference's scan from the diagonal down, which takes a row
+// only if it is larger than the best before it: a NaN is never taken, and one on the
+// diagonal never given up.
 
 // The high word of a magnitude plus one (a non-negative float orders like its
-// bits); a NaN ranks like zero.
-__device__ __forceinline__ unsigned rank_hi(float v) { return (v == v) ? __float_as_uint(v) + 1 : 1u; }
-__device__ __forceinline__ unsigned rank_hi(double v) {
-    return (v == v) ? (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) + 1 : 1u;
+// bits); a NaN ranks like zero, and first of all in the diagonal's row.
+__device__ __forceinline__ unsigned rank_hi(float v, bool diagonal) {
+    return (v == v) ? __float_as_uint(v) + 1 : diagonal ? ~0u : 1u;
+}
+__device__ __forceinline__ unsigned rank_hi(double v, bool diagonal) {
+    return (v == v) ? (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) + 1 : diagonal ? ~0u : 1u;
 }
 __device__ __forceinline__ unsigned rank_lo(float) { return 0u; }
 __device__ __forceinline__ unsigned rank_lo(double v) {
