@@ -37,8 +37,8 @@
 // right-hand sides 56 -> 17.9 and 39.5 -> 17.2 us.
 //
 // The loads come next: with a test and a 64-bit product per load, a wave spends
-// some 500 instructions before the first barrier.  Whole blocks and rows load
-// without tests, from addresses a scalar apart: solves of order 4096 4 % faster
+// some 500 instructions before the first barrier.  So no load has a test, and those
+// of a whole block are a constant or a scalar apart: solves of order 4096 4 % faster
 // (LU 541 -> 520 us, 16 right-hand sides 1,017 -> 980; Cholesky 588 -> 567).
 // Taking four entries at a time from the lanes, and their solution redundantly in
 // each, is slower (541 -> 594 us): the chain is bound by instructions issued.
@@ -183,7 +183,7 @@ __device__ __forceinline__ int exponent(float v) { return __builtin_amdgcn_frexp
 // multiple of the smallest subnormal number show in it (LOW): neither the entries
 // that are not zero, nor the products whose sum could have come out as zero.
 // ENTRY, SOLVED and RHS are bounds on the three kinds of exponent that together
-// imply both.  (They cost 1 % of a solve of order 4096, 562 to 569 us.)
+// imply both.  (They cost 1 % of a solve of order 4096, 541 to 546 us.)
 template <class T> struct Range;
 template <> struct Range<double> {
     static constexpr int NORMAL = -1021, LOW = -1009, ENTRY = -500, SOLVED = -500, RHS = -1000;
@@ -237,16 +237,21 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
     // product form: the wave's 16 rows (row ls of them per lane), the lane's
     // columns 4 VL u + VL grp + e, and the W entries of its accumulator
     const int jp = u0 + (int)blockIdx.x * RPW + wave * 16;
-    // full block and rows: no test per load, and row addresses a scalar apart
-    static_assert(RPW == CPW, "one test for both forms");
-    const bool full = S == TSB * SB && u0 + ((int)blockIdx.x + 1) * RPW <= u1;
+    // No test per load: rows past u1 read row u1 - 1 (their sums are not stored), and
+    // with a block of fewer than 128 columns those past it read its last column and
+    // count as zero.  (Tested one by one they were waited for one by one: the last
+    // workgroup of a launch, if its rows are not 64, then took 13 us where the others
+    // took 7.)
+    const bool rows = u1 > u0, whole = S == TSB * SB;
+    const auto row_of = [&](int j) __attribute__((always_inline)) { return (long)min(j, u1 - 1); };
     T mv[PRODUCT ? CW : MODE == LOWER_T ? CW : NIT * NC];
     T wpre[PRODUCT ? 1 : RDOT][PRODUCT ? 4 : MODE == LOWER_T ? 1 : NIT];
     if constexpr (PRODUCT) {
         typedef T vT __attribute__((ext_vector_type(VL)));
-        const int j = jp + ls;
-        if (full && (vec || MODE == LOWER_T)) {
-            const T *p = MODE == LOWER_T ? M + (long)(s0 + grp * VL) * lda + j : M + (long)j * lda + s0 + grp * VL;
+        const long j = row_of(jp + ls);
+        const T *const mrow = MODE == LOWER_T ? M + (long)s0 * lda + j : M + j * lda + s0;
+        if (rows && whole && (vec || MODE == LOWER_T)) {
+            const T *const p = MODE == LOWER_T ? mrow + (long)(grp * VL) * lda : mrow + grp * VL;
 #pragma unroll
             for (int u = 0; u < CW / VL; ++u) {
                 if constexpr (MODE == LOWER_T) {
@@ -258,75 +263,68 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
                     for (int e = 0; e < VL; ++e) mv[u * VL + e] = x[e];
                 }
             }
-        } else {
+        } else if (rows && whole) {
 #pragma unroll
-            for (int u = 0; u < CW / VL; ++u) {
-                const int c = (4 * u + grp) * VL;
-                if (MODE != LOWER_T && vec && c + VL <= S) {
-                    const vT x = j < u1 ? *reinterpret_cast<const vT *>(M + (long)j * lda + s0 + c) : vT(T(0));
+            for (int i = 0; i < CW; ++i) mv[i] = mrow[(4 * (i / VL) + grp) * VL + i % VL];
+        } else if (rows) {
 #pragma unroll
-                    for (int e = 0; e < VL; ++e) mv[u * VL + e] = x[e];
-                } else {
+            for (int i = 0; i < CW; ++i) {
+                const int c = (4 * (i / VL) + grp) * VL + i % VL;
+                const T v = mrow[MODE == LOWER_T ? (long)min(c, S - 1) * lda : (long)min(c, S - 1)];
+                mv[i] = c < S ? v : T(0);
+            }
+        }
+        if (rows) {  // (lanes past nrhs: the last vector's, not stored)
 #pragma unroll
-                    for (int e = 0; e < VL; ++e)
-                        mv[u * VL + e] =
-                            j < u1 && c + e < S
-                                ? M[MODE == LOWER_T ? (long)(s0 + c + e) * lda + j : (long)j * lda + s0 + c + e]
-                                : T(0);
+            for (int q = 0; q < 4; ++q) wpre[0][q] = W[(long)min(ls, nrhs - 1) * ldw + row_of(jp + Mfma<T>::row(grp, q))];
+        }
+    } else if constexpr (MODE == LOWER_T) {
+        if (rows) {
+            const T *const p = M + (long)(s0 + wave * CW) * lda + row_of(jt);
+            if (whole) {
+#pragma unroll
+                for (int q = 0; q < CW; ++q) mv[q] = p[q * lda];
+            } else {
+#pragma unroll
+                for (int q = 0; q < CW; ++q) {
+                    const int c = wave * CW + q;
+                    const T v = p[(long)(min(c, S - 1) - wave * CW) * lda];
+                    mv[q] = c < S ? v : T(0);
+                }
+            }
+            if (wave == 0) {
+#pragma unroll
+                for (int r = 0; r < RDOT; ++r) {
+                    if (r >= nrhs) break;
+                    wpre[r][0] = W[(long)r * ldw + row_of(jt)];
                 }
             }
         }
+    } else if (rows) {
+        const T *p[NIT];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int jw = jp + Mfma<T>::row(grp, q);
-            wpre[0][q] = jw < u1 && ls < nrhs ? W[(long)ls * ldw + jw] : T(0);
-        }
-    } else if constexpr (MODE == LOWER_T) {
-        const bool act = jt < u1;
-        if (full) {
-            const T *p = M + (long)(s0 + wave * CW) * lda + jt;
+        for (int it = 0; it < NIT; ++it) p[it] = M + row_of(rbase + it * 4) * lda + s0;
+        if (whole) {
 #pragma unroll
-            for (int q = 0; q < CW; ++q) mv[q] = p[q * lda];
+            for (int it = 0; it < NIT; ++it)
+#pragma unroll
+                for (int k = 0; k < NC; ++k) mv[it * NC + k] = p[it][ls + 16 * k];
         } else {
 #pragma unroll
-            for (int q = 0; q < CW; ++q) {
-                const int c = wave * CW + q;
-                mv[q] = (act && c < S) ? M[(long)(s0 + c) * lda + jt] : T(0);
-            }
+            for (int it = 0; it < NIT; ++it)
+#pragma unroll
+                for (int k = 0; k < NC; ++k) {
+                    const int c = ls + 16 * k;
+                    const T v = p[it][min(c, S - 1)];
+                    mv[it * NC + k] = c < S ? v : T(0);
+                }
         }
-#pragma unroll
-        for (int r = 0; r < RDOT; ++r)
-            wpre[r][0] = (wave == 0 && act && r < nrhs) ? W[(long)r * ldw + jt] : T(0);
-    } else if (full) {
-        const T *p = M + (long)rbase * lda + s0 + ls, *wp = W + rbase;
-#pragma unroll
-        for (int it = 0; it < NIT; ++it)
-#pragma unroll
-            for (int k = 0; k < NC; ++k) mv[it * NC + k] = p[it * (4 * lda) + 16 * k];
 #pragma unroll
         for (int r = 0; r < RDOT; ++r) {
             if (r >= nrhs) break;
 #pragma unroll
-            for (int it = 0; it < NIT; ++it) wpre[r][it] = wp[r * ldw + it * 4];
+            for (int it = 0; it < NIT; ++it) wpre[r][it] = W[(long)r * ldw + row_of(rbase + it * 4)];
         }
-    } else {
-#pragma unroll
-        for (int it = 0; it < NIT; ++it) {
-            const int j = rbase + it * 4;
-            const T *mrow = M + (long)j * lda + s0;
-#pragma unroll
-            for (int k = 0; k < NC; ++k) {
-                const int c = ls + 16 * k;
-                mv[it * NC + k] = (j < u1 && c < S) ? mrow[c] : T(0);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < RDOT; ++r)
-#pragma unroll
-            for (int it = 0; it < NIT; ++it) {
-                const int j = rbase + it * 4;
-                wpre[r][it] = (ls == 0 && j < u1 && r < nrhs) ? W[(long)r * ldw + j] : T(0);
-            }
     }
     {
         T v0[TPER], v1[TPER], v2[TPER];
@@ -416,19 +414,27 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
 #pragma unroll
                     for (int k = 0; k < NR; ++k) y[k] = fma(-m[c], lane_get(y[k], c), y[k]);
                 }
+                // one test for all of them: a branch costs as much as 30 instructions
+                const auto wild = [](T v) __attribute__((always_inline)) {
+                    return !(fabs(v) < std::numeric_limits<T>::infinity());
+                };
+                bool odd = false;
 #pragma unroll
                 for (int k = 0; k < NR; ++k) {
-                    const bool wild = !(fabs(y[k]) < std::numeric_limits<T>::infinity());
-                    if constexpr (MODE == LOWER_UNIT) {
-                        if (__any(wild)) y[k] = sweep_plain<T, MODE>(t, x[k], dl, lane);
-                    } else {
-                        using R = Range<T>;
-                        const int ed = exponent(dl);
-                        const bool small = low - ed < R::ENTRY || exponent(y[k]) < R::SOLVED ||
-                                           exponent(x[k]) - ed < R::RHS;
-                        if (__any(wild | small) && (__any(wild) || sweep_lossy<T, MODE>(t, x[k], dl, y[k], lane)))
+                    odd |= wild(y[k]);
+                    if constexpr (MODE != LOWER_UNIT)
+                        odd |= (exponent(y[k]) < Range<T>::SOLVED) | (exponent(x[k]) - exponent(dl) < Range<T>::RHS);
+                }
+                if constexpr (MODE != LOWER_UNIT) odd |= low - exponent(dl) < Range<T>::ENTRY;
+                if (__any(odd)) {
+#pragma unroll
+                    for (int k = 0; k < NR; ++k)
+                        if (__any(wild(y[k])) ||
+                            (MODE != LOWER_UNIT && sweep_lossy<T, MODE>(t, x[k], dl, y[k], lane)))
                             y[k] = sweep_plain<T, MODE>(t, x[k], dl, lane);
-                    }
+                }
+#pragma unroll
+                for (int k = 0; k < NR; ++k) {
                     if (lane >= (second ? bs1 : bs0)) y[k] = T(0);
                     sol[qi][k] = y[k];
                 }
@@ -450,6 +456,7 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
             for (int c = lane; c < S; c += 64) X[(long)r * ldx + s0 + c] = xs[r][c];
 
     // ---- 2. remove the solved rows from this workgroup's share of [u0, u1)
+    if (!rows) return;
     if constexpr (PRODUCT) {
         // four sums of 32 products each: one of 128 gave a solution of order 4096
         // 1.5 times the backward error
