@@ -172,14 +172,18 @@ __device__ __forceinline__ void panel_moves(int kb, const int *piv, int *mdst, i
 // ---------------------------------------------------------------- LU
 
 // (The phases stay called functions: with all of them forced inline, and their
-// registers spilled, the kernel faulted the GPU, for a cause not shown.)
-//
+// registers spilled, the kernel faulted the GPU, for a cause not shown.  Not marked
+// as tail calls, they need not save the registers that their caller does not use:
+// saved, up to 340 per thread went to scratch memory and back at every call, and 512
+// systems of order 1 (plain LU) took 41 us where they now take 18.)
+#define PHASE __attribute__((noinline, not_tail_called))
+
 // Factor the n x n matrix A (ld = n, type T) in place with RHS vectors B
 // (nrhs x n, may be null) carried along as extra columns, so that on return
 // B holds L^-1 P B.  Pivots go to piv_out[0..n).  Returns the first failing
 // step or n.
 template <class T, int NB>
-__device__ __attribute__((noinline)) int lu_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs,
+__device__ PHASE int lu_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs,
                         int64_t *__restrict__ piv_out, Smem &sm) {
     T *P = reinterpret_cast<T *>(sm.panel);
     constexpr int LD = NB + 1;
@@ -559,14 +563,22 @@ __device__ __attribute__((noinline)) void tri_solve(const T *__restrict__ A, int
         const int cnt = hi - lo;
         for (int q = tid; q < cnt * nrhs; q += BTH) {
             const int r = q / cnt, i = lo + (q - r * cnt);
-            T av[TB];
+            T av[TB], s;
+            if (bs == TB) {  // no branch per entry
 #pragma unroll
-            for (int c = 0; c < TB; ++c)
-                if (c < bs) av[c] = MODE == TS_LOWER_T ? A[(long)(b0 + c) * n + i] : A[(long)i * n + b0 + c];
-            T s = X[(long)r * n + i];
+                for (int c = 0; c < TB; ++c) av[c] = MODE == TS_LOWER_T ? A[(long)(b0 + c) * n + i] : A[(long)i * n + b0 + c];
+                s = X[(long)r * n + i];
 #pragma unroll
-            for (int c = 0; c < TB; ++c)
-                if (c < bs) s = s - av[c] * XB[r * TB + c];
+                for (int c = 0; c < TB; ++c) s = s - av[c] * XB[r * TB + c];
+            } else {
+#pragma unroll
+                for (int c = 0; c < TB; ++c)
+                    if (c < bs) av[c] = MODE == TS_LOWER_T ? A[(long)(b0 + c) * n + i] : A[(long)i * n + b0 + c];
+                s = X[(long)r * n + i];
+#pragma unroll
+                for (int c = 0; c < TB; ++c)
+                    if (c < bs) s = s - av[c] * XB[r * TB + c];
+            }
             X[(long)r * n + i] = s;
         }
         __syncthreads();
@@ -578,7 +590,7 @@ __device__ __attribute__((noinline)) void tri_solve(const T *__restrict__ A, int
 // Left-looking Cholesky of A in place (lower triangle), RHS forward-solved
 // along the way (B := L^-1 B).  Returns the first failing column or n.
 template <class T, int NB>
-__device__ __attribute__((noinline)) int chol_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs, Smem &sm) {
+__device__ PHASE int chol_fused(T *__restrict__ A, int n, T *__restrict__ B, int nrhs, Smem &sm) {
     T *P = reinterpret_cast<T *>(sm.panel);
     constexpr int LD = NB + 1;
     // (arguments of a called function count as different in every lane: the
@@ -832,6 +844,190 @@ __device__ __forceinline__ double wave_max_f64(double v) {
     return fmax(fmax(lane_get(v, 0), lane_get(v, 16)), fmax(lane_get(v, 32), lane_get(v, 48)));
 }
 
+// A pointer argument of a called function, known to be the same in every lane.
+template <class P> __device__ __forceinline__ P *uniform_ptr(P *p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    const uint64_t lo = (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+    const uint64_t hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32));
+    return reinterpret_cast<P *>(hi << 32 | lo);
+}
+
+// The FP32 copy of A (eight loads in flight); returns ||A||inf, one row per wave.
+__device__ PHASE double mixed_start(const double *A, int n, float *a32, Smem &sm) {
+    A = uniform_ptr(A);
+    a32 = uniform_ptr(a32);
+    n = __builtin_amdgcn_readfirstlane(n);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int e0 = tid; e0 < n * n; e0 += 8 * BTH) {
+        double v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = e0 + q * BTH < n * n ? A[e0 + q * BTH] : 0.0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (e0 + q * BTH < n * n) a32[e0 + q * BTH] = (float)v[q];
+    }
+    // four rows per wave step, so four rows' loads are in flight at once
+    double rs = 0.0;
+    for (int i0 = 4 * wave; i0 < n; i0 += 4 * BNW) {
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int j = lane; j < n; j += 64) {
+            double a[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[q] = i0 + q < n ? A[(long)(i0 + q) * n + j] : 0.0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) s[q] += fabs(a[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i0 + q < n) rs = fmax(rs, wave_sum_f64(s[q]));
+    }
+    if (lane == 0) sm.red_v[wave] = rs;
+    __syncthreads();
+    double anorm = sm.red_v[0];
+#pragma unroll
+    for (int q = 1; q < BNW; ++q) anorm = fmax(anorm, sm.red_v[q]);
+    __syncthreads();
+    return anorm;
+}
+
+// Refines all right-hand sides together with the FP32 factor in ms.a32: the
+// solutions to ms.x.  Returns whether every backward error reached tol (the same in
+// every thread); a vector that stops halving its error fails the system.
+__device__ PHASE bool mixed_refine(int kind, int n, int nrhs, const double *A, const double *b, char *slot,
+                                   double anorm, int info, int max_iter, double tol, Smem &sm) {
+    kind = __builtin_amdgcn_readfirstlane(kind);
+    n = __builtin_amdgcn_readfirstlane(n);
+    nrhs = __builtin_amdgcn_readfirstlane(nrhs);
+    max_iter = __builtin_amdgcn_readfirstlane(max_iter);
+    A = uniform_ptr(A);
+    b = uniform_ptr(b);
+    const MixedSlot ms = slot_of(uniform_ptr(slot), 0);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // per-vector norms and convergence state in the panel buffer past
+    // what the triangular solves (first 1568 doubles) and the row map use
+    double *bmax = sm.panel + 6144, *xmax = bmax + BMAXR, *rmax = xmax + BMAXR;  // rmax[BNW][BMAXR]
+    double *etab = rmax + BNW * BMAXR;                                            // etab[2][BMAXR]
+    // row permutation of the FP32 factor: raw[k] = original row at k
+    int *raw = reinterpret_cast<int *>(sm.panel + 4096);
+    if (tid == 0 && kind == RLG_KIND_LU && info == n) {
+        for (int i = 0; i < n; ++i) raw[i] = i;
+        for (int k = 0; k < n; ++k) {
+            const int p = (int)ms.piv[k];
+            if (p != k) { const int t = raw[k]; raw[k] = raw[p]; raw[p] = t; }
+        }
+    }
+    // refinement of all right-hand sides together: x = 0, r = b, |b|
+    double *X = ms.x, *R = ms.res;
+    float *D = ms.d32;
+    for (int r = wave; r < nrhs; r += BNW) {
+        double bm = 0.0;
+        for (int i = lane; i < n; i += 64) {
+            const double bv = b[(long)r * n + i];
+            X[(long)r * n + i] = 0.0;
+            R[(long)r * n + i] = bv;
+            bm = fmax(bm, fabs(bv));
+        }
+        bm = wave_max_f64(bm);
+        if (lane == 0) bmax[r] = bm;
+    }
+    __syncthreads();
+    // done: vectors whose backward error reached tol (the same bits in every thread)
+    unsigned done = 0u;
+    const unsigned all = nrhs >= 32 ? ~0u : (1u << nrhs) - 1u;
+    bool stalled = info != n;
+    for (int itn = 0; itn < max_iter && !stalled && done != all; ++itn) {
+        for (int e = tid; e < nrhs * n; e += BTH) {
+            const int r = e / n, i = e - r * n;
+            const int src = kind == RLG_KIND_LU ? raw[i] : i;
+            D[e] = (done >> r) & 1u ? 0.f : (float)R[(long)r * n + src];
+        }
+        __syncthreads();
+        if (kind == RLG_KIND_LU) {
+            tri_solve<float, TS_LOWER_UNIT>(ms.a32, n, D, nrhs, sm);
+            tri_solve<float, TS_UPPER>(ms.a32, n, D, nrhs, sm);
+        } else {
+            tri_solve<float, TS_LOWER>(ms.a32, n, D, nrhs, sm);
+            tri_solve<float, TS_LOWER_T>(ms.a32, n, D, nrhs, sm);
+        }
+        // x += d and |x|, one vector per wave
+        for (int r = wave; r < nrhs; r += BNW) {
+            if ((done >> r) & 1u) continue;
+            double xm = 0.0;
+            for (int i = lane; i < n; i += 64) {
+                const double v = X[(long)r * n + i] + (double)D[(long)r * n + i];
+                X[(long)r * n + i] = v;
+                xm = fmax(xm, fabs(v));
+            }
+            xm = wave_max_f64(xm);
+            if (lane == 0) xmax[r] = xm;
+        }
+        __syncthreads();
+        // r = b - A x in FP64: a wave takes four rows and four vectors per
+        // pass over the rows (lanes across the row), so four rows' loads
+        // are in flight at once; |r| per vector kept in the wave's own LDS
+        // slots.  Each (row, vector) sum keeps one fixed order.
+        if (lane == 0) {
+#pragma unroll
+            for (int r = 0; r < BMAXR; ++r) rmax[wave * BMAXR + r] = 0.0;
+        }
+        for (int i0 = 4 * wave; i0 < n; i0 += 4 * BNW) {
+            for (int rb = 0; rb < nrhs; rb += 4) {
+                double acc[4][4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) acc[u][q] = 0.0;
+                for (int j = lane; j < n; j += 64) {
+                    double a[4], xv[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) a[u] = i0 + u < n ? A[(long)(i0 + u) * n + j] : 0.0;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) xv[q] = rb + q < nrhs ? X[(long)(rb + q) * n + j] : 0.0;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) acc[u][q] += a[u] * xv[q];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        if (i0 + u < n && rb + q < nrhs) {
+                            const int i = i0 + u, r = rb + q;
+                            const double res = b[(long)r * n + i] - wave_sum_f64(acc[u][q]);
+                            if (lane == 0) {
+                                R[(long)r * n + i] = res;
+                                rmax[wave * BMAXR + r] = fmax(rmax[wave * BMAXR + r], fabs(res));
+                            }
+                        }
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        // every thread takes the same decisions; the errors of this step
+        // go to etab[itn & 1], the previous step's are read from the other
+        for (int r = 0; r < nrhs; ++r) {
+            if ((done >> r) & 1u) continue;
+            double rn = rmax[r];
+#pragma unroll
+            for (int q = 1; q < BNW; ++q) rn = fmax(rn, rmax[q * BMAXR + r]);
+            const double den = anorm * xmax[r] + bmax[r];
+            const double eta = den > 0 ? rn / den : 0.0;
+            if (eta <= tol) {
+                done |= 1u << r;
+            } else if (itn >= 1 && !(eta <= 0.5 * etab[((itn + 1) & 1) * BMAXR + r])) {
+                stalled = true;
+            }
+            if (tid == 0) etab[(itn & 1) * BMAXR + r] = eta;
+        }
+        __syncthreads();
+    }
+    return !stalled && done == all;
+}
+
+// Between the phases the kernel keeps a few uniform values only: with the refinement
+// in it, what it kept in registers across a call was spilled, or saved by the phase.
 __global__ __launch_bounds__(BTH) void k_batch_mixed(rlg_batch_item *__restrict__ items,
                                                      const int *__restrict__ order,
                                                      const unsigned char *__restrict__ nbs, int count,
@@ -839,7 +1035,8 @@ __global__ __launch_bounds__(BTH) void k_batch_mixed(rlg_batch_item *__restrict_
                                                      int max_iter, double tol,
                                                      unsigned *__restrict__ fallbacks) {
     __shared__ Smem sm;
-    const MixedSlot ms = slot_of(ws, blockIdx.x);
+    char *const slot = ws + (size_t)blockIdx.x * SLOT_BYTES;
+    const MixedSlot ms = slot_of(slot, 0);
     const int tid = threadIdx.x;
     for (;;) {
         if (tid == 0) sm.item = (int)atomicAdd(counter, 1u);
@@ -850,43 +1047,7 @@ __global__ __launch_bounds__(BTH) void k_batch_mixed(rlg_batch_item *__restrict_
         const int id = order[idx];
         rlg_batch_item it = items[id];
         const int n = it.n, nrhs = it.nrhs;
-        const double *A = it.a;
-        const int lane = tid & 63, wave = tid >> 6;
-        // per-vector norms and convergence state in the panel buffer past
-        // what the triangular solves (first 1568 doubles) and the row map use
-        double *bmax = sm.panel + 6144, *xmax = bmax + BMAXR, *rmax = xmax + BMAXR;  // rmax[BNW][BMAXR]
-        double *etab = rmax + BNW * BMAXR;                                            // etab[2][BMAXR]
-        // FP32 copy (eight loads in flight), ||A||inf one row per wave
-        for (int e0 = tid; e0 < n * n; e0 += 8 * BTH) {
-            double v[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) v[q] = e0 + q * BTH < n * n ? A[e0 + q * BTH] : 0.0;
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-                if (e0 + q * BTH < n * n) ms.a32[e0 + q * BTH] = (float)v[q];
-        }
-        {   // four rows per wave step, so four rows' loads are in flight at once
-            double rs = 0.0;
-            for (int i0 = 4 * wave; i0 < n; i0 += 4 * BNW) {
-                double s[4] = {0.0, 0.0, 0.0, 0.0};
-                for (int j = lane; j < n; j += 64) {
-                    double a[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) a[q] = i0 + q < n ? A[(long)(i0 + q) * n + j] : 0.0;
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) s[q] += fabs(a[q]);
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (i0 + q < n) rs = fmax(rs, wave_sum_f64(s[q]));
-            }
-            if (lane == 0) sm.red_v[wave] = rs;
-        }
-        __syncthreads();
-        double anorm = sm.red_v[0];
-#pragma unroll
-        for (int q = 1; q < BNW; ++q) anorm = fmax(anorm, sm.red_v[q]);
-        __syncthreads();
+        const double anorm = mixed_start(it.a, n, ms.a32, sm);
         int info;
         if (it.kind == RLG_KIND_LU) {
             const int nb = nbs[id];
@@ -899,130 +1060,13 @@ __global__ __launch_bounds__(BTH) void k_batch_mixed(rlg_batch_item *__restrict_
             else if (nb == 32) info = chol_fused<float, 32>(ms.a32, n, nullptr, 0, sm);
             else info = chol_fused<float, 16>(ms.a32, n, nullptr, 0, sm);
         }
-        // row permutation of the FP32 factor: raw[k] = original row at k
-        int *raw = reinterpret_cast<int *>(sm.panel + 4096);
-        if (tid == 0 && it.kind == RLG_KIND_LU && info == n) {
-            for (int i = 0; i < n; ++i) raw[i] = i;
-            for (int k = 0; k < n; ++k) {
-                const int p = (int)ms.piv[k];
-                if (p != k) { const int t = raw[k]; raw[k] = raw[p]; raw[p] = t; }
-            }
-        }
-        // refinement of all right-hand sides together: x = 0, r = b, |b|
-        double *X = ms.x, *R = ms.res;
-        float *D = ms.d32;
-        for (int r = wave; r < nrhs; r += BNW) {
-            double bm = 0.0;
-            for (int i = lane; i < n; i += 64) {
-                const double bv = it.b[(long)r * n + i];
-                X[(long)r * n + i] = 0.0;
-                R[(long)r * n + i] = bv;
-                bm = fmax(bm, fabs(bv));
-            }
-            bm = wave_max_f64(bm);
-            if (lane == 0) bmax[r] = bm;
-        }
-        __syncthreads();
-        // done: vectors whose backward error reached tol (the same bits in
-        // every thread); a vector that stops halving its error fails the system
-        unsigned done = 0u;
-        const unsigned all = nrhs >= 32 ? ~0u : (1u << nrhs) - 1u;
-        bool stalled = info != n;
-        for (int itn = 0; itn < max_iter && !stalled && done != all; ++itn) {
-            for (int e = tid; e < nrhs * n; e += BTH) {
-                const int r = e / n, i = e - r * n;
-                const int src = it.kind == RLG_KIND_LU ? raw[i] : i;
-                D[e] = (done >> r) & 1u ? 0.f : (float)R[(long)r * n + src];
-            }
-            __syncthreads();
-            if (it.kind == RLG_KIND_LU) {
-                tri_solve<float, TS_LOWER_UNIT>(ms.a32, n, D, nrhs, sm);
-                tri_solve<float, TS_UPPER>(ms.a32, n, D, nrhs, sm);
-            } else {
-                tri_solve<float, TS_LOWER>(ms.a32, n, D, nrhs, sm);
-                tri_solve<float, TS_LOWER_T>(ms.a32, n, D, nrhs, sm);
-            }
-            // x += d and |x|, one vector per wave
-            for (int r = wave; r < nrhs; r += BNW) {
-                if ((done >> r) & 1u) continue;
-                double xm = 0.0;
-                for (int i = lane; i < n; i += 64) {
-                    const double v = X[(long)r * n + i] + (double)D[(long)r * n + i];
-                    X[(long)r * n + i] = v;
-                    xm = fmax(xm, fabs(v));
-                }
-                xm = wave_max_f64(xm);
-                if (lane == 0) xmax[r] = xm;
-            }
-            __syncthreads();
-            // r = b - A x in FP64: a wave takes four rows and four vectors per
-            // pass over the rows (lanes across the row), so four rows' loads
-            // are in flight at once; |r| per vector kept in the wave's own LDS
-            // slots.  Each (row, vector) sum keeps one fixed order.
-            if (lane == 0) {
-#pragma unroll
-                for (int r = 0; r < BMAXR; ++r) rmax[wave * BMAXR + r] = 0.0;
-            }
-            for (int i0 = 4 * wave; i0 < n; i0 += 4 * BNW) {
-                for (int rb = 0; rb < nrhs; rb += 4) {
-                    double acc[4][4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) acc[u][q] = 0.0;
-                    for (int j = lane; j < n; j += 64) {
-                        double a[4], xv[4];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) a[u] = i0 + u < n ? A[(long)(i0 + u) * n + j] : 0.0;
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) xv[q] = rb + q < nrhs ? X[(long)(rb + q) * n + j] : 0.0;
-#pragma unroll
-                        for (int u = 0; u < 4; ++u)
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) acc[u][q] += a[u] * xv[q];
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            if (i0 + u < n && rb + q < nrhs) {
-                                const int i = i0 + u, r = rb + q;
-                                const double res = it.b[(long)r * n + i] - wave_sum_f64(acc[u][q]);
-                                if (lane == 0) {
-                                    R[(long)r * n + i] = res;
-                                    rmax[wave * BMAXR + r] = fmax(rmax[wave * BMAXR + r], fabs(res));
-                                }
-                            }
-                        }
-                    }
-                }
-            }
-            __syncthreads();
-            // every thread takes the same decisions; the errors of this step
-            // go to etab[itn & 1], the previous step's are read from the other
-            for (int r = 0; r < nrhs; ++r) {
-                if ((done >> r) & 1u) continue;
-                double rn = rmax[r];
-#pragma unroll
-                for (int q = 1; q < BNW; ++q) rn = fmax(rn, rmax[q * BMAXR + r]);
-                const double den = anorm * xmax[r] + bmax[r];
-                const double eta = den > 0 ? rn / den : 0.0;
-                if (eta <= tol) {
-                    done |= 1u << r;
-                } else if (itn >= 1 && !(eta <= 0.5 * etab[((itn + 1) & 1) * BMAXR + r])) {
-                    stalled = true;
-                }
-                if (tid == 0) etab[(itn & 1) * BMAXR + r] = eta;
-            }
-            __syncthreads();
-        }
-        const bool converged = !stalled && done == all;
+        const bool converged = mixed_refine(it.kind, n, nrhs, it.a, it.b, slot, anorm, info, max_iter, tol, sm);
         if (converged) {
             for (int e = tid; e < nrhs * n; e += BTH) it.b[e] = ms.x[e];
             if (tid == 0) items[id].status = RLG_OK;
         } else {
             // fallback: plain FP64 on a copy of A
-            for (int e = tid; e < n * n; e += BTH) ms.a64[e] = A[e];
+            for (int e = tid; e < n * n; e += BTH) ms.a64[e] = it.a[e];
             __syncthreads();
             const int inf64 = solve_system<double>(it.kind, nbs[id], ms.a64, n, it.b, nrhs, ms.piv, sm);
             if (tid == 0) {
