@@ -422,8 +422,10 @@ __global__ __launch_bounds__(256) void k_trsv_step(const T *__restrict__ M, long
 #pragma unroll
                 for (int k = 0; k < NR; ++k) {
                     odd |= wild(y[k]);
-                    if constexpr (MODE != LOWER_UNIT)
-                        odd |= (exponent(y[k]) < Range<T>::SOLVED) | (exponent(x[k]) - exponent(dl) < Range<T>::RHS);
+                    if constexpr (MODE != LOWER_UNIT) {
+                        odd |= exponent(y[k]) < Range<T>::SOLVED;
+                        odd |= exponent(x[k]) - exponent(dl) < Range<T>::RHS;
+                    }
                 }
                 if constexpr (MODE != LOWER_UNIT) odd |= low - exponent(dl) < Range<T>::ENTRY;
                 if (__any(odd)) {
