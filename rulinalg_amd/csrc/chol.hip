@@ -180,14 +180,17 @@ __global__ __launch_bounds__(128) void k_chol_block(T *__restrict__ A, long lda,
 // product, a square root and a division each, 66 us in FP64 whatever the
 // height.  Larger orders take k_chol_col, which does the same work in 16-column
 // panels: one wave factors a panel with the rows of the diagonal block in its
-// lanes (no barrier per column, the square root and its reciprocal from one
-// Goldschmidt iteration, fused multiply-adds), the matrix cores apply it to
+// lanes (no barrier per column, the square root and its reciprocal from
+// Goldschmidt's iteration, fused multiply-adds), the matrix cores apply it to
 // the rest of the diagonal block, and the rows below are solved panel by panel
 // beside the next panel's factorization.  Like the reference's dot products,
 // every panel's products are summed before they are subtracted (subtracted one
-// by one, the factor's residual at order 128 was 19 % larger).  It is bound by the serial chain of
-// the 64 columns (about 180 cycles each).  Order 4096: 6.27 -> 2.58 ms for the
-// factorization, order 16384: 49.6 -> 33.2 ms (44 TF).
+// by one, the factor's residual at order 128 was 19 % larger).  Of a launch's 55,000
+// cycles at order 4096 (stamps of wave 0) the chain of the 64 columns takes 29,700
+// (460 each, the multiply-adds onto the panel's later columns included), the loads and
+// the arrival count 12,300, products and barriers between panels 3,500, the wait for the rows
+// below 2,200, their last panel 3,400 and the stores 3,900.  Order 4096: 6.27 ->
+// 2.58 ms for the factorization, order 16384: 49.6 -> 33.2 ms (44 TF).
 
 // s = sqrt(d) and r = 1 / s for d >= epsilon (two steps of Goldschmidt's iteration
 // from the hardware's reciprocal square root estimate, then one residual step for

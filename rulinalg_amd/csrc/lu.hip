@@ -32,9 +32,9 @@ namespace rlg {
 
 constexpr int PNB = 64;    // inner panel width
 constexpr int SPW = 16;    // columns held in registers at a time
-// Panel rows per workgroup (LDS-resident), one per thread: 256 in FP64 (146 KB
-// of LDS, one workgroup per CU, so every workgroup of a panel is resident at
-// once) and 512 in FP32 (the same bytes).
+// Panel rows per workgroup (LDS-resident), one per thread: 256 in FP64
+// (154,592 bytes of LDS, one workgroup per CU, so every workgroup of a panel is
+// resident at once) and 512 in FP32 (151,648 bytes).
 template <class T> struct PanelRows { static constexpr int value = 256; };
 template <> struct PanelRows<float> { static constexpr int value = 512; };
 constexpr int ONB = 512;   // outer block: depth of the trailing GEMM
@@ -234,7 +234,7 @@ template <class T> constexpr int TW = PNB + TilePad<T>::value;
 // arithmetic.  Rows of 64 kept in LDS with three barriers per column and an
 // update of the whole row per column took, in FP64, 122 us for a panel of 256
 // rows and, on average over the factorization, 188 at order 1,531 and 209 at
-// 16,384; this form takes 68, 137 and 184.
+// 16,384; this form takes 68, 163 (151 to 164 between runs) and 189.
 //
 // EXACT (FP32, and FP64 orders up to 64): divisions, and separately rounded
 // products and differences in the reference's order.
