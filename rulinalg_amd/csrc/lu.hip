@@ -288,7 +288,9 @@ __global__ __launch_bounds__(PanelRows<T>::value) void k_lu_panel(
         for (int j = cb; j < min(cb + SPW, w); ++j) {
             const int c = j - cb, par = j & 1;
             const T av = fabs(x[0]);
-            const unsigned hi = pos >= j ? rank_hi(av, pos == j) : 0u, lo = rank_lo(av);
+            // (opaque: its tests' masks would be kept for the swap below, and spilled)
+            const int ahead = opaque(pos - j);
+            const unsigned hi = ahead >= 0 ? rank_hi(av, ahead == 0) : 0u, lo = rank_lo(av);
             const int wl = first_max_lane(hi, lo, pos);
             if (lane == max(wl, 0)) {
                 red[par][wave] = uint4{wl < 0 ? 0u : hi, lo, (unsigned)pos, (unsigned)tid};

@@ -127,12 +127,13 @@ __device__ __forceinline__ int wave_min_i32(int k) {
 // diagonal never given up.
 
 // The high word of a magnitude plus one (a non-negative float orders like its
-// bits); a NaN ranks like zero, and first of all in the diagonal's row.
+// bits); a NaN ranks like zero, but in the diagonal's row by its bits, which are at
+// least infinity's (the tie that leaves goes to the lower row, the diagonal's).
 __device__ __forceinline__ unsigned rank_hi(float v, bool diagonal) {
-    return (v == v) ? __float_as_uint(v) + 1 : diagonal ? ~0u : 1u;
+    return (int)(v == v) | (int)diagonal ? __float_as_uint(v) + 1 : 1u;
 }
 __device__ __forceinline__ unsigned rank_hi(double v, bool diagonal) {
-    return (v == v) ? (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) + 1 : diagonal ? ~0u : 1u;
+    return (int)(v == v) | (int)diagonal ? (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) + 1 : 1u;
 }
 __device__ __forceinline__ unsigned rank_lo(float) { return 0u; }
 __device__ __forceinline__ unsigned rank_lo(double v) {
