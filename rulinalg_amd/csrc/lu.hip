@@ -234,7 +234,7 @@ template <class T> constexpr int TW = PNB + TilePad<T>::value;
 // arithmetic.  Rows of 64 kept in LDS with three barriers per column and an
 // update of the whole row per column took, in FP64, 122 us for a panel of 256
 // rows and, on average over the factorization, 188 at order 1,531 and 209 at
-// 16,384; this form takes 68, 163 (151 to 164 between runs) and 189.
+// 16,384; this form takes 68, 152 to 165 (on different cards) and 189.
 //
 // EXACT (FP32, and FP64 orders up to 64): divisions, and separately rounded
 // products and differences in the reference's order.
